@@ -34,6 +34,7 @@ SOURCES = [
     ("sim.cpp", "hiphost"),
     ("gred.hip", "hip"),
     ("gred_realign.hip", "hip"),
+    ("gnarrow.hip", "hip"),
     ("sim.hip", "hip"),
     ("mlp.hip", "hip"),
     ("scratch.hip", "hip"),

@@ -27,6 +27,8 @@ hipError_t launch_gred(int dtype, int max_lg, const GredItem* items, uint32_t n,
                        const LaunchShape& sh, hipStream_t st);
 hipError_t launch_grun(uint32_t esize, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
                        const BufTable* tabs, bool batch, uint32_t allow_vec, const LaunchShape& sh, hipStream_t st);
+hipError_t launch_gnarrow(int dtype, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
+                          const BufTable* tabs, bool batch, int threads, hipStream_t st);
 hipError_t launch_reduce_local(int dtype, const void* a, const void* b, void* out, uint64_t n, hipStream_t st);
 size_t scratch_bytes();
 hipError_t scratch_init(int device);
@@ -124,6 +126,21 @@ int install(Lowered&& low, int max_lg, int64_t tile_elems, const LaunchShape& sh
     return BINE_OK;
 }
 
+// The general launch shape (default_shape) runs small lists on the narrow kernel.
+bool is_general(const LaunchShape& sh) {
+    return sh.vpt == 1 && sh.threads == 256 && sh.persistent == 0 && !sh.nontemporal && !sh.two_phase;
+}
+
+bool use_narrow(const std::vector<std::vector<Group>>& gs, size_t ds, const LaunchShape& sh) {
+    return is_general(sh) && narrow_pays(gs, (int)(16 / ds));
+}
+
+// Whether two launch shapes give a list the same items (the rest of a shape only changes the launch).
+bool same_lowering(const LaunchShape& a, const LaunchShape& b) {
+    return a.vpt == b.vpt && a.threads == b.threads && a.two_phase == b.two_phase &&
+           a.double_tiles == b.double_tiles && is_general(a) == is_general(b);
+}
+
 int max_lg_of(const std::vector<std::vector<Group>>& gs) {
     int m = 0;
     for (const auto& v : gs)
@@ -134,8 +151,11 @@ int max_lg_of(const std::vector<std::vector<Group>>& gs) {
 int upload(const std::vector<std::vector<Group>>& gs, size_t ds, const LaunchShape& sh, uint32_t bucket, DevArrays* d,
            Retired* retire = nullptr) {
     Lowered low;
-    lower_groups(gs, shallow_tile_elems(sh, ds), (int)(16 / ds), bucket, ds, &low, deep_tile_elems(sh, ds), split_lg(sh),
-                 nullptr, nullptr, sh.two_phase, sh.double_tiles ? 2 : 1);
+    if (use_narrow(gs, ds, sh))
+        lower_narrow(gs, (int)(16 / ds), bucket, ds, &low);
+    else
+        lower_groups(gs, shallow_tile_elems(sh, ds), (int)(16 / ds), bucket, ds, &low, deep_tile_elems(sh, ds),
+                     split_lg(sh), nullptr, nullptr, sh.two_phase, sh.double_tiles ? 2 : 1);
     return install(std::move(low), max_lg_of(gs), shallow_tile_elems(sh, ds), sh, d, retire);
 }
 
@@ -431,6 +451,12 @@ int launch_arrays(const DevArrays& d, int dtype, const BufTable& tab, uint32_t a
     if ((allow_vec & 1u) && realign_pays(d.low, off16(tab))) allow_vec |= 2u;
     for (size_t li = 0; li < d.low.launches.size(); ++li) {
         const auto& l = d.low.launches[li];
+        if (d.low.narrow_threads) {
+            hipError_t e = launch_gnarrow(dtype, d.items + l.first, l.second, d.pool, tab, nullptr, false,
+                                          d.low.narrow_threads, st);
+            if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("narrow launch: ") + hipGetErrorString(e));
+            continue;
+        }
         const uint32_t nrun = d.low.runs[li], nred = l.second - nrun;
         if (nred) {
             hipError_t e = launch_gred(dtype, d.max_lg, d.items + l.first, nred, d.pool, tab, nullptr, false,
@@ -961,10 +987,13 @@ extern "C" int bine_plan_dump(const bine_vcomm_config_t* cfg, int32_t coll, int 
     if (exec == BINE_EXEC_FUSED && !cp.fused_ok) return fail(BINE_ERR_UNSUPPORTED, "schedule cannot be fused: " + cp.fused_why);
     LaunchShape sh = default_shape();
     int64_t deep = deep_tile_elems(sh, ds);
+    const bool narrow = tile_elems < 0;
     if (tile_elems <= 0) tile_elems = default_tile_elems(ds);
     else deep = tile_elems;
     Lowered low;
-    if (exec == BINE_EXEC_FUSED)
+    if (exec == BINE_EXEC_FUSED && narrow)
+        lower_narrow(std::vector<std::vector<Group>>(1, cp.fused), (int)(16 / ds), 0, ds, &low);
+    else if (exec == BINE_EXEC_FUSED)
         lower_groups(std::vector<std::vector<Group>>(1, cp.fused), tile_elems, (int)(16 / ds), 0, ds, &low, deep, split_lg(sh),
                      nullptr, nullptr, two_phase & 3, (two_phase & 4) ? 2 : 1);
     else
@@ -1147,8 +1176,12 @@ int lower_list(bine_batch_t b, bine_batch_s::TypeList& l) {
         Lowered all;
         std::vector<uint8_t> bucket_vec(b->tabs.size());
         for (size_t i = 0; i < b->tabs.size(); ++i) bucket_vec[i] = (uint8_t)vec_ok(b->tabs[i]);
-        lower_groups(l.groups, shallow_tile_elems(l.shape, ds), (int)(16 / ds), 0, ds, &all, deep_tile_elems(l.shape, ds),
-                     split_lg(l.shape), &l.group_bucket, &bucket_vec, l.shape.two_phase, l.shape.double_tiles ? 2 : 1);
+        if (use_narrow(l.groups, ds, l.shape))
+            lower_narrow(l.groups, (int)(16 / ds), 0, ds, &all, &l.group_bucket);
+        else
+            lower_groups(l.groups, shallow_tile_elems(l.shape, ds), (int)(16 / ds), 0, ds, &all,
+                         deep_tile_elems(l.shape, ds), split_lg(l.shape), &l.group_bucket, &bucket_vec,
+                         l.shape.two_phase, l.shape.double_tiles ? 2 : 1);
         int max_lg = max_lg_of(l.groups);
         bool tables_off16 = false;
         for (uint32_t gb : l.group_bucket) tables_off16 = tables_off16 || off16(b->tabs[gb]);
@@ -1172,6 +1205,12 @@ int batch_lower(bine_batch_t b) {
 int run_list(bine_batch_t b, const bine_batch_s::TypeList& l, hipStream_t st) {
     const Lowered& low = l.arr.low;
     for (size_t li = 0; li < low.launches.size(); ++li) {
+        if (low.narrow_threads) {
+            hipError_t e = launch_gnarrow(l.dtype, l.arr.items + low.launches[li].first, low.launches[li].second,
+                                          l.arr.pool, BufTable{}, b->d_tabs, true, low.narrow_threads, st);
+            if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("batch narrow launch: ") + hipGetErrorString(e));
+            continue;
+        }
         const uint32_t first = low.launches[li].first, nrun = low.runs[li], nred = low.launches[li].second - nrun;
         if (nred) {
             hipError_t e = launch_gred(l.dtype, l.arr.max_lg, l.arr.items + first, nred, l.arr.pool, BufTable{},
@@ -1341,8 +1380,7 @@ extern "C" int bine_batch_set_tuning(bine_batch_t b, int32_t vpt, int32_t thread
     b->shape = sh;
     drop_graph(b);
     for (auto& l : b->lists) {
-        const bool relower = sh.vpt != l.shape.vpt || sh.threads != l.shape.threads || sh.two_phase != l.shape.two_phase ||
-                             sh.double_tiles != l.shape.double_tiles;
+        const bool relower = !same_lowering(sh, l.shape);
         l.shape = sh;
         if (relower) {
             int rc = lower_list(b, l);
@@ -1432,8 +1470,7 @@ extern "C" int bine_batch_autotune(bine_batch_t b, void* stream, int iters) {
     std::vector<std::vector<std::pair<float, LaunchShape>>> timed(nl);
     auto trial = [&](size_t i, const LaunchShape& c) -> int {
         auto& l = b->lists[i];
-        const bool relower = c.vpt != l.shape.vpt || c.threads != l.shape.threads || c.two_phase != l.shape.two_phase ||
-                             c.double_tiles != l.shape.double_tiles;
+        const bool relower = !same_lowering(c, l.shape);
         l.shape = c;
         int rc = relower ? lower_list(b, l) : BINE_OK;
         if (rc) return rc;
@@ -1462,8 +1499,7 @@ extern "C" int bine_batch_autotune(bine_batch_t b, void* stream, int iters) {
     size_t dominant = 0;
     for (size_t i = 0; i < nl; ++i) {
         auto& l = b->lists[i];
-        const bool relower = pick[i].vpt != l.shape.vpt || pick[i].threads != l.shape.threads ||
-                             pick[i].two_phase != l.shape.two_phase || pick[i].double_tiles != l.shape.double_tiles;
+        const bool relower = !same_lowering(pick[i], l.shape);
         l.shape = pick[i];
         if (relower) {
             int rc = lower_list(b, l);

@@ -17,6 +17,7 @@ inline PoolEntry make_entry(uint32_t buf, uint32_t rank, uint32_t off) { return 
 enum : uint16_t {
     ITEM_VEC = 1,  // the tile moves as 16-byte vectors: whole vectors, every leaf/output address dword-aligned
     ITEM_RUN = 2,  // a run of `pad` one-leaf, one-output copies (see GredItem)
+    ITEM_NARROW = 4,  // a tile of the narrow kernel (gnarrow.hip): any alignment, any length up to its workgroup's units
 };
 
 // Longest run of copies merged into one item: two, one pass of the copy-run kernel.  Lowering also cuts a

@@ -1917,6 +1917,110 @@ void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shall
     }
 }
 
+namespace {
+
+// 16-byte units of a group's block: whole vectors plus one that ends at the block's end, or single elements.
+int64_t narrow_units(const Group& g, int vec) { return g.n >= vec ? (g.n + vec - 1) / vec : g.n; }
+
+uint32_t pow2_at_least(uint64_t x) {
+    uint32_t p = 1;
+    while (p < x) p <<= 1;
+    return p;
+}
+
+// Lanes that leave each one about eight leaves to load and eight outputs to store.
+uint64_t narrow_segments(const Group& g) {
+    return pow2_at_least((std::max(g.leaves.size(), g.outs.size()) + 7) / 8);
+}
+
+constexpr int64_t kNarrowMinUnits = 4;    // units of a reduction's tile: at least 64 bytes
+constexpr int64_t kNarrowCopyUnits = 64;  // units of a copy's tile: 1 KiB of each output
+constexpr uint32_t kNarrowThreads = 1024;
+
+}  // namespace
+
+// The narrow kernel spreads leaves and outputs over the lanes, the general shape (256 lanes, one vector each) only
+// elements, so the line is where the general shape leaves the chip idle: too few workgroups for 256 compute units, or
+// blocks that fill a small part of a tile.  Microseconds per launch, general / narrow, fp32:
+//   few workgroups: 512 ranks, reduce of 32768 elements (128 workgroups) 27.2 / 16.2, of 98304 (384) 34.6 / 43.8 or
+//     36.7 by workgroup size, of 131072 (512) 43 / 58; 64 ranks, allreduce of 65536 (256) 9.7 / 8.4, of 131072 (512)
+//     14.0 / 14.8; bcast to 512 ranks of 131072 (128) 84 / 44, of 262144 (256) 119 / 107;
+//   eight leaves or outputs need no spreading: 8 ranks, allreduce of 65536 (64) 4.65 / 4.58, of 131072 (128) 4.9 / 5.1;
+//   short blocks on 512 ranks: allreduce of 65536 (32 vectors a block) 92 / 53, of 262144 (128) 288 / 259; allgather of
+//     256 (64) 101 / 59, of 512 (128) 141 / 140; reduce_scatter of 128 (32) 36.9 / 31.0, of 192 (48) 37.5 / 45.1.
+bool narrow_pays(const std::vector<std::vector<Group>>& launches, int vec) {
+    if (launches.size() != 1) return false;
+    size_t fan = 0;
+    uint64_t workgroups = 0, units = 0, short_units = 0;
+    for (const Group& g : launches[0]) {
+        fan = std::max({fan, g.leaves.size(), g.outs.size()});
+        const uint64_t u = (uint64_t)narrow_units(g, vec), ends = g.leaves.size() + g.outs.size();
+        const uint64_t tile = g.lg >= 5 ? 64 : 256;
+        workgroups += (u + tile - 1) / tile;
+        units += u * ends;
+        if (u <= (g.lg > 0 && g.outs.size() == 1 ? 32u : 128u)) short_units += u * ends;
+    }
+    if (fan < 16) return fan >= 4 && workgroups < 128;
+    return workgroups < 512 || 2 * short_units >= units;
+}
+
+void lower_narrow(const std::vector<std::vector<Group>>& launches, int vec, uint32_t bucket, size_t dtsize,
+                  Lowered* out, const std::vector<uint32_t>* group_bucket) {
+    const std::vector<Group>& gs = launches[0];
+    uint64_t lanes = 0;  // that give each lane its eight leaves and outputs
+    uint64_t need = 1;   // of them, those of the widest tree's smallest tile
+    for (const Group& g : gs) {
+        const uint64_t u = (uint64_t)narrow_units(g, vec);
+        lanes += u * narrow_segments(g);
+        if (g.lg > 0) need = std::max(need, std::min<uint64_t>(kNarrowMinUnits, pow2_at_least(u)) * narrow_segments(g));
+    }
+    // workgroups as small as leaves one for every compute unit: against 1024 lanes always, 8 ranks' allreduce of 131072
+    // fp32 elements takes 5.1 us instead of 6.0 (512 lanes), 512 ranks' of 1024 7.9 instead of 9.4
+    const uint32_t threads =
+        (uint32_t)std::min<uint64_t>(kNarrowThreads, std::max<uint64_t>({64, need, pow2_at_least(lanes / 256)}));
+    out->narrow_threads = (int)threads;
+    for (size_t gi = 0; gi < gs.size(); ++gi) {
+        const Group& g = gs[gi];
+        if (g.n <= 0) continue;
+        const uint32_t leaf_off = (uint32_t)out->pool.size();
+        out->pool.insert(out->pool.end(), g.leaves.begin(), g.leaves.end());
+        const uint32_t out_off = (uint32_t)out->pool.size();
+        out->pool.insert(out->pool.end(), g.outs.begin(), g.outs.end());
+        const int64_t units = narrow_units(g, vec);
+        const int64_t least = g.lg > 0 ? kNarrowMinUnits : kNarrowCopyUnits;
+        int64_t w = std::min<int64_t>(std::max<int64_t>(least, threads / narrow_segments(g)), threads);
+        const int64_t tiles = (units + w - 1) / w;
+        w = (units + tiles - 1) / tiles;
+        // outputs per item: all of a reduction's; a copy's outputs in ranges of eight per segment
+        const int64_t segs = std::max<int64_t>(1, (int64_t)threads / pow2_at_least((uint64_t)w));
+        const uint32_t per = g.lg > 0 ? (uint32_t)g.outs.size() : (uint32_t)(8 * segs);
+        const int64_t elems = g.n >= vec ? w * vec : w;
+        for (int64_t d = 0; d < g.n;) {
+            int64_t n = std::min(elems, g.n - d);
+            const int64_t rest = g.n - d - n;
+            if (g.n >= vec && rest > 0 && rest < vec) n -= vec;  // the last tile holds a whole vector
+            for (uint32_t o = 0; o < g.outs.size(); o += per) {
+                GredItem it{};
+                it.leaf_off = leaf_off;
+                it.out_off = out_off + o;
+                it.lg = g.lg;
+                it.flags = ITEM_NARROW;
+                it.nouts = std::min<uint32_t>(per, (uint32_t)g.outs.size() - o);
+                it.delta = (uint32_t)d;
+                it.n = (uint32_t)n;
+                it.bucket = group_bucket ? (*group_bucket)[gi] : bucket;
+                out->items.push_back(it);
+            }
+            d += n;
+        }
+        out->bytes_read += (uint64_t)g.n * g.leaves.size() * dtsize;
+        out->bytes_written += (uint64_t)g.n * g.outs.size() * dtsize;
+        out->max_leaves = std::max<uint64_t>(out->max_leaves, g.leaves.size());
+    }
+    out->launches.push_back({0, (uint32_t)out->items.size()});
+    out->runs.push_back(0);
+}
+
 bool has_multi_output_reduction(const std::vector<std::vector<Group>>& launches) {
     for (const auto& gs : launches)
         for (const Group& g : gs)

@@ -111,6 +111,7 @@ struct Lowered {
     std::vector<std::pair<uint32_t, uint32_t>> launches;  // (first item, item count)
     std::vector<uint32_t> runs;  // per launch: how many of its items are ITEM_RUN items (they come last)
     uint64_t bytes_read = 0, bytes_written = 0, max_leaves = 0;
+    int narrow_threads = 0;  // > 0: every item is ITEM_NARROW, run by the narrow kernel with workgroups of that many lanes
     bool unaligned_outs = false;  // some vector item writes an output whose offset is not a whole number of vectors
 };
 // tile_elems: elements per work item; vec_elems: elements per 16-byte vector.
@@ -127,6 +128,11 @@ void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t tile_
                   uint32_t bucket, size_t dtsize, Lowered* out, int64_t deep_tile_elems = 0, int deep_lg = 99,
                   const std::vector<uint32_t>* group_bucket = nullptr, const std::vector<uint8_t>* bucket_vec = nullptr,
                   int two_phase = 0, int reduction_tiles = 1);
+// Whether a list (one launch, at the general launch shape) is better run by the narrow kernel (gnarrow.hip).
+bool narrow_pays(const std::vector<std::vector<Group>>& launches, int vec_elems);
+// The list as ITEM_NARROW items; same groups, same results.  Arguments as for lower_groups.
+void lower_narrow(const std::vector<std::vector<Group>>& launches, int vec_elems, uint32_t bucket, size_t dtsize,
+                  Lowered* out, const std::vector<uint32_t>* group_bucket = nullptr);
 // Whether some launch holds a reduction with several outputs (the lists a two-phase lowering changes).
 bool has_multi_output_reduction(const std::vector<std::vector<Group>>& launches);
 
