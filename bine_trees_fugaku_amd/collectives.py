@@ -289,8 +289,8 @@ def plan_dump(dims: Sequence[int], coll: str, count: int, dtype, op: str = "SUM"
               num_ports: int = 1, tile_elems: int = 0, in_place: bool = False, two_phase: int = 0, **overrides):
     """Compile a schedule on the host (no GPU) and return its lowered work as
     numpy arrays: (info dict, items structured array, pool structured array,
-    launches (n, 2) array).  tile_elems: elements per tile, 0 for the general shape's, negative for the narrow list a
-    small call uploads.  in_place: the allreduce schedule for sendbuf == recvbuf.
+    launches (n, 2) array).  tile_elems: elements per tile, 0 for the general shape's, -1 for the narrow list a small
+    call uploads, -t for tiles of up to t elements whose end vectors overlap their neighbours.  in_place: the allreduce schedule for sendbuf == recvbuf.
     two_phase: 1 or 2 lowers reductions with several outputs as two launches (see Batch.set_tuning); adding 4
     gives the reduction launch items of two tiles."""
     import numpy as np

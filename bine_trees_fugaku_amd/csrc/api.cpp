@@ -23,10 +23,10 @@
 
 namespace bine {
 hipError_t launch_gred(int dtype, int max_lg, const GredItem* items, uint32_t n, const PoolEntry* pool,
-                       const BufTable& tab, const BufTable* tabs, bool batch, uint32_t allow_vec,
+                       const BufTable& tab, const BufTable* tabs, bool batch, bool realign,
                        const LaunchShape& sh, hipStream_t st);
 hipError_t launch_grun(uint32_t esize, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
-                       const BufTable* tabs, bool batch, uint32_t allow_vec, const LaunchShape& sh, hipStream_t st);
+                       const BufTable* tabs, bool batch, const LaunchShape& sh, hipStream_t st);
 hipError_t launch_gnarrow(int dtype, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
                           const BufTable* tabs, bool batch, int threads, hipStream_t st);
 hipError_t launch_reduce_local(int dtype, const void* a, const void* b, void* out, uint64_t n, hipStream_t st);
@@ -126,6 +126,20 @@ int install(Lowered&& low, int max_lg, int64_t tile_elems, const LaunchShape& sh
     return BINE_OK;
 }
 
+// A list that writes at least twice what it reads: such lists may run the realigning kernels (realign_pays), whose
+// items hold whole vectors.
+inline bool write_heavy(uint64_t read, uint64_t written) { return written >= 2 * read; }
+
+bool write_heavy(const std::vector<std::vector<Group>>& gs) {
+    uint64_t read = 0, written = 0;
+    for (const auto& v : gs)
+        for (const Group& g : v) {
+            read += (uint64_t)g.n * g.leaves.size();
+            written += (uint64_t)g.n * g.outs.size();
+        }
+    return write_heavy(read, written);
+}
+
 // The general launch shape (default_shape) runs small lists on the narrow kernel.
 bool is_general(const LaunchShape& sh) {
     return sh.vpt == 1 && sh.threads == 256 && sh.persistent == 0 && !sh.nontemporal && !sh.two_phase;
@@ -148,14 +162,15 @@ int max_lg_of(const std::vector<std::vector<Group>>& gs) {
     return m;
 }
 
-int upload(const std::vector<std::vector<Group>>& gs, size_t ds, const LaunchShape& sh, uint32_t bucket, DevArrays* d,
+// fused: the groups' outputs share no memory with their leaves (every fused list)
+int upload(const std::vector<std::vector<Group>>& gs, size_t ds, const LaunchShape& sh, bool fused, DevArrays* d,
            Retired* retire = nullptr) {
     Lowered low;
     if (use_narrow(gs, ds, sh))
-        lower_narrow(gs, (int)(16 / ds), bucket, ds, &low);
+        lower_narrow(gs, (int)(16 / ds), 0, ds, &low);
     else
-        lower_groups(gs, shallow_tile_elems(sh, ds), (int)(16 / ds), bucket, ds, &low, deep_tile_elems(sh, ds),
-                     split_lg(sh), nullptr, nullptr, sh.two_phase, sh.double_tiles ? 2 : 1);
+        lower_groups(gs, shallow_tile_elems(sh, ds), (int)(16 / ds), 0, ds, &low, deep_tile_elems(sh, ds),
+                     split_lg(sh), nullptr, sh.two_phase, sh.double_tiles ? 2 : 1, fused && !write_heavy(gs));
     return install(std::move(low), max_lg_of(gs), shallow_tile_elems(sh, ds), sh, d, retire);
 }
 
@@ -293,7 +308,7 @@ int get_plan(bine_vcomm_t comm, const CollRequest& req, int dtype, std::shared_p
     }
     dp->dtype = dtype;
     dp->ds = ds;
-    int rc = upload(dp->cp.step_groups, ds, default_shape(), 0, &dp->step);
+    int rc = upload(dp->cp.step_groups, ds, default_shape(), false, &dp->step);
     if (rc) return rc;
     if (dp->cp.fused_ok && max_lg_of(std::vector<std::vector<Group>>(1, dp->cp.fused)) > 14) {
         dp->cp.fused_ok = false;  // the kernel's register stack holds trees of up to 2^14 leaves
@@ -302,7 +317,7 @@ int get_plan(bine_vcomm_t comm, const CollRequest& req, int dtype, std::shared_p
     }
     if (dp->cp.fused_ok) {
         std::vector<std::vector<Group>> one(1, dp->cp.fused);
-        rc = upload(one, ds, initial_shape(one, ds), 0, &dp->fused);
+        rc = upload(one, ds, initial_shape(one, ds), true, &dp->fused);
         if (rc) return rc;
     }
     // temporaries are allocated only when some step touches them
@@ -424,14 +439,6 @@ BufTable make_table(const DevPlan* dp, const void* send, void* recv) {
     return t;
 }
 
-// 16-byte vector accesses need 4-byte aligned addresses only (global memory runs in the
-// unaligned access mode); partitions aligned below that (odd int8 counts) take the scalar path.
-uint32_t vec_ok(const BufTable& t) {
-    for (int b = 0; b < 4; ++b)
-        if ((t.base[b] & 3) || (t.stride[b] & 3)) return 0;
-    return 1;
-}
-
 // some buffer base or partition stride is not a multiple of 16 bytes
 bool off16(const BufTable& t) {
     for (int b = 0; b < 4; ++b)
@@ -443,12 +450,11 @@ bool off16(const BufTable& t) {
 // allgather-like list that writes many outputs per leaf it reads ran 16 % faster with them, while 1:1 copies
 // ran 16 % slower and reductions 1.5 % slower than with plain unaligned 16-byte stores.
 bool realign_pays(const Lowered& low, bool tables_off16) {
-    return (low.unaligned_outs || tables_off16) && low.bytes_written >= 2 * low.bytes_read;
+    return (low.unaligned_outs || tables_off16) && write_heavy(low.bytes_read, low.bytes_written);
 }
 
-// allow_vec bit 0: vector items may run; the launch adds bit 1 (realigning kernels) where realign_pays.
-int launch_arrays(const DevArrays& d, int dtype, const BufTable& tab, uint32_t allow_vec, hipStream_t st) {
-    if ((allow_vec & 1u) && realign_pays(d.low, off16(tab))) allow_vec |= 2u;
+int launch_arrays(const DevArrays& d, int dtype, const BufTable& tab, hipStream_t st) {
+    const bool realign = realign_pays(d.low, off16(tab));
     for (size_t li = 0; li < d.low.launches.size(); ++li) {
         const auto& l = d.low.launches[li];
         if (d.low.narrow_threads) {
@@ -460,12 +466,12 @@ int launch_arrays(const DevArrays& d, int dtype, const BufTable& tab, uint32_t a
         const uint32_t nrun = d.low.runs[li], nred = l.second - nrun;
         if (nred) {
             hipError_t e = launch_gred(dtype, d.max_lg, d.items + l.first, nred, d.pool, tab, nullptr, false,
-                                       allow_vec, d.shape, st);
+                                       realign, d.shape, st);
             if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("gather-reduce launch: ") + hipGetErrorString(e));
         }
         if (nrun) {
             hipError_t e = launch_grun((uint32_t)dtsize(dtype), d.items + l.first + nred, nrun, d.pool, tab, nullptr,
-                                       false, allow_vec, d.shape, st);
+                                       false, d.shape, st);
             if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("copy-run launch: ") + hipGetErrorString(e));
         }
     }
@@ -476,11 +482,10 @@ int launch_arrays(const DevArrays& d, int dtype, const BufTable& tab, uint32_t a
 // the previous per-step run of the same plan (on whatever stream it ran) and record their own end, so calls on
 // different streams never share the temporaries at once.  Under capture the caller orders the graph.
 int launch_step_ordered(bine_vcomm_t comm, DevPlan* dp, const BufTable& tab, hipStream_t st) {
-    const uint32_t av = vec_ok(tab);
-    if (!dp->tmp_total() || capturing(st)) return launch_arrays(dp->step, dp->dtype, tab, av, st);
+    if (!dp->tmp_total() || capturing(st)) return launch_arrays(dp->step, dp->dtype, tab, st);
     std::lock_guard<std::mutex> lock(comm->mu);
     if (dp->tmp_recorded) HIPCHK(hipStreamWaitEvent(st, dp->tmp_done, 0));
-    int rc = launch_arrays(dp->step, dp->dtype, tab, av, st);
+    int rc = launch_arrays(dp->step, dp->dtype, tab, st);
     if (rc) return rc;
     HIPCHK(hipEventRecord(dp->tmp_done, st));
     dp->tmp_recorded = true;
@@ -516,7 +521,7 @@ int run_coll(bine_vcomm_t comm, const CollRequest& req0, int dtype, const void* 
     HIPCHK(hipSetDevice(comm->cfg.device));
     BufTable tab = make_table(dp, req.in_place ? recv : send, recv);
     if (exec == BINE_EXEC_STEP) return launch_step_ordered(comm, dp, tab, (hipStream_t)stream);
-    return launch_arrays(dp->fused, dtype, tab, vec_ok(tab), (hipStream_t)stream);
+    return launch_arrays(dp->fused, dtype, tab, (hipStream_t)stream);
 }
 
 // A cached schedule, or nullptr; never compiles (the allocation-free entry point uses it).
@@ -758,7 +763,7 @@ extern "C" int bine_allreduce_noalloc(const void* sendbuf, void* recvbuf, int co
         tab.base[BUF_TMP] = dp->tmp_bytes[0] ? (uint64_t)(uintptr_t)ptr : 0;
         tab.base[BUF_TMP2] = dp->tmp_bytes[1] ? (uint64_t)(uintptr_t)(ptr + align256(dp->tmp_bytes[0])) : 0;
     }
-    return launch_arrays(exec == BINE_EXEC_FUSED ? dp->fused : dp->step, datatype, tab, vec_ok(tab),
+    return launch_arrays(exec == BINE_EXEC_FUSED ? dp->fused : dp->step, datatype, tab,
                          (hipStream_t)stream);
 }
 
@@ -929,7 +934,7 @@ extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* s
     auto trial = [&](const LaunchShape& c) {
         // the arrays in place before the call may be named by captured graphs: they are kept, not freed;
         // the candidates' own arrays never leave this loop
-        if ((rc = upload(groups, dp->ds, c, 0, &d, first ? &dp->retired : nullptr))) return;
+        if ((rc = upload(groups, dp->ds, c, exec == BINE_EXEC_FUSED, &d, first ? &dp->retired : nullptr))) return;
         first = false;
         if ((rc = issue(comm, coll, sendbuf, recvbuf, count, datatype, op, root, stream))) return;
         if (hipEventRecord(e0, st) != hipSuccess) {
@@ -961,7 +966,7 @@ extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* s
     (void)hipEventDestroy(e1);
     comm->cfg.exec = saved_exec;
     if (rc) return rc;
-    return upload(groups, dp->ds, bestc, 0, &d);
+    return upload(groups, dp->ds, bestc, exec == BINE_EXEC_FUSED, &d);
 }
 
 extern "C" int bine_plan_dump(const bine_vcomm_config_t* cfg, int32_t coll, int count, bine_datatype_t datatype,
@@ -987,7 +992,8 @@ extern "C" int bine_plan_dump(const bine_vcomm_config_t* cfg, int32_t coll, int 
     if (exec == BINE_EXEC_FUSED && !cp.fused_ok) return fail(BINE_ERR_UNSUPPORTED, "schedule cannot be fused: " + cp.fused_why);
     LaunchShape sh = default_shape();
     int64_t deep = deep_tile_elems(sh, ds);
-    const bool narrow = tile_elems < 0;
+    const bool narrow = tile_elems == -1, shared_ends = tile_elems < -1;
+    if (shared_ends) tile_elems = -tile_elems;
     if (tile_elems <= 0) tile_elems = default_tile_elems(ds);
     else deep = tile_elems;
     Lowered low;
@@ -995,9 +1001,9 @@ extern "C" int bine_plan_dump(const bine_vcomm_config_t* cfg, int32_t coll, int 
         lower_narrow(std::vector<std::vector<Group>>(1, cp.fused), (int)(16 / ds), 0, ds, &low);
     else if (exec == BINE_EXEC_FUSED)
         lower_groups(std::vector<std::vector<Group>>(1, cp.fused), tile_elems, (int)(16 / ds), 0, ds, &low, deep, split_lg(sh),
-                     nullptr, nullptr, two_phase & 3, (two_phase & 4) ? 2 : 1);
+                     nullptr, two_phase & 3, (two_phase & 4) ? 2 : 1, shared_ends);
     else
-        lower_groups(cp.step_groups, tile_elems, (int)(16 / ds), 0, ds, &low, deep, split_lg(sh), nullptr, nullptr,
+        lower_groups(cp.step_groups, tile_elems, (int)(16 / ds), 0, ds, &low, deep, split_lg(sh), nullptr,
                      two_phase & 3, (two_phase & 4) ? 2 : 1);
     info->n_items = low.items.size();
     info->n_pool = low.pool.size();
@@ -1148,7 +1154,7 @@ struct bine_batch_s {
         std::vector<uint32_t> group_bucket;      // bucket of each group
         DevArrays arr;
         LaunchShape shape = default_shape();     // each element type is tuned on its own
-        uint32_t allow_vec = 1;                  // bit 1 set when some output can start off a 16-byte boundary
+        bool realign = false;                    // launched with the realigning kernels (realign_pays)
     };
     std::vector<TypeList> lists;
     BufTable* d_tabs = nullptr;
@@ -1174,21 +1180,19 @@ int lower_list(bine_batch_t b, bine_batch_s::TypeList& l) {
         // one lowering for the whole list: every work item carries its group's bucket index, runs of copies
         // form within a bucket, and items are ordered tile-major across all buckets
         Lowered all;
-        std::vector<uint8_t> bucket_vec(b->tabs.size());
-        for (size_t i = 0; i < b->tabs.size(); ++i) bucket_vec[i] = (uint8_t)vec_ok(b->tabs[i]);
         if (use_narrow(l.groups, ds, l.shape))
             lower_narrow(l.groups, (int)(16 / ds), 0, ds, &all, &l.group_bucket);
         else
             lower_groups(l.groups, shallow_tile_elems(l.shape, ds), (int)(16 / ds), 0, ds, &all,
-                         deep_tile_elems(l.shape, ds), split_lg(l.shape), &l.group_bucket, &bucket_vec,
-                         l.shape.two_phase, l.shape.double_tiles ? 2 : 1);
+                         deep_tile_elems(l.shape, ds), split_lg(l.shape), &l.group_bucket, l.shape.two_phase,
+                         l.shape.double_tiles ? 2 : 1, !write_heavy(l.groups));
         int max_lg = max_lg_of(l.groups);
         bool tables_off16 = false;
         for (uint32_t gb : l.group_bucket) tables_off16 = tables_off16 || off16(b->tabs[gb]);
-        const uint32_t allow = realign_pays(all, tables_off16) ? 3u : 1u;
+        const bool realign = realign_pays(all, tables_off16);
         int rc = install(std::move(all), max_lg, shallow_tile_elems(l.shape, ds), l.shape, &l.arr, nullptr);
         if (rc) return rc;
-        l.allow_vec = allow;
+        l.realign = realign;
     }
     return BINE_OK;
 }
@@ -1214,12 +1218,12 @@ int run_list(bine_batch_t b, const bine_batch_s::TypeList& l, hipStream_t st) {
         const uint32_t first = low.launches[li].first, nrun = low.runs[li], nred = low.launches[li].second - nrun;
         if (nred) {
             hipError_t e = launch_gred(l.dtype, l.arr.max_lg, l.arr.items + first, nred, l.arr.pool, BufTable{},
-                                       b->d_tabs, true, l.allow_vec, l.shape, st);
+                                       b->d_tabs, true, l.realign, l.shape, st);
             if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("batch launch: ") + hipGetErrorString(e));
         }
         if (nrun) {
             hipError_t e = launch_grun((uint32_t)dtsize(l.dtype), l.arr.items + first + nred, nrun, l.arr.pool,
-                                       BufTable{}, b->d_tabs, true, l.allow_vec, l.shape, st);
+                                       BufTable{}, b->d_tabs, true, l.shape, st);
             if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("batch copy-run launch: ") + hipGetErrorString(e));
         }
     }

@@ -27,8 +27,6 @@ namespace bine {
 
 namespace {
 
-typedef u4 u4b __attribute__((aligned(1)));  // 16 bytes at any byte address
-
 template <typename T>
 __device__ __forceinline__ Vec<T> load_unit(const char* p, Vec<T>*) {
     Vec<T> r;

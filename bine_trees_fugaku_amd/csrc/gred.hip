@@ -125,8 +125,7 @@ __device__ __forceinline__ void store_rounds_shifted(char* p, uint32_t k, const 
 template <int VPT, bool BATCH, bool NT>
 __global__ void __launch_bounds__(512) grun_kernel(const GredItem* __restrict__ items, uint32_t nitems,
                                                    const PoolEntry* __restrict__ pool, BufTable tab,
-                                                   const BufTable* __restrict__ tabs, uint32_t allow_vec,
-                                                   uint32_t esize) {
+                                                   const BufTable* __restrict__ tabs, uint32_t esize) {
     for (uint32_t ii = blockIdx.x; ii < nitems; ii += gridDim.x) {
         const GredItem it = cload(cptr(items + ii));
         Table t;
@@ -141,7 +140,7 @@ __global__ void __launch_bounds__(512) grun_kernel(const GredItem* __restrict__ 
         const PoolEntry l0 = cload(lp), ls = cload(lp + 1);
         const PoolEntry o0 = cload(op), os = cload(op + 1);
         const uint64_t delta = it.delta;
-        const bool vec = (it.flags & ITEM_VEC) && (allow_vec & 1u);
+        const bool vec = it.flags & (ITEM_VEC | ITEM_ANY);
         // two copies per pass, so every thread keeps 2 * VPT 16-byte loads in flight
         for (uint32_t j = 0; j < it.pad; j += 2) {
             const uint32_t j1 = j + 1 < it.pad ? j + 1 : j;  // an odd tail copies its last block twice
@@ -157,8 +156,8 @@ __global__ void __launch_bounds__(512) grun_kernel(const GredItem* __restrict__ 
                     for (int u = 0; u < VPT; ++u) {
                         const uint32_t vi = base + threadIdx.x + u * blockDim.x;
                         if (vi < nvec) {
-                            const BINE_GLOBAL u4* q0 = gptr<const u4>(s0 + (uint64_t)vi * 16);
-                            const BINE_GLOBAL u4* q1 = gptr<const u4>(s1 + (uint64_t)vi * 16);
+                            const BINE_GLOBAL u4b* q0 = gptr<const u4b>(s0 + (uint64_t)vi * 16);
+                            const BINE_GLOBAL u4b* q1 = gptr<const u4b>(s1 + (uint64_t)vi * 16);
                             a[u] = NT ? __builtin_nontemporal_load(q0) : *q0;
                             c[u] = NT ? __builtin_nontemporal_load(q1) : *q1;
                         }
@@ -167,8 +166,8 @@ __global__ void __launch_bounds__(512) grun_kernel(const GredItem* __restrict__ 
                     for (int u = 0; u < VPT; ++u) {
                         const uint32_t vi = base + threadIdx.x + u * blockDim.x;
                         if (vi < nvec) {
-                            BINE_GLOBAL u4* q0 = gptr<u4>(d0 + (uint64_t)vi * 16);
-                            BINE_GLOBAL u4* q1 = gptr<u4>(d1 + (uint64_t)vi * 16);
+                            BINE_GLOBAL u4b* q0 = gptr<u4b>(d0 + (uint64_t)vi * 16);
+                            BINE_GLOBAL u4b* q1 = gptr<u4b>(d1 + (uint64_t)vi * 16);
                             if (NT) {
                                 __builtin_nontemporal_store(a[u], q0);
                                 __builtin_nontemporal_store(c[u], q1);
@@ -206,7 +205,7 @@ constexpr int leaf_group() {
 template <typename T, int VPT, int MAXS, bool BATCH, bool NT, bool REALIGN>
 __global__ void __launch_bounds__(512) gred_kernel(const GredItem* __restrict__ items, uint32_t nitems,
                                                    const PoolEntry* __restrict__ pool, BufTable tab,
-                                                   const BufTable* __restrict__ tabs, uint32_t allow_vec) {
+                                                   const BufTable* __restrict__ tabs) {
     constexpr int VE = Vec<T>::N;
     constexpr int G = leaf_group<VPT, MAXS>();
     // partial subtree sums of the waves, [wave][u][lane] 16-byte vectors
@@ -230,27 +229,34 @@ __global__ void __launch_bounds__(512) gred_kernel(const GredItem* __restrict__ 
         const BINE_CONST PoolEntry* outs = cptr(pool + it.out_off);
         const uint32_t lg = it.lg;
         const uint64_t delta = it.delta;
+        // byte offset of vector v inside the tile (see GredItem::pad)
+        const int32_t pad = (int32_t)it.pad, last = (int32_t)it.n - VE;
+        auto at = [&](uint32_t v) __attribute__((always_inline)) {
+            const int32_t e = (int32_t)(v * VE) - pad;
+            return (uint32_t)((e < 0 ? 0 : e > last ? last : e) * (int32_t)sizeof(T));
+        };
         auto addp = [](const Pack<T, VPT>& a, const Pack<T, VPT>& b) __attribute__((always_inline)) {
             Pack<T, VPT> r;
 #pragma unroll
             for (int u = 0; u < VPT; ++u) r.x[u] = vadd<T>(a.x[u], b.x[u]);
             return r;
         };
-        const bool vec = (it.flags & ITEM_VEC) && (allow_vec & 1u);
+        const bool vec = it.flags & (ITEM_VEC | ITEM_ANY);
         if (vec && nw > 1 && lg >= lgw + 3) {
             // Deep tree: wave w reduces the contiguous leaf range [w << lgs, (w+1) << lgs),
             // a whole subtree of the balanced tree; the top lgw levels are then
             // joined pairwise from LDS, so the association is unchanged.
             const uint32_t lgs = lg - lgw;
             const BINE_CONST PoolEntry* my = cptr(pool + it.leaf_off + ((size_t)wave << lgs));
-            const uint32_t nvec = it.n / VE;
+            const uint32_t nvec = (it.n + it.pad + VE - 1) / VE;
             for (uint32_t base = 0; base < nvec; base += 64 * VPT) {
-                uint32_t vi[VPT];
+                uint32_t vi[VPT], off[VPT];
                 bool ok[VPT];
 #pragma unroll
                 for (int u = 0; u < VPT; ++u) {
                     vi[u] = base + lane + u * 64;
                     ok[u] = vi[u] < nvec;
+                    off[u] = at(vi[u]);
                 }
                 auto loadp = [&](uint32_t k) __attribute__((always_inline)) {
                     const PoolEntry e = cload(my + k);
@@ -258,7 +264,7 @@ __global__ void __launch_bounds__(512) gred_kernel(const GredItem* __restrict__ 
                     Pack<T, VPT> r;
 #pragma unroll
                     for (int u = 0; u < VPT; ++u) {
-                        if (ok[u]) r.x[u] = vload<T, NT>(p + (uint64_t)vi[u] * 16);
+                        if (ok[u]) r.x[u] = vload<T, NT>(p + off[u]);
                         else r.x[u] = Vec<T>{};
                     }
                     return r;
@@ -299,7 +305,7 @@ __global__ void __launch_bounds__(512) gred_kernel(const GredItem* __restrict__ 
                         } else {
 #pragma unroll
                             for (int u = 0; u < VPT; ++u)
-                                if (ok[u]) vstore<T, NT>(p + (uint64_t)vi[u] * 16, sum.x[u]);
+                                if (ok[u]) vstore<T, NT>(p + off[u], sum.x[u]);
                         }
                     }
                 } else {
@@ -308,20 +314,21 @@ __global__ void __launch_bounds__(512) gred_kernel(const GredItem* __restrict__ 
                         char* p = t.at(e.rb, (uint64_t)e.off + delta, sizeof(T));
 #pragma unroll
                         for (int u = 0; u < VPT; ++u)
-                            if (ok[u]) vstore<T, NT>(p + (uint64_t)vi[u] * 16, sum.x[u]);
+                            if (ok[u]) vstore<T, NT>(p + off[u], sum.x[u]);
                     }
                 }
             }
         } else if (vec) {
-            const uint32_t nvec = it.n / VE;
+            const uint32_t nvec = (it.n + it.pad + VE - 1) / VE;
             for (uint32_t base = 0; base < nvec; base += blockDim.x * VPT) {
-                uint32_t vi[VPT];
+                uint32_t vi[VPT], off[VPT];
                 bool ok[VPT];
 #pragma unroll
                 for (int u = 0; u < VPT; ++u) {
                     // realigning: each wave holds 64 * VPT consecutive vectors
                     vi[u] = REALIGN ? base + wave * (64u * VPT) + u * 64u + lane : base + threadIdx.x + u * blockDim.x;
                     ok[u] = vi[u] < nvec;
+                    off[u] = at(vi[u]);
                 }
                 auto loadp = [&](uint32_t k) __attribute__((always_inline)) {
                     const PoolEntry e = cload(leaves + k);
@@ -329,7 +336,7 @@ __global__ void __launch_bounds__(512) gred_kernel(const GredItem* __restrict__ 
                     Pack<T, VPT> r;
 #pragma unroll
                     for (int u = 0; u < VPT; ++u) {
-                        if (ok[u]) r.x[u] = vload<T, NT>(p + (uint64_t)vi[u] * 16);
+                        if (ok[u]) r.x[u] = vload<T, NT>(p + off[u]);
                         else r.x[u] = Vec<T>{};
                     }
                     return r;
@@ -352,7 +359,7 @@ __global__ void __launch_bounds__(512) gred_kernel(const GredItem* __restrict__ 
                         } else {
 #pragma unroll
                             for (int u = 0; u < VPT; ++u)
-                                if (ok[u]) vstore<T, NT>(p + (uint64_t)vi[u] * 16, s.x[u]);
+                                if (ok[u]) vstore<T, NT>(p + off[u], s.x[u]);
                         }
                     }
                 } else {
@@ -361,7 +368,7 @@ __global__ void __launch_bounds__(512) gred_kernel(const GredItem* __restrict__ 
                         char* p = t.at(e.rb, (uint64_t)e.off + delta, sizeof(T));
 #pragma unroll
                         for (int u = 0; u < VPT; ++u)
-                            if (ok[u]) vstore<T, NT>(p + (uint64_t)vi[u] * 16, s.x[u]);
+                            if (ok[u]) vstore<T, NT>(p + off[u], s.x[u]);
                     }
                 }
             }
@@ -421,7 +428,7 @@ __global__ void __launch_bounds__(256) reduce_local_kernel(const T* a, const T* 
 
 template <typename T, int VPT, int MAXS, bool BATCH, bool RA>
 static hipError_t launch_t(const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
-                           const BufTable* tabs, uint32_t allow_vec, const LaunchShape& sh, hipStream_t st) {
+                           const BufTable* tabs, const LaunchShape& sh, hipStream_t st) {
     uint32_t grid = sh.persistent > 0 ? (uint32_t)sh.persistent : n;
     if (grid > n) grid = n;
     if (grid == 0) return hipSuccess;
@@ -429,46 +436,46 @@ static hipError_t launch_t(const GredItem* items, uint32_t n, const PoolEntry* p
     const size_t lds = (size_t)(sh.threads / 64) * VPT * 64 * 16;
     if (sh.nontemporal)
         hipLaunchKernelGGL((gred_kernel<T, VPT, MAXS, BATCH, true, RA>), dim3(grid), dim3(sh.threads), lds, st, items,
-                           n, pool, tab, tabs, allow_vec);
+                           n, pool, tab, tabs);
     else
         hipLaunchKernelGGL((gred_kernel<T, VPT, MAXS, BATCH, false, RA>), dim3(grid), dim3(sh.threads), lds, st, items,
-                           n, pool, tab, tabs, allow_vec);
+                           n, pool, tab, tabs);
     return hipGetLastError();
 }
 
 template <typename T, bool BATCH, bool RA>
 static hipError_t launch_v(int max_lg, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
-                           const BufTable* tabs, uint32_t allow_vec, const LaunchShape& sh, hipStream_t st) {
+                           const BufTable* tabs, const LaunchShape& sh, hipStream_t st) {
     const bool small = max_lg <= 9;
     switch (sh.vpt) {
     case 1:
-        return small ? launch_t<T, 1, 6, BATCH, RA>(items, n, pool, tab, tabs, allow_vec, sh, st)
-                     : launch_t<T, 1, 11, BATCH, RA>(items, n, pool, tab, tabs, allow_vec, sh, st);
+        return small ? launch_t<T, 1, 6, BATCH, RA>(items, n, pool, tab, tabs, sh, st)
+                     : launch_t<T, 1, 11, BATCH, RA>(items, n, pool, tab, tabs, sh, st);
     case 2:
-        return small ? launch_t<T, 2, 6, BATCH, RA>(items, n, pool, tab, tabs, allow_vec, sh, st)
-                     : launch_t<T, 2, 11, BATCH, RA>(items, n, pool, tab, tabs, allow_vec, sh, st);
+        return small ? launch_t<T, 2, 6, BATCH, RA>(items, n, pool, tab, tabs, sh, st)
+                     : launch_t<T, 2, 11, BATCH, RA>(items, n, pool, tab, tabs, sh, st);
     default:  // four vectors per thread; deep trees run with two
         // trees of up to 64 leaves: groups of 4 leaves, four stack levels, 163 VGPRs, three waves per SIMD
-        if (max_lg <= 6) return launch_t<T, 4, 4, BATCH, RA>(items, n, pool, tab, tabs, allow_vec, sh, st);
-        if (!small) return launch_t<T, 2, 11, BATCH, RA>(items, n, pool, tab, tabs, allow_vec, sh, st);
+        if (max_lg <= 6) return launch_t<T, 4, 4, BATCH, RA>(items, n, pool, tab, tabs, sh, st);
+        if (!small) return launch_t<T, 2, 11, BATCH, RA>(items, n, pool, tab, tabs, sh, st);
         // up to 512 leaves: groups of 8 leaves and six stack levels (250 VGPRs, no scratch; 0.3-1.4 % faster on
         // the 512-rank allreduce than groups of 4 with seven levels), except where those registers do not fit:
         // int8's byte arithmetic and the realigning stores
         if constexpr (sizeof(T) > 1 && !RA)
-            return launch_t<T, 4, 6, BATCH, RA>(items, n, pool, tab, tabs, allow_vec, sh, st);
+            return launch_t<T, 4, 6, BATCH, RA>(items, n, pool, tab, tabs, sh, st);
         else
-            return launch_t<T, 4, 7, BATCH, RA>(items, n, pool, tab, tabs, allow_vec, sh, st);
+            return launch_t<T, 4, 7, BATCH, RA>(items, n, pool, tab, tabs, sh, st);
     }
 }
 
 // dtype codes follow bine_datatype_t
 template <bool RA>
 hipError_t launch_gred_t(int dtype, int max_lg, const GredItem* items, uint32_t n, const PoolEntry* pool,
-                         const BufTable& tab, const BufTable* tabs, bool batch, uint32_t allow_vec,
+                         const BufTable& tab, const BufTable* tabs, bool batch,
                          const LaunchShape& sh, hipStream_t st) {
 #define BINE_DISPATCH(T)                                                                               \
-    return batch ? launch_v<T, true, RA>(max_lg, items, n, pool, tab, tabs, allow_vec, sh, st)         \
-                 : launch_v<T, false, RA>(max_lg, items, n, pool, tab, tabs, allow_vec, sh, st)
+    return batch ? launch_v<T, true, RA>(max_lg, items, n, pool, tab, tabs, sh, st)         \
+                 : launch_v<T, false, RA>(max_lg, items, n, pool, tab, tabs, sh, st)
     switch (dtype) {
     case 0: BINE_DISPATCH(int32_t);
     case 1: BINE_DISPATCH(int64_t);
@@ -483,29 +490,29 @@ hipError_t launch_gred_t(int dtype, int max_lg, const GredItem* items, uint32_t 
 #if BINE_GRED_REALIGN
 // this unit holds the realigning instantiations only
 template hipError_t launch_gred_t<true>(int, int, const GredItem*, uint32_t, const PoolEntry*, const BufTable&,
-                                        const BufTable*, bool, uint32_t, const LaunchShape&, hipStream_t);
+                                        const BufTable*, bool, const LaunchShape&, hipStream_t);
 #else
 extern template hipError_t launch_gred_t<true>(int, int, const GredItem*, uint32_t, const PoolEntry*, const BufTable&,
-                                               const BufTable*, bool, uint32_t, const LaunchShape&, hipStream_t);
+                                               const BufTable*, bool, const LaunchShape&, hipStream_t);
 
-// allow_vec: bit 0 permits ITEM_VEC items; bit 1 selects the realigning kernels
+// realign: the realigning kernels
 hipError_t launch_gred(int dtype, int max_lg, const GredItem* items, uint32_t n, const PoolEntry* pool,
-                       const BufTable& tab, const BufTable* tabs, bool batch, uint32_t allow_vec,
+                       const BufTable& tab, const BufTable* tabs, bool batch, bool realign,
                        const LaunchShape& sh, hipStream_t st) {
     if (n == 0) return hipSuccess;
-    return (allow_vec & 2u) ? launch_gred_t<true>(dtype, max_lg, items, n, pool, tab, tabs, batch, allow_vec, sh, st)
-                            : launch_gred_t<false>(dtype, max_lg, items, n, pool, tab, tabs, batch, allow_vec, sh, st);
+    return realign ? launch_gred_t<true>(dtype, max_lg, items, n, pool, tab, tabs, batch, sh, st)
+                            : launch_gred_t<false>(dtype, max_lg, items, n, pool, tab, tabs, batch, sh, st);
 }
 
 hipError_t launch_grun(uint32_t esize, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
-                       const BufTable* tabs, bool batch, uint32_t allow_vec, const LaunchShape& sh, hipStream_t st) {
+                       const BufTable* tabs, bool batch, const LaunchShape& sh, hipStream_t st) {
     if (n == 0) return hipSuccess;
     if (sh.threads < 64 || sh.threads > 512 || (sh.threads & (sh.threads - 1))) return hipErrorInvalidValue;
     uint32_t grid = sh.persistent > 0 ? (uint32_t)sh.persistent : n;
     if (grid > n) grid = n;
 #define BINE_RUN(V, B, N)                                                                                     \
     hipLaunchKernelGGL((grun_kernel<V, B, N>), dim3(grid), dim3(sh.threads), 0, st, items, n, pool, tab, tabs, \
-                       allow_vec, esize)
+                       esize)
 #define BINE_RUN_V(B, N)           \
     switch (sh.vpt) {              \
     case 1: BINE_RUN(1, B, N); break; \

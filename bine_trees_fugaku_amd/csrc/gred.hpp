@@ -15,8 +15,9 @@ struct PoolEntry {
 inline PoolEntry make_entry(uint32_t buf, uint32_t rank, uint32_t off) { return PoolEntry{rank | (buf << 28), off}; }
 
 enum : uint16_t {
-    ITEM_VEC = 1,  // the tile moves as 16-byte vectors: whole vectors, every leaf/output address dword-aligned
+    ITEM_VEC = 1,  // the tile moves as 16-byte vectors, every leaf and output offset dword-aligned
     ITEM_RUN = 2,  // a run of `pad` one-leaf, one-output copies (see GredItem)
+    ITEM_ANY = 8,  // the tile moves as 16-byte vectors, offsets at any byte
     ITEM_NARROW = 4,  // a tile of the narrow kernel (gnarrow.hip): any alignment, any length up to its workgroup's units
 };
 
@@ -39,6 +40,10 @@ struct alignas(16) GredItem {
     uint32_t pad;       // ITEM_RUN: number of copies k >= 2.  The pool holds {first leaf, leaf step}
                         // at leaf_off and {first output, output step} at out_off; copy j reads
                         // first leaf + j * step (rank and offset both advance) and writes likewise.
+                        // Other vector items: how many elements before delta the first vector would start
+                        // (below a whole vector).  Vector v covers elements v * N - pad onwards, moved inside
+                        // [0, n - N] at either end: the elements that two vectors then share are computed and
+                        // stored by both, with the same bits.
 };
 static_assert(sizeof(GredItem) == 32, "GredItem layout");
 

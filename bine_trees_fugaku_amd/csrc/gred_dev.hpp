@@ -20,7 +20,7 @@ typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 // (one s_load_dwordx8 for four consecutive pool entries) that never wait on the data loads.
 #define BINE_GLOBAL __attribute__((address_space(1)))
 #define BINE_CONST __attribute__((address_space(4)))
-typedef BINE_GLOBAL u4 gu4;
+typedef u4 u4b __attribute__((aligned(1)));  // 16 bytes at any byte address (global memory runs in the unaligned mode)
 
 template <typename X>
 __device__ __forceinline__ BINE_GLOBAL X* gptr(const void* p) {
@@ -100,15 +100,15 @@ __device__ __forceinline__ Vec<int8_t> vadd<int8_t>(const Vec<int8_t>& a, const 
 template <typename T, bool NT>
 __device__ __forceinline__ Vec<T> vload(const char* p) {
     Vec<T> r;
-    if (NT) r.raw = __builtin_nontemporal_load(gptr<const u4>(p));
-    else r.raw = *gptr<const u4>(p);
+    if (NT) r.raw = __builtin_nontemporal_load(gptr<const u4b>(p));
+    else r.raw = *gptr<const u4b>(p);
     return r;
 }
 
 template <typename T, bool NT>
 __device__ __forceinline__ void vstore(char* p, const Vec<T>& v) {
-    if (NT) __builtin_nontemporal_store(v.raw, gptr<u4>(p));
-    else *gptr<u4>(p) = v.raw;
+    if (NT) __builtin_nontemporal_store(v.raw, gptr<u4b>(p));
+    else *gptr<u4b>(p) = v.raw;
 }
 
 // Buffer address of a (buffer, rank, element offset) entry.  The buffer is

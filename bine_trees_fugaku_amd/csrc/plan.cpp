@@ -1702,8 +1702,7 @@ bool compile_program(const Program& prog, bool want_fused, CompiledPlan* out, st
 
 void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shallow_tile, int vec, uint32_t bucket,
                   size_t dtsize, Lowered* out, int64_t deep_tile_elems, int deep_lg,
-                  const std::vector<uint32_t>* group_bucket, const std::vector<uint8_t>* bucket_vec, int two_phase,
-                  int reduction_tiles) {
+                  const std::vector<uint32_t>* group_bucket, int two_phase, int reduction_tiles, bool shared_ends) {
     auto lower_launch = [&](const std::vector<Group>& gs, const std::vector<uint32_t>* gbk, bool copies_by_tile,
                             int64_t tiles_per_item) {
         const uint32_t first = (uint32_t)out->items.size();
@@ -1713,13 +1712,12 @@ void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shall
         uint32_t run_len = 0;
         std::vector<uint32_t> tile_no;  // per emitted item: its tile's index within its group
         PoolEntry run_leaf{}, run_out{}, step_leaf{}, step_out{};
-        auto vec_bucket = [&](uint32_t b) { return !bucket_vec || (*bucket_vec)[b]; };
-        // 16-byte vector accesses need dword-aligned addresses only: loads run at full rate unaligned and
-        // the kernels realign the stores, so leaves and outputs need not share a residue modulo the vector.
+        // 16-byte vectors move at any byte address: leaves and outputs need not share a residue modulo the vector.
+        // Bytes at odd counts moved one element per lane before: int8 allreduce of 1048573 on 64 ranks 175 -> 22 us of
+        // GPU time (6 TB/s), reduce_scatter of 65643 805 -> 63, allgather 386 -> 51.
         auto word_ok = [&](const PoolEntry& e) { return ((uint64_t)e.off * dtsize) % 4 == 0; };
-        auto single_copy = [&](const Group& g, uint32_t b) {
-            return g.lg == 0 && g.leaves.size() == 1 && g.outs.size() == 1 && g.n <= shallow_tile && g.n % vec == 0 &&
-                   word_ok(g.leaves[0]) && word_ok(g.outs[0]) && vec_bucket(b);
+        auto single_copy = [&](const Group& g) {
+            return g.lg == 0 && g.leaves.size() == 1 && g.outs.size() == 1 && g.n <= shallow_tile && g.n % vec == 0;
         };
         // step b - a with non-negative rank and offset parts in the same buffer
         auto step_of = [](const PoolEntry& a, const PoolEntry& b, PoolEntry* st) {
@@ -1734,7 +1732,7 @@ void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shall
             const Group& g = gs[gi];
             const uint32_t gb = gbk ? (*gbk)[gi] : bucket;
             if (g.n <= 0) continue;
-            if (single_copy(g, gb) && run_item >= 0 && run_len < kMaxRun && out->items[run_item].n == (uint32_t)g.n &&
+            if (single_copy(g) && run_item >= 0 && run_len < kMaxRun && out->items[run_item].n == (uint32_t)g.n &&
                 out->items[run_item].bucket == gb) {
                 bool ok;
                 if (run_len == 1) {
@@ -1775,24 +1773,26 @@ void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shall
             out->pool.insert(out->pool.end(), g.leaves.begin(), g.leaves.end());
             const uint32_t out_off = (uint32_t)out->pool.size();
             out->pool.insert(out->pool.end(), g.outs.begin(), g.outs.end());
-            // vectors need every address dword-aligned; the body starts where the first output's offset is
-            // a whole number of vectors (outputs sharing its residue then store without realignment)
+            // the body starts where the first output's offset is a whole number of vectors (outputs sharing its
+            // residue then store without realignment)
             const int64_t res = (g.outs.empty() ? g.leaves[0].off : g.outs[0].off) % vec;
-            bool same = vec_bucket(gb);
-            for (const PoolEntry& e : g.leaves) same &= word_ok(e);
-            for (const PoolEntry& e : g.outs) same &= word_ok(e);
+            bool words = true;
+            for (const PoolEntry& e : g.leaves) words &= word_ok(e);
+            for (const PoolEntry& e : g.outs) words &= word_ok(e);
+            const uint16_t vec_flag = words ? ITEM_VEC : ITEM_ANY;
             uint32_t tiles = 0;
-            auto emit = [&](int64_t d, int64_t n, bool v) {
+            auto emit = [&](int64_t d, int64_t n, bool v, int64_t pad = 0) {
                 tile_no.push_back(tiles++);
                 GredItem it{};
                 it.leaf_off = leaf_off;
                 it.out_off = out_off;
                 it.lg = g.lg;
-                it.flags = v ? ITEM_VEC : 0;
+                it.flags = v ? vec_flag : 0;
                 it.nouts = (uint32_t)g.outs.size();
                 it.delta = (uint32_t)d;
                 it.n = (uint32_t)n;
                 it.bucket = gb;
+                it.pad = (uint32_t)pad;
                 out->items.push_back(it);
             };
             // two consecutive whole tiles of a long single copy as one copy run: one pass of the copy-run
@@ -1807,7 +1807,7 @@ void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shall
                 out->pool.push_back(PoolEntry{g.outs[0].rb, (uint32_t)(g.outs[0].off + d0)});
                 out->pool.push_back(PoolEntry{0, (uint32_t)n});
                 it.lg = 0;
-                it.flags = ITEM_VEC | ITEM_RUN;
+                it.flags = vec_flag | ITEM_RUN;
                 it.nouts = 1;
                 it.n = (uint32_t)n;
                 it.bucket = gb;
@@ -1816,7 +1816,27 @@ void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shall
             };
             const bool long_copy = g.lg == 0 && g.leaves.size() == 1 && g.outs.size() == 1 && kMaxRun >= 2;
             int64_t d = 0;
-            if (same) {
+            const bool single = g.lg == 0 && g.outs.size() == 1;
+            if (shared_ends && !single && g.n >= vec) {
+                // Vectors that overlap at the block's ends instead of items of single elements, each of which walked
+                // the whole tree on a few lanes, in tiles of one length (whole multiples of eight vectors, 128 bytes)
+                // instead of whole tiles and a short one.  512 ranks, fp32, microseconds before / after: allreduce of
+                // 262146 485 / 339, reduce of 262146 169 / 97; 64 ranks: allreduce of 262147 40.3 / 24.1,
+                // reduce_scatter of 5002 24.8 / 15.6; 32 uneven buckets (4.9 GB) 1037 / 1019.
+                int64_t tv = tile_elems / vec;
+                const int64_t vecs = (g.n + res + vec - 1) / vec;
+                int64_t count = (vecs + tv - 1) / tv;
+                if (count > 1) {
+                    tv = std::min(tv, ((vecs + count - 1) / count + 7) / 8 * 8);
+                    count = (vecs + tv - 1) / tv;
+                }
+                for (int64_t k = 0; k < count; ++k) {
+                    int64_t end = k + 1 == count ? g.n : (k + 1) * tv * vec - res;
+                    if (k + 2 == count && g.n - end < vec) end = g.n - vec;  // the last tile holds a whole vector
+                    emit(d, end - d, true, k ? 0 : res);
+                    d = end;
+                }
+            } else {
                 int64_t head = (vec - res) % vec;
                 if (head > g.n) head = g.n;
                 if (head) emit(0, head, false);
@@ -1829,7 +1849,7 @@ void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shall
                 d += body;
             }
             for (; d < g.n; d += tile_elems) emit(d, std::min(tile_elems, g.n - d), false);
-            if (single_copy(g, gb)) {  // exactly one aligned item: a run may start here
+            if (single_copy(g)) {  // exactly one aligned item: a run may start here
                 run_item = (int64_t)out->items.size() - 1;
                 run_len = 1;
                 run_leaf = g.leaves[0];
@@ -1869,7 +1889,7 @@ void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shall
         }
         std::copy(sorted.begin(), sorted.end(), out->items.begin() + first);
         for (const GredItem& it : sorted) {
-            if (!(it.flags & ITEM_VEC)) continue;
+            if (!(it.flags & (ITEM_VEC | ITEM_ANY))) continue;
             if (it.flags & ITEM_RUN) {  // first output and the per-copy step
                 out->unaligned_outs |= out->pool[it.out_off].off % vec != 0 || out->pool[it.out_off + 1].off % vec != 0;
             } else {
@@ -1944,7 +1964,8 @@ constexpr uint32_t kNarrowThreads = 1024;
 // blocks that fill a small part of a tile.  Microseconds per launch, general / narrow, fp32:
 //   few workgroups: 512 ranks, reduce of 32768 elements (128 workgroups) 27.2 / 16.2, of 98304 (384) 34.6 / 43.8 or
 //     36.7 by workgroup size, of 131072 (512) 43 / 58; 64 ranks, allreduce of 65536 (256) 9.7 / 8.4, of 131072 (512)
-//     14.0 / 14.8; bcast to 512 ranks of 131072 (128) 84 / 44, of 262144 (256) 119 / 107;
+//     14.0 / 14.8; bcast to 512 ranks of 131072 (128) 84 / 44, of 262144 (256) 119 / 107
+//     but of 262146 (257, realigned stores) 156 / 167;
 //   eight leaves or outputs need no spreading: 8 ranks, allreduce of 65536 (64) 4.65 / 4.58, of 131072 (128) 4.9 / 5.1;
 //   short blocks on 512 ranks: allreduce of 65536 (32 vectors a block) 92 / 53, of 262144 (128) 288 / 259; allgather of
 //     256 (64) 101 / 59, of 512 (128) 141 / 140; reduce_scatter of 128 (32) 36.9 / 31.0, of 192 (48) 37.5 / 45.1.
@@ -1952,8 +1973,10 @@ bool narrow_pays(const std::vector<std::vector<Group>>& launches, int vec) {
     if (launches.size() != 1) return false;
     size_t fan = 0;
     uint64_t workgroups = 0, units = 0, short_units = 0;
+    bool reduces = false;
     for (const Group& g : launches[0]) {
         fan = std::max({fan, g.leaves.size(), g.outs.size()});
+        reduces = reduces || g.lg > 0;
         const uint64_t u = (uint64_t)narrow_units(g, vec), ends = g.leaves.size() + g.outs.size();
         const uint64_t tile = g.lg >= 5 ? 64 : 256;
         workgroups += (u + tile - 1) / tile;
@@ -1961,7 +1984,7 @@ bool narrow_pays(const std::vector<std::vector<Group>>& launches, int vec) {
         if (u <= (g.lg > 0 && g.outs.size() == 1 ? 32u : 128u)) short_units += u * ends;
     }
     if (fan < 16) return fan >= 4 && workgroups < 128;
-    return workgroups < 512 || 2 * short_units >= units;
+    return workgroups < (reduces ? 512u : 256u) || 2 * short_units >= units;
 }
 
 void lower_narrow(const std::vector<std::vector<Group>>& launches, int vec, uint32_t bucket, size_t dtsize,

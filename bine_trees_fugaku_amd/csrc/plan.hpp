@@ -118,16 +118,18 @@ struct Lowered {
 // Groups whose tree has at least 2^deep_lg leaves use deep_tile_elems instead:
 // the kernel splits their leaves across the waves of a workgroup, so their
 // tile is one wave wide.
-// group_bucket (one launch only): the buffer-table index of every group, instead of `bucket`;
-// bucket_vec: per buffer table, whether its addresses allow 16-byte vector access (no ITEM_VEC otherwise).
+// group_bucket (one launch only): the buffer-table index of every group, instead of `bucket`.
 // two_phase (1 or 2): a launch holding reductions with several outputs becomes two launches, the reductions
 // writing their first output, then copies of it to the other outputs (1: copies in group order, 2: tile by
 // tile across the groups, as the reductions).  reduction_tiles: tiles per item in the reduction launch of a
 // two-phase lowering (1 or 2).
+// shared_ends: blocks of at least one vector become vector items whose first and last vectors may overlap their
+// neighbours (GredItem::pad), so the elements in them are computed and stored twice: only for lists whose outputs
+// share no memory with their leaves.  Otherwise a block's unaligned ends are items of single elements.
 void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t tile_elems, int vec_elems,
                   uint32_t bucket, size_t dtsize, Lowered* out, int64_t deep_tile_elems = 0, int deep_lg = 99,
-                  const std::vector<uint32_t>* group_bucket = nullptr, const std::vector<uint8_t>* bucket_vec = nullptr,
-                  int two_phase = 0, int reduction_tiles = 1);
+                  const std::vector<uint32_t>* group_bucket = nullptr, int two_phase = 0, int reduction_tiles = 1,
+                  bool shared_ends = false);
 // Whether a list (one launch, at the general launch shape) is better run by the narrow kernel (gnarrow.hip).
 bool narrow_pays(const std::vector<std::vector<Group>>& launches, int vec_elems);
 // The list as ITEM_NARROW items; same groups, same results.  Arguments as for lower_groups.
