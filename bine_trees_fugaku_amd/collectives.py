@@ -165,7 +165,7 @@ class VComm:
 
     # ---- MPI entry points (lib/libbine.cc) --------------------------------------
     def allreduce(self, sendbuf, recvbuf, op: str = "SUM", stream=None):
-        """MPI_Allreduce (lib/libbine.cc:1012).  sendbuf is recvbuf: MPI_IN_PLACE (per-step schedule)."""
+        """MPI_Allreduce (lib/libbine.cc:1012).  sendbuf is recvbuf: MPI_IN_PLACE."""
         count = self._per_rank(sendbuf)
         self._expect(recvbuf, self.size * count, "recvbuf", sendbuf)
         _lib.check(self._lib.bine_allreduce(sendbuf.data_ptr(), recvbuf.data_ptr(), count, _torch_dtype_code(sendbuf),

@@ -162,15 +162,14 @@ int max_lg_of(const std::vector<std::vector<Group>>& gs) {
     return m;
 }
 
-// fused: the groups' outputs share no memory with their leaves (every fused list)
-int upload(const std::vector<std::vector<Group>>& gs, size_t ds, const LaunchShape& sh, bool fused, DevArrays* d,
+int upload(const std::vector<std::vector<Group>>& gs, size_t ds, const LaunchShape& sh, Ends ends, DevArrays* d,
            Retired* retire = nullptr) {
     Lowered low;
     if (use_narrow(gs, ds, sh))
         lower_narrow(gs, (int)(16 / ds), 0, ds, &low);
     else
         lower_groups(gs, shallow_tile_elems(sh, ds), (int)(16 / ds), 0, ds, &low, deep_tile_elems(sh, ds),
-                     split_lg(sh), nullptr, sh.two_phase, sh.double_tiles ? 2 : 1, fused && !write_heavy(gs));
+                     split_lg(sh), nullptr, sh.two_phase, sh.double_tiles ? 2 : 1, write_heavy(gs) ? Ends::EXACT : ends);
     return install(std::move(low), max_lg_of(gs), shallow_tile_elems(sh, ds), sh, d, retire);
 }
 
@@ -196,6 +195,7 @@ struct DevPlan {
         if (tmp_done) (void)hipEventDestroy(tmp_done);
     }
     size_t tmp_total() const { return tmp_bytes[0] + tmp_bytes[1]; }
+    Ends fused_ends() const { return cp.aliased ? Ends::IN_PLACE : Ends::SHARED; }
 };
 
 struct PlanKey {
@@ -308,16 +308,16 @@ int get_plan(bine_vcomm_t comm, const CollRequest& req, int dtype, std::shared_p
     }
     dp->dtype = dtype;
     dp->ds = ds;
-    int rc = upload(dp->cp.step_groups, ds, default_shape(), false, &dp->step);
+    int rc = upload(dp->cp.step_groups, ds, default_shape(), Ends::EXACT, &dp->step);
     if (rc) return rc;
-    if (dp->cp.fused_ok && max_lg_of(std::vector<std::vector<Group>>(1, dp->cp.fused)) > 14) {
-        dp->cp.fused_ok = false;  // the kernel's register stack holds trees of up to 2^14 leaves
+    if (dp->cp.auto_fused && max_lg_of(std::vector<std::vector<Group>>(1, dp->cp.fused)) > 14) {
+        dp->cp.fused_ok = dp->cp.auto_fused = false;  // the kernel's register stack holds trees of up to 2^14 leaves
         dp->cp.fused.clear();
         dp->cp.fused_why = "reduction tree wider than 2^14 leaves";
     }
-    if (dp->cp.fused_ok) {
+    if (dp->cp.auto_fused) {
         std::vector<std::vector<Group>> one(1, dp->cp.fused);
-        rc = upload(one, ds, initial_shape(one, ds), true, &dp->fused);
+        rc = upload(one, ds, initial_shape(one, ds), dp->fused_ends(), &dp->fused);
         if (rc) return rc;
     }
     // temporaries are allocated only when some step touches them
@@ -492,9 +492,22 @@ int launch_step_ordered(bine_vcomm_t comm, DevPlan* dp, const BufTable& tab, hip
     return BINE_OK;
 }
 
+// The execution mode of one call: the vcomm's, AUTO resolved.
+int choose_exec(bine_vcomm_t comm, const DevPlan* dp, bool in_place, int* out) {
+    const int exec = comm->cfg.exec;
+    if (in_place && exec == BINE_EXEC_FUSED)
+        return fail(BINE_ERR_UNSUPPORTED, "fused execution cannot run in place (sendbuf == recvbuf)");
+    if (exec == BINE_EXEC_FUSED && !dp->cp.fused_ok)
+        return fail(BINE_ERR_UNSUPPORTED, "schedule cannot be fused: " + dp->cp.fused_why);
+    *out = exec != BINE_EXEC_AUTO ? exec : dp->cp.auto_fused ? BINE_EXEC_FUSED : BINE_EXEC_STEP;
+    return BINE_OK;
+}
+
 // Run a collective call end to end.  sendbuf == recvbuf (allreduce only) is MPI_IN_PLACE: the input is read
 // from recvbuf by a schedule compiled and race-checked for that aliasing.
-int run_coll(bine_vcomm_t comm, const CollRequest& req0, int dtype, const void* send, void* recv, void* stream) {
+// tune: the list an autotune is timing (BINE_EXEC_STEP or BINE_EXEC_FUSED, whatever the vcomm's mode).
+int run_coll(bine_vcomm_t comm, const CollRequest& req0, int dtype, const void* send, void* recv, void* stream,
+             int tune = -1) {
     if (!comm) return fail(BINE_ERR_ARG, "NULL vcomm");
     CollRequest req = req0;
     std::shared_ptr<DevPlan> dpp;
@@ -511,12 +524,8 @@ int run_coll(bine_vcomm_t comm, const CollRequest& req0, int dtype, const void* 
     DevPlan* dp = dpp.get();
     if ((rc = check_range(send, sbytes, "sendbuf"))) return rc;
     if ((rc = check_range(recv, rbytes, "recvbuf"))) return rc;
-    int exec = comm->cfg.exec;
-    if (req.in_place && exec == BINE_EXEC_FUSED)
-        return fail(BINE_ERR_UNSUPPORTED, "fused execution cannot run in place (sendbuf == recvbuf)");
-    if (exec == BINE_EXEC_FUSED && !dp->cp.fused_ok)
-        return fail(BINE_ERR_UNSUPPORTED, "schedule cannot be fused: " + dp->cp.fused_why);
-    if (exec == BINE_EXEC_AUTO) exec = dp->cp.fused_ok ? BINE_EXEC_FUSED : BINE_EXEC_STEP;
+    int exec = tune;
+    if (tune < 0 && (rc = choose_exec(comm, dp, req.in_place, &exec))) return rc;
     if (exec == BINE_EXEC_STEP && (rc = ensure_tmp(comm, dp))) return rc;
     HIPCHK(hipSetDevice(comm->cfg.device));
     BufTable tab = make_table(dp, req.in_place ? recv : send, recv);
@@ -741,15 +750,12 @@ extern "C" int bine_allreduce_noalloc(const void* sendbuf, void* recvbuf, int co
     int rc;
     if ((rc = check_range(req.in_place ? nullptr : sendbuf, req.in_place ? 0 : bytes, "sendbuf"))) return rc;
     if ((rc = check_range(recvbuf, bytes, "recvbuf"))) return rc;
-    int exec = comm->cfg.exec;
-    if (req.in_place && exec == BINE_EXEC_FUSED)
-        return fail(BINE_ERR_UNSUPPORTED, "fused execution cannot run in place (sendbuf == recvbuf)");
-    if (exec == BINE_EXEC_FUSED && !dp->cp.fused_ok)
-        return fail(BINE_ERR_UNSUPPORTED, "schedule cannot be fused: " + dp->cp.fused_why);
-    if (exec == BINE_EXEC_AUTO) exec = dp->cp.fused_ok ? BINE_EXEC_FUSED : BINE_EXEC_STEP;
+    int exec = BINE_EXEC_AUTO;
+    if ((rc = choose_exec(comm, dp, req.in_place, &exec))) return rc;
     HIPCHK(hipSetDevice(comm->cfg.device));
     BufTable tab = make_table(dp, req.in_place ? recvbuf : sendbuf, recvbuf);
-    if (exec == BINE_EXEC_STEP && dp->tmp_total()) {
+    // the sizes served are those whose per-step schedule fits, also where AUTO runs an in-place list fused
+    if ((exec == BINE_EXEC_STEP || req.in_place) && dp->tmp_total()) {
         // the per-step temporaries come from the device's scratch array instead of the plan's allocations
         const size_t need = align256(dp->tmp_bytes[0]) + dp->tmp_bytes[1];
         if (need > scratch_bytes())
@@ -831,8 +837,8 @@ extern "C" int bine_plan_stats(bine_vcomm_t comm, int32_t coll, int count, bine_
     int rc = get_plan(comm, r, datatype, &dpp);
     if (rc) return rc;
     const DevPlan* dp = dpp.get();
-    if (exec == BINE_EXEC_AUTO) exec = dp->cp.fused_ok ? BINE_EXEC_FUSED : BINE_EXEC_STEP;
     if (exec == BINE_EXEC_FUSED && !dp->cp.fused_ok) return fail(BINE_ERR_UNSUPPORTED, "schedule cannot be fused: " + dp->cp.fused_why);
+    if (exec == BINE_EXEC_AUTO) exec = dp->cp.auto_fused ? BINE_EXEC_FUSED : BINE_EXEC_STEP;
     const DevArrays& d = exec == BINE_EXEC_FUSED ? dp->fused : dp->step;
     out->launches = kernel_launches(d.low);
     out->items = d.low.items.size();
@@ -875,29 +881,6 @@ std::vector<LaunchShape> two_phase_trials(std::vector<std::pair<float, LaunchSha
     return out;
 }
 
-// Issue one call of a collective (argument layout of its entry point).
-int issue(bine_vcomm_t comm, int32_t coll, const void* send, void* recv, int count, int dtype, int op, int root,
-          void* stream) {
-    switch (coll) {
-    case BINE_COLL_ALLREDUCE: return bine_allreduce(send, recv, count, (bine_datatype_t)dtype, (bine_op_t)op, comm, stream);
-    case BINE_COLL_REDUCE_SCATTER: {
-        std::vector<int> rc(comm->t.size, count);
-        return bine_reduce_scatter(send, recv, rc.data(), (bine_datatype_t)dtype, (bine_op_t)op, comm, stream);
-    }
-    case BINE_COLL_ALLGATHER:
-        return bine_allgather(send, count, (bine_datatype_t)dtype, recv, count, (bine_datatype_t)dtype, comm, stream);
-    case BINE_COLL_BCAST: return bine_bcast(recv, count, (bine_datatype_t)dtype, root, comm, stream);
-    case BINE_COLL_ALLTOALL:
-        return bine_alltoall(send, count, (bine_datatype_t)dtype, recv, count, (bine_datatype_t)dtype, comm, stream);
-    case BINE_COLL_SCATTER:
-        return bine_scatter(send, count, (bine_datatype_t)dtype, recv, count, (bine_datatype_t)dtype, root, comm, stream);
-    case BINE_COLL_GATHER:
-        return bine_gather(send, count, (bine_datatype_t)dtype, recv, count, (bine_datatype_t)dtype, root, comm, stream);
-    case BINE_COLL_REDUCE: return bine_reduce(send, recv, count, (bine_datatype_t)dtype, (bine_op_t)op, root, comm, stream);
-    default: return fail(BINE_ERR_ARG, "unknown collective");
-    }
-}
-
 }  // namespace
 
 extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* sendbuf, void* recvbuf, int count,
@@ -910,13 +893,13 @@ extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* s
     int rc = get_plan(comm, r, datatype, &dpp);
     if (rc) return rc;
     DevPlan* dp = dpp.get();
-    if (exec == BINE_EXEC_AUTO) exec = dp->cp.fused_ok ? BINE_EXEC_FUSED : BINE_EXEC_STEP;
     if (exec == BINE_EXEC_FUSED && !dp->cp.fused_ok) return fail(BINE_ERR_UNSUPPORTED, "schedule cannot be fused");
+    if (exec == BINE_EXEC_AUTO) exec = dp->cp.auto_fused ? BINE_EXEC_FUSED : BINE_EXEC_STEP;
+    const Ends ends = exec == BINE_EXEC_FUSED ? dp->fused_ends() : Ends::EXACT;
+    if (coll == BINE_COLL_BCAST) sendbuf = nullptr;  // as in bine_bcast
     DevArrays& d = exec == BINE_EXEC_FUSED ? dp->fused : dp->step;
     const std::vector<std::vector<Group>> one(1, dp->cp.fused);
     const std::vector<std::vector<Group>>& groups = exec == BINE_EXEC_FUSED ? one : dp->cp.step_groups;
-    const int32_t saved_exec = comm->cfg.exec;
-    comm->cfg.exec = exec;
     HIPCHK(hipSetDevice(comm->cfg.device));
     int cus = 256;
     hipDeviceProp_t prop;
@@ -934,14 +917,14 @@ extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* s
     auto trial = [&](const LaunchShape& c) {
         // the arrays in place before the call may be named by captured graphs: they are kept, not freed;
         // the candidates' own arrays never leave this loop
-        if ((rc = upload(groups, dp->ds, c, exec == BINE_EXEC_FUSED, &d, first ? &dp->retired : nullptr))) return;
+        if ((rc = upload(groups, dp->ds, c, ends, &d, first ? &dp->retired : nullptr))) return;
         first = false;
-        if ((rc = issue(comm, coll, sendbuf, recvbuf, count, datatype, op, root, stream))) return;
+        if ((rc = run_coll(comm, r, datatype, sendbuf, recvbuf, stream, exec))) return;
         if (hipEventRecord(e0, st) != hipSuccess) {
             rc = fail(BINE_ERR_HIP, "event");
             return;
         }
-        for (int i = 0; i < iters && !rc; ++i) rc = issue(comm, coll, sendbuf, recvbuf, count, datatype, op, root, stream);
+        for (int i = 0; i < iters && !rc; ++i) rc = run_coll(comm, r, datatype, sendbuf, recvbuf, stream, exec);
         if (rc) return;
         (void)hipEventRecord(e1, st);
         (void)hipEventSynchronize(e1);
@@ -964,9 +947,8 @@ extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* s
         }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    comm->cfg.exec = saved_exec;
     if (rc) return rc;
-    return upload(groups, dp->ds, bestc, exec == BINE_EXEC_FUSED, &d);
+    return upload(groups, dp->ds, bestc, ends, &d);
 }
 
 extern "C" int bine_plan_dump(const bine_vcomm_config_t* cfg, int32_t coll, int count, bine_datatype_t datatype,
@@ -988,8 +970,8 @@ extern "C" int bine_plan_dump(const bine_vcomm_config_t* cfg, int32_t coll, int 
     std::string err;
     if (!build_program(t, *cfg, r, &prog, &err)) return fail(BINE_ERR_UNSUPPORTED, err);
     if (!compile_program(prog, true, &cp, &err)) return fail(BINE_ERR_UNSUPPORTED, err);
-    if (exec == BINE_EXEC_AUTO) exec = cp.fused_ok ? BINE_EXEC_FUSED : BINE_EXEC_STEP;
     if (exec == BINE_EXEC_FUSED && !cp.fused_ok) return fail(BINE_ERR_UNSUPPORTED, "schedule cannot be fused: " + cp.fused_why);
+    if (exec == BINE_EXEC_AUTO) exec = cp.auto_fused ? BINE_EXEC_FUSED : BINE_EXEC_STEP;
     LaunchShape sh = default_shape();
     int64_t deep = deep_tile_elems(sh, ds);
     const bool narrow = tile_elems == -1, shared_ends = tile_elems < -1;
@@ -1001,7 +983,8 @@ extern "C" int bine_plan_dump(const bine_vcomm_config_t* cfg, int32_t coll, int 
         lower_narrow(std::vector<std::vector<Group>>(1, cp.fused), (int)(16 / ds), 0, ds, &low);
     else if (exec == BINE_EXEC_FUSED)
         lower_groups(std::vector<std::vector<Group>>(1, cp.fused), tile_elems, (int)(16 / ds), 0, ds, &low, deep, split_lg(sh),
-                     nullptr, two_phase & 3, (two_phase & 4) ? 2 : 1, shared_ends);
+                     nullptr, two_phase & 3, (two_phase & 4) ? 2 : 1,
+                     !shared_ends ? Ends::EXACT : cp.aliased ? Ends::IN_PLACE : Ends::SHARED);
     else
         lower_groups(cp.step_groups, tile_elems, (int)(16 / ds), 0, ds, &low, deep, split_lg(sh), nullptr,
                      two_phase & 3, (two_phase & 4) ? 2 : 1);
@@ -1154,6 +1137,7 @@ struct bine_batch_s {
         std::vector<uint32_t> group_bucket;      // bucket of each group
         DevArrays arr;
         LaunchShape shape = default_shape();     // each element type is tuned on its own
+        Ends ends = Ends::SHARED;                // IN_PLACE when some item runs in place
         bool realign = false;                    // launched with the realigning kernels (realign_pays)
     };
     std::vector<TypeList> lists;
@@ -1185,7 +1169,7 @@ int lower_list(bine_batch_t b, bine_batch_s::TypeList& l) {
         else
             lower_groups(l.groups, shallow_tile_elems(l.shape, ds), (int)(16 / ds), 0, ds, &all,
                          deep_tile_elems(l.shape, ds), split_lg(l.shape), &l.group_bucket, l.shape.two_phase,
-                         l.shape.double_tiles ? 2 : 1, !write_heavy(l.groups));
+                         l.shape.double_tiles ? 2 : 1, write_heavy(l.groups) ? Ends::EXACT : l.ends);
         int max_lg = max_lg_of(l.groups);
         bool tables_off16 = false;
         for (uint32_t gb : l.group_bucket) tables_off16 = tables_off16 || off16(b->tabs[gb]);
@@ -1235,7 +1219,7 @@ int batch_run(bine_batch_t b, hipStream_t st) {
         int rc = run_list(b, l, st);
         if (rc) return rc;
     }
-    // collectives whose schedule cannot be fused run their step launches after
+    // collectives whose schedule has no fused list run their step launches after
     for (size_t i = 0; i < b->items.size(); ++i) {
         if (b->use_fused[i]) continue;
         int rc = launch_step_ordered(b->comm, b->plans[i].get(), b->tabs[i], st);
@@ -1255,7 +1239,7 @@ extern "C" int bine_batch_create(bine_vcomm_t comm, const bine_batch_item_t* ite
         const bine_batch_item_t& it = items[i];
         if (it.count < 0) return fail(BINE_ERR_ARG, "negative count");
         CollRequest r{it.coll, it.count, it.op, it.root};
-        // an allreduce with sendbuf == recvbuf runs its in-place schedule per step
+        // an allreduce with sendbuf == recvbuf has a schedule of its own
         r.in_place = it.coll == BINE_COLL_ALLREDUCE && it.sendbuf && it.sendbuf == it.recvbuf;
         std::shared_ptr<DevPlan> dpp;
         int rc = get_plan(comm, r, it.datatype, &dpp);
@@ -1269,7 +1253,8 @@ extern "C" int bine_batch_create(bine_vcomm_t comm, const bine_batch_item_t* ite
             return fail(BINE_ERR_ARG, "batch item buffers overlap");
         if (r.in_place && comm->cfg.exec == BINE_EXEC_FUSED)
             return fail(BINE_ERR_UNSUPPORTED, "fused execution cannot run in place (sendbuf == recvbuf)");
-        const bool fuse = dp->cp.fused_ok && comm->cfg.exec != BINE_EXEC_STEP;
+        const bool fuse = comm->cfg.exec == BINE_EXEC_AUTO ? dp->cp.auto_fused
+                                                           : dp->cp.fused_ok && comm->cfg.exec != BINE_EXEC_STEP;
         if (!fuse && (rc = ensure_tmp(comm, dp))) return rc;
         b->plans.push_back(dpp);
         b->tabs.push_back(make_table(dp, r.in_place ? it.recvbuf : send, it.recvbuf));
@@ -1280,6 +1265,7 @@ extern "C" int bine_batch_create(bine_vcomm_t comm, const bine_batch_item_t* ite
             b->lists.push_back(bine_batch_s::TypeList{it.datatype, std::vector<std::vector<Group>>(1), {}, DevArrays()});
             lit = b->lists.end() - 1;
         }
+        if (dp->cp.aliased) lit->ends = Ends::IN_PLACE;
         for (const Group& g : dp->cp.fused) {
             lit->groups[0].push_back(g);
             lit->group_bucket.push_back((uint32_t)i);

@@ -82,9 +82,11 @@ struct CompiledPlan {
     int64_t extent[kNumBufs] = {0, 0, 0, 0};
     bool single[kNumBufs] = {false, false, false, false};
     std::vector<std::vector<Group>> step_groups;  // STEP execution: one launch per entry
-    std::vector<Group> fused;                     // FUSED execution (empty when not realisable)
-    bool fused_ok = false;
-    std::string fused_why;
+    std::vector<Group> fused;                     // the fused list (empty when not realisable)
+    bool fused_ok = false;                        // exec = FUSED may run it
+    bool auto_fused = false;                      // exec = AUTO runs it
+    bool aliased = false;                         // its outputs are its own leaves' memory (an in-place allreduce)
+    std::string fused_why;                        // why fused_ok is false
 };
 
 struct CollRequest {
@@ -123,13 +125,17 @@ struct Lowered {
 // writing their first output, then copies of it to the other outputs (1: copies in group order, 2: tile by
 // tile across the groups, as the reductions).  reduction_tiles: tiles per item in the reduction launch of a
 // two-phase lowering (1 or 2).
-// shared_ends: blocks of at least one vector become vector items whose first and last vectors may overlap their
-// neighbours (GredItem::pad), so the elements in them are computed and stored twice: only for lists whose outputs
-// share no memory with their leaves.  Otherwise a block's unaligned ends are items of single elements.
+// ends: how the unaligned ends of a block of at least one vector are handled.
+enum class Ends {
+    EXACT,     // items of single elements (lists whose outputs may share memory with other elements' leaves)
+    SHARED,    // vector items whose first and last vectors may overlap their neighbours (GredItem::pad): the elements
+               // in them are computed and stored twice.  Only for lists whose outputs share no memory with their leaves.
+    IN_PLACE,  // SHARED where the outputs are the item's own leaves and the tile allows it, else EXACT
+};
 void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t tile_elems, int vec_elems,
                   uint32_t bucket, size_t dtsize, Lowered* out, int64_t deep_tile_elems = 0, int deep_lg = 99,
                   const std::vector<uint32_t>* group_bucket = nullptr, int two_phase = 0, int reduction_tiles = 1,
-                  bool shared_ends = false);
+                  Ends ends = Ends::EXACT);
 // Whether a list (one launch, at the general launch shape) is better run by the narrow kernel (gnarrow.hip).
 bool narrow_pays(const std::vector<std::vector<Group>>& launches, int vec_elems);
 // The list as ITEM_NARROW items; same groups, same results.  Arguments as for lower_groups.

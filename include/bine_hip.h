@@ -31,9 +31,10 @@
  * their own schedules.
  *
  * MPI_IN_PLACE: bine_allreduce with sendbuf == recvbuf reads the input from
- * recvbuf.  It runs the per-step schedule compiled for that aliasing (every
- * algorithm: B and B_CONT drop their initial copy, L keeps its running value
- * off RECV at the first step); other collectives reject overlapping buffers.
+ * recvbuf.  It runs a schedule compiled for that aliasing (every algorithm: B
+ * and B_CONT drop their initial copy, L keeps its running value off RECV at the
+ * first step), as one launch under AUTO where every output lies on its own
+ * reduction's leaves, else per step; other collectives reject overlapping buffers.
  *
  * Per-step runs of one schedule share its temporaries.  Outside graph
  * capture, each such run waits on the GPU for the previous one, whatever
@@ -275,8 +276,9 @@ typedef struct bine_batch_s* bine_batch_t;
 
 /* Compile `n` collectives on one vcomm into one fused work list.  The buffers
  * are bound here and must stay allocated, and the vcomm alive, until
- * bine_batch_destroy.  An allreduce item with sendbuf == recvbuf runs in place,
- * per step, after the fused lists.  Retuning a batch (set_tuning, autotune)
+ * bine_batch_destroy.  An allreduce item with sendbuf == recvbuf runs in place:
+ * with the fused lists where its schedule allows (powers of two, algorithms B and
+ * B_CONT), else per step after them.  Retuning a batch (set_tuning, autotune)
  * replaces its work lists: graphs the caller captured from bine_batch_launch
  * before that must be captured again (bine_batch_launch_graph does so itself). */
 int bine_batch_create(bine_vcomm_t comm, const bine_batch_item_t* items, int n, bine_batch_t* out);
