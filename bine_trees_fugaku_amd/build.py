@@ -35,6 +35,7 @@ SOURCES = [
     ("gred.hip", "hip"),
     ("gred_realign.hip", "hip"),
     ("gnarrow.hip", "hip"),
+    ("gtree.hip", "hip"),
     ("sim.hip", "hip"),
     ("mlp.hip", "hip"),
     ("scratch.hip", "hip"),

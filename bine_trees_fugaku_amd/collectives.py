@@ -290,15 +290,17 @@ def plan_dump(dims: Sequence[int], coll: str, count: int, dtype, op: str = "SUM"
     """Compile a schedule on the host (no GPU) and return its lowered work as
     numpy arrays: (info dict, items structured array, pool structured array,
     launches (n, 2) array).  tile_elems: elements per tile, 0 for the general shape's, -1 for the narrow list a small
-    call uploads, -t for tiles of up to t elements whose end vectors overlap their neighbours.  in_place: the allreduce schedule for sendbuf == recvbuf.
+    call uploads, -t for tiles of up to t elements whose end vectors overlap their neighbours.  in_place: the allreduce
+    schedule for sendbuf == recvbuf.  exec: also "TREES", the list of general trees that AUTO runs on tori that are no
+    powers of two.
     two_phase: 1 or 2 lowers reductions with several outputs as two launches (see Batch.set_tuning); adding 4
     gives the reduction launch items of two tiles."""
     import numpy as np
     L = _lib.load()
     cfg = make_config(dims, num_ports=num_ports, **overrides)
     info = _lib.PlanDumpInfo()
-    args = (ctypes.byref(cfg), COLL[coll], count, _dtype_code(dtype), OP[op], root, 1 if in_place else 0, EXEC[exec],
-            tile_elems, two_phase, ctypes.byref(info))
+    args = (ctypes.byref(cfg), COLL[coll], count, _dtype_code(dtype), OP[op], root, 1 if in_place else 0,
+            3 if exec == "TREES" else EXEC[exec], tile_elems, two_phase, ctypes.byref(info))
     _lib.check(L.bine_plan_dump(*args, None, None, None), "bine_plan_dump")
     item_dt = np.dtype([("leaf_off", "<u4"), ("out_off", "<u4"), ("lg", "<u2"), ("flags", "<u2"), ("nouts", "<u4"),
                         ("delta", "<u4"), ("n", "<u4"), ("bucket", "<u4"), ("pad", "<u4")])

@@ -29,6 +29,8 @@ hipError_t launch_grun(uint32_t esize, const GredItem* items, uint32_t n, const 
                        const BufTable* tabs, bool batch, const LaunchShape& sh, hipStream_t st);
 hipError_t launch_gnarrow(int dtype, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
                           const BufTable* tabs, bool batch, int threads, hipStream_t st);
+hipError_t launch_gtree(int dtype, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
+                        const BufTable* tabs, bool batch, int waves, int stack, hipStream_t st);
 hipError_t launch_reduce_local(int dtype, const void* a, const void* b, void* out, uint64_t n, hipStream_t st);
 size_t scratch_bytes();
 hipError_t scratch_init(int device);
@@ -162,10 +164,12 @@ int max_lg_of(const std::vector<std::vector<Group>>& gs) {
     return m;
 }
 
-int upload(const std::vector<std::vector<Group>>& gs, size_t ds, const LaunchShape& sh, Ends ends, DevArrays* d,
-           Retired* retire = nullptr) {
+int upload(const std::vector<std::vector<Group>>& gs, size_t ds, const LaunchShape& sh, Ends ends, bool trees,
+           DevArrays* d, Retired* retire = nullptr) {
     Lowered low;
-    if (use_narrow(gs, ds, sh))
+    if (trees)
+        lower_trees(gs[0], (int)(16 / ds), 0, ds, &low);
+    else if (use_narrow(gs, ds, sh))
         lower_narrow(gs, (int)(16 / ds), 0, ds, &low);
     else
         lower_groups(gs, shallow_tile_elems(sh, ds), (int)(16 / ds), 0, ds, &low, deep_tile_elems(sh, ds),
@@ -308,7 +312,7 @@ int get_plan(bine_vcomm_t comm, const CollRequest& req, int dtype, std::shared_p
     }
     dp->dtype = dtype;
     dp->ds = ds;
-    int rc = upload(dp->cp.step_groups, ds, default_shape(), Ends::EXACT, &dp->step);
+    int rc = upload(dp->cp.step_groups, ds, default_shape(), Ends::EXACT, false, &dp->step);
     if (rc) return rc;
     if (dp->cp.auto_fused && max_lg_of(std::vector<std::vector<Group>>(1, dp->cp.fused)) > 14) {
         dp->cp.fused_ok = dp->cp.auto_fused = false;  // the kernel's register stack holds trees of up to 2^14 leaves
@@ -317,7 +321,7 @@ int get_plan(bine_vcomm_t comm, const CollRequest& req, int dtype, std::shared_p
     }
     if (dp->cp.auto_fused) {
         std::vector<std::vector<Group>> one(1, dp->cp.fused);
-        rc = upload(one, ds, initial_shape(one, ds), dp->fused_ends(), &dp->fused);
+        rc = upload(one, ds, initial_shape(one, ds), dp->fused_ends(), dp->cp.trees, &dp->fused);
         if (rc) return rc;
     }
     // temporaries are allocated only when some step touches them
@@ -457,6 +461,12 @@ int launch_arrays(const DevArrays& d, int dtype, const BufTable& tab, hipStream_
     const bool realign = realign_pays(d.low, off16(tab));
     for (size_t li = 0; li < d.low.launches.size(); ++li) {
         const auto& l = d.low.launches[li];
+        if (d.low.tree_waves) {
+            hipError_t e = launch_gtree(dtype, d.items + l.first, l.second, d.pool, tab, nullptr, false,
+                                        d.low.tree_waves, d.low.tree_stack, st);
+            if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("tree launch: ") + hipGetErrorString(e));
+            continue;
+        }
         if (d.low.narrow_threads) {
             hipError_t e = launch_gnarrow(dtype, d.items + l.first, l.second, d.pool, tab, nullptr, false,
                                           d.low.narrow_threads, st);
@@ -896,6 +906,7 @@ extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* s
     if (exec == BINE_EXEC_FUSED && !dp->cp.fused_ok) return fail(BINE_ERR_UNSUPPORTED, "schedule cannot be fused");
     if (exec == BINE_EXEC_AUTO) exec = dp->cp.auto_fused ? BINE_EXEC_FUSED : BINE_EXEC_STEP;
     const Ends ends = exec == BINE_EXEC_FUSED ? dp->fused_ends() : Ends::EXACT;
+    const bool trees = exec == BINE_EXEC_FUSED && dp->cp.trees;
     if (coll == BINE_COLL_BCAST) sendbuf = nullptr;  // as in bine_bcast
     DevArrays& d = exec == BINE_EXEC_FUSED ? dp->fused : dp->step;
     const std::vector<std::vector<Group>> one(1, dp->cp.fused);
@@ -917,7 +928,7 @@ extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* s
     auto trial = [&](const LaunchShape& c) {
         // the arrays in place before the call may be named by captured graphs: they are kept, not freed;
         // the candidates' own arrays never leave this loop
-        if ((rc = upload(groups, dp->ds, c, ends, &d, first ? &dp->retired : nullptr))) return;
+        if ((rc = upload(groups, dp->ds, c, ends, trees, &d, first ? &dp->retired : nullptr))) return;
         first = false;
         if ((rc = run_coll(comm, r, datatype, sendbuf, recvbuf, stream, exec))) return;
         if (hipEventRecord(e0, st) != hipSuccess) {
@@ -940,7 +951,7 @@ extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* s
         trial(c);
         if (rc) break;
     }
-    if (!rc && has_multi_output_reduction(groups))
+    if (!rc && !trees && has_multi_output_reduction(groups))
         for (const LaunchShape& c : two_phase_trials(timed)) {
             trial(c);
             if (rc) break;
@@ -948,8 +959,11 @@ extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* s
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc;
-    return upload(groups, dp->ds, bestc, ends, &d);
+    return upload(groups, dp->ds, bestc, ends, trees, &d);
 }
+
+// bine_plan_dump: the list of general trees that AUTO runs where FUSED is refused
+constexpr int kDumpTrees = 3;
 
 extern "C" int bine_plan_dump(const bine_vcomm_config_t* cfg, int32_t coll, int count, bine_datatype_t datatype,
                               bine_op_t op, int root, int32_t in_place, int32_t exec, int64_t tile_elems,
@@ -971,7 +985,9 @@ extern "C" int bine_plan_dump(const bine_vcomm_config_t* cfg, int32_t coll, int 
     if (!build_program(t, *cfg, r, &prog, &err)) return fail(BINE_ERR_UNSUPPORTED, err);
     if (!compile_program(prog, true, &cp, &err)) return fail(BINE_ERR_UNSUPPORTED, err);
     if (exec == BINE_EXEC_FUSED && !cp.fused_ok) return fail(BINE_ERR_UNSUPPORTED, "schedule cannot be fused: " + cp.fused_why);
-    if (exec == BINE_EXEC_AUTO) exec = cp.auto_fused ? BINE_EXEC_FUSED : BINE_EXEC_STEP;
+    const bool trees = exec == kDumpTrees;
+    if (trees && !cp.trees) return fail(BINE_ERR_UNSUPPORTED, "no list of general trees: AUTO runs the steps");
+    if (exec == BINE_EXEC_AUTO) exec = cp.auto_fused && !cp.trees ? BINE_EXEC_FUSED : BINE_EXEC_STEP;
     LaunchShape sh = default_shape();
     int64_t deep = deep_tile_elems(sh, ds);
     const bool narrow = tile_elems == -1, shared_ends = tile_elems < -1;
@@ -979,7 +995,9 @@ extern "C" int bine_plan_dump(const bine_vcomm_config_t* cfg, int32_t coll, int 
     if (tile_elems <= 0) tile_elems = default_tile_elems(ds);
     else deep = tile_elems;
     Lowered low;
-    if (exec == BINE_EXEC_FUSED && narrow)
+    if (trees)
+        lower_trees(cp.fused, (int)(16 / ds), 0, ds, &low);
+    else if (exec == BINE_EXEC_FUSED && narrow)
         lower_narrow(std::vector<std::vector<Group>>(1, cp.fused), (int)(16 / ds), 0, ds, &low);
     else if (exec == BINE_EXEC_FUSED)
         lower_groups(std::vector<std::vector<Group>>(1, cp.fused), tile_elems, (int)(16 / ds), 0, ds, &low, deep, split_lg(sh),
@@ -1137,6 +1155,7 @@ struct bine_batch_s {
         std::vector<uint32_t> group_bucket;      // bucket of each group
         DevArrays arr;
         LaunchShape shape = default_shape();     // each element type is tuned on its own
+        bool trees = false;                      // general trees (a list of their own)
         Ends ends = Ends::SHARED;                // IN_PLACE when some item runs in place
         bool realign = false;                    // launched with the realigning kernels (realign_pays)
     };
@@ -1164,7 +1183,9 @@ int lower_list(bine_batch_t b, bine_batch_s::TypeList& l) {
         // one lowering for the whole list: every work item carries its group's bucket index, runs of copies
         // form within a bucket, and items are ordered tile-major across all buckets
         Lowered all;
-        if (use_narrow(l.groups, ds, l.shape))
+        if (l.trees)
+            lower_trees(l.groups[0], (int)(16 / ds), 0, ds, &all, &l.group_bucket);
+        else if (use_narrow(l.groups, ds, l.shape))
             lower_narrow(l.groups, (int)(16 / ds), 0, ds, &all, &l.group_bucket);
         else
             lower_groups(l.groups, shallow_tile_elems(l.shape, ds), (int)(16 / ds), 0, ds, &all,
@@ -1193,6 +1214,13 @@ int batch_lower(bine_batch_t b) {
 int run_list(bine_batch_t b, const bine_batch_s::TypeList& l, hipStream_t st) {
     const Lowered& low = l.arr.low;
     for (size_t li = 0; li < low.launches.size(); ++li) {
+        if (low.tree_waves) {
+            hipError_t e = launch_gtree(l.dtype, l.arr.items + low.launches[li].first, low.launches[li].second,
+                                        l.arr.pool, BufTable{}, b->d_tabs, true, low.tree_waves,
+                                        low.tree_stack, st);
+            if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("batch tree launch: ") + hipGetErrorString(e));
+            continue;
+        }
         if (low.narrow_threads) {
             hipError_t e = launch_gnarrow(l.dtype, l.arr.items + low.launches[li].first, low.launches[li].second,
                                           l.arr.pool, BufTable{}, b->d_tabs, true, low.narrow_threads, st);
@@ -1260,10 +1288,11 @@ extern "C" int bine_batch_create(bine_vcomm_t comm, const bine_batch_item_t* ite
         b->tabs.push_back(make_table(dp, r.in_place ? it.recvbuf : send, it.recvbuf));
         b->use_fused.push_back(fuse ? 1 : 0);
         if (!fuse) continue;
-        auto lit = std::find_if(b->lists.begin(), b->lists.end(), [&](const bine_batch_s::TypeList& l) { return l.dtype == it.datatype; });
+        auto lit = std::find_if(b->lists.begin(), b->lists.end(), [&](const bine_batch_s::TypeList& l) { return l.dtype == it.datatype && l.trees == dp->cp.trees; });
         if (lit == b->lists.end()) {
             b->lists.push_back(bine_batch_s::TypeList{it.datatype, std::vector<std::vector<Group>>(1), {}, DevArrays()});
             lit = b->lists.end() - 1;
+            lit->trees = dp->cp.trees;
         }
         if (dp->cp.aliased) lit->ends = Ends::IN_PLACE;
         for (const Group& g : dp->cp.fused) {
@@ -1483,7 +1512,7 @@ extern "C" int bine_batch_autotune(bine_batch_t b, void* stream, int iters) {
         for (size_t i = 0; i < nl; ++i)
             if (int rc = trial(i, c)) return rc;
     for (size_t i = 0; i < nl; ++i)
-        if (has_multi_output_reduction(b->lists[i].groups))
+        if (!b->lists[i].trees && has_multi_output_reduction(b->lists[i].groups))
             for (const LaunchShape& c : two_phase_trials(timed[i]))
                 if (int rc = trial(i, c)) return rc;
     size_t dominant = 0;

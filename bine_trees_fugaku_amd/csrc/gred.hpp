@@ -17,6 +17,7 @@ inline PoolEntry make_entry(uint32_t buf, uint32_t rank, uint32_t off) { return 
 enum : uint16_t {
     ITEM_VEC = 1,  // the tile moves as 16-byte vectors, every leaf and output offset dword-aligned
     ITEM_RUN = 2,  // a run of `pad` one-leaf, one-output copies (see GredItem)
+    ITEM_TREE = 16,  // a tile of the tree kernel
     ITEM_ANY = 8,  // the tile moves as 16-byte vectors, offsets at any byte
     ITEM_NARROW = 4,  // a tile of the narrow kernel (gnarrow.hip): any alignment, any length up to its workgroup's units
 };
@@ -26,6 +27,11 @@ enum : uint16_t {
 // (int64, 4 KiB per rank pair) runs of 2 moved 6.2 TB/s, of 4 5.9, of 8 5.9, of 16 5.6 and of 32 5.3 TB/s:
 // longer runs serialise passes inside one workgroup and leave fewer, longer items; unmerged copies ran 5.75.
 constexpr uint32_t kMaxRun = 2;
+
+// Items of the tree kernel (gtree.hip): lg is the number of subtrees, at most one per wave.  The pool holds one entry
+// per subtree at leaf_off (rb: its number of leaves; off: the additions that follow when the subtree sums are joined on
+// a stack), then the subtrees' leaves, each padded to whole groups of eight; a leaf's rb holds the rank in bits 0..23
+// and in bits 24..27 the additions that follow it.
 
 // One tile of one group: elements [delta, delta + n) of the group.
 struct alignas(16) GredItem {

@@ -111,6 +111,34 @@ __device__ __forceinline__ void vstore(char* p, const Vec<T>& v) {
     else *gptr<u4b>(p) = v.raw;
 }
 
+// Units of the narrow and tree kernels: a 16-byte vector at any byte address, or one element.
+template <typename T>
+__device__ __forceinline__ Vec<T> load_unit(const char* p, Vec<T>*) {
+    Vec<T> r;
+    r.raw = *gptr<const u4b>(p);
+    return r;
+}
+template <typename T>
+__device__ __forceinline__ T load_unit(const char* p, T*) {
+    return *gptr<const T>(p);
+}
+template <typename T>
+__device__ __forceinline__ void store_unit(char* p, const Vec<T>& v) {
+    *gptr<u4b>(p) = v.raw;
+}
+template <typename T>
+__device__ __forceinline__ void store_unit(char* p, T v) {
+    *gptr<T>(p) = v;
+}
+template <typename T>
+__device__ __forceinline__ Vec<T> add_unit(const Vec<T>& a, const Vec<T>& b) {
+    return vadd<T>(a, b);
+}
+template <typename T>
+__device__ __forceinline__ T add_unit(T a, T b) {
+    return add1<T>(a, b);
+}
+
 // Buffer address of a (buffer, rank, element offset) entry.  The buffer is
 // picked with masks rather than an indexed or selected load so the table stays
 // in scalar registers.

@@ -1319,6 +1319,7 @@ struct Node {
     uint32_t nleaves;
     uint16_t height;
     bool perfect;
+    uint8_t need;  // partial sums held at once by an evaluation that takes the child needing more first
 };
 
 struct Piece {
@@ -1346,7 +1347,7 @@ public:
             if (p.extent[b] <= 0) continue;
             for (uint32_t r = 0; r < P; ++r) {
                 if (p.single[b] && r != p.root) continue;
-                Node n{0, (uint8_t)b, r, {-1, 0}, {-1, 0}, 1, 0, true};
+                Node n{0, (uint8_t)b, r, {-1, 0}, {-1, 0}, 1, 0, true, 1};
                 nodes.push_back(n);
                 maps[(size_t)b * P + r][0] = Piece{p.extent[b], SymVal{(int32_t)nodes.size() - 1, 0}};
             }
@@ -1385,6 +1386,7 @@ public:
         n.nleaves = na.nleaves + nb.nleaves;
         n.height = (uint16_t)(std::max(na.height, nb.height) + 1);
         n.perfect = na.perfect && nb.perfect && na.height == nb.height;
+        n.need = na.need == nb.need ? (uint8_t)(na.need + 1) : std::max(na.need, nb.need);
         nodes.push_back(n);
         return (int32_t)nodes.size() - 1;
     }
@@ -1472,6 +1474,24 @@ void flatten(const Sym& s, int32_t node, int64_t pos, std::vector<Flat>* out) {
     }
     flatten(s, n.a.node, pos + n.a.delta, out);
     flatten(s, n.b.node, pos + n.b.delta, out);
+}
+
+// The same leaves, each with the number of additions that follow it: evaluated on a stack, an addition joins the two
+// topmost values.  The child that needs more of the stack goes first (the sum of two values does not depend on their
+// order), so the stack stays as low as the tree allows.
+void flatten_postfix(const Sym& s, int32_t node, int64_t pos, std::vector<Flat>* out, std::vector<uint8_t>* pops) {
+    const Node& n = s.nodes[node];
+    if (n.kind == 0) {
+        out->push_back({n.buf, n.rank, pos});
+        pops->push_back(0);
+        return;
+    }
+    const bool swap = s.nodes[n.b.node].need > s.nodes[n.a.node].need;
+    const SymVal& x = swap ? n.b : n.a;
+    const SymVal& y = swap ? n.a : n.b;
+    flatten_postfix(s, x.node, pos + x.delta, out, pops);
+    flatten_postfix(s, y.node, pos + y.delta, out, pops);
+    if (pops->back() < 255) ++pops->back();
 }
 
 struct PairHash {
@@ -1586,6 +1606,8 @@ bool compile_program(const Program& prog, bool want_fused, CompiledPlan* out, st
     std::unordered_map<uint64_t, size_t> group_of;  // (hash, len) -> group index
     std::unordered_map<uint64_t, char> verified;  // (node, pos, expected source) already checked
     bool fused_ok = want_fused;
+    bool perfect = true;  // every tree is
+    bool trees_fit = prog.P < (1u << 24);  // the tree kernel's entries hold 24 bits of rank
     std::string why;
     std::vector<Flat> fl;
     std::vector<char> seen(prog.P);
@@ -1639,9 +1661,8 @@ bool compile_program(const Program& prog, bool want_fused, CompiledPlan* out, st
             // identity output (an input left in place): nothing to write
             if (nd.kind == 0 && nd.buf == o.buf && nd.rank == o.rank && pos == lo) continue;
             if (!nd.perfect) {
-                fused_ok = false;
+                perfect = false;
                 why = "a reduction tree is not perfect (non power-of-two schedule)";
-                continue;
             }
             uint64_t h = canon_hash(sym, v.node, pos, &memo);
             uint64_t gk = mix64(h ^ mix64((uint64_t)(hi - lo)));
@@ -1650,8 +1671,15 @@ bool compile_program(const Program& prog, bool want_fused, CompiledPlan* out, st
                 Group g;
                 g.n = hi - lo;
                 fl.clear();
-                flatten(sym, v.node, pos, &fl);
-                g.lg = (uint16_t)nd.height;
+                if (nd.perfect) {
+                    flatten(sym, v.node, pos, &fl);
+                    g.lg = (uint16_t)nd.height;
+                    trees_fit = trees_fit && nd.height < kMaxTreeStack;
+                } else {
+                    flatten_postfix(sym, v.node, pos, &fl, &g.pops);
+                    g.lg = (uint16_t)ceil_log2((uint32_t)fl.size());
+                    trees_fit = trees_fit && nd.need <= kMaxTreeStack;
+                }
                 for (const Flat& f : fl) g.leaves.push_back(make_entry(f.buf, f.rank, (uint32_t)f.pos));
                 g.outs.push_back(make_entry(o.buf, o.rank, (uint32_t)lo));
                 group_of[gk] = out->fused.size();
@@ -1698,16 +1726,26 @@ bool compile_program(const Program& prog, bool want_fused, CompiledPlan* out, st
                 }
             }
         }
-        if (aliased) {
-            fused_ok = false;
-            why = "an output overlaps an input of the fused launch";
-            out->auto_fused = own;
-        }
+        if (aliased && perfect) why = "an output overlaps an input of the fused launch";
+        out->auto_fused = !aliased || own;
     }
-    if (want_fused && prog.outputs.empty()) fused_ok = false;
+    if (want_fused && prog.outputs.empty()) fused_ok = out->auto_fused = false;
+    if (!perfect) {
+        // general trees pay where they move no more than the schedule's steps do: allreduce L, whose ranks each build a
+        // tree of their own, would read every input once per rank
+        auto moved = [](const std::vector<Group>& gs) {
+            uint64_t n = 0;
+            for (const Group& g : gs) n += (uint64_t)g.n * (g.leaves.size() + g.outs.size());
+            return n;
+        };
+        uint64_t stepped = 0;
+        for (const auto& gs : out->step_groups) stepped += moved(gs);
+        out->auto_fused = out->auto_fused && trees_fit && moved(out->fused) <= stepped;
+        out->trees = out->auto_fused;
+    }
+    fused_ok = fused_ok && perfect && !aliased;
     out->fused_ok = fused_ok;
     out->aliased = aliased && out->auto_fused;
-    out->auto_fused = out->auto_fused || fused_ok;
     out->fused_why = why;
     if (!out->auto_fused) out->fused.clear();
     return true;
@@ -2059,6 +2097,133 @@ void lower_narrow(const std::vector<std::vector<Group>>& launches, int vec, uint
                 it.bucket = group_bucket ? (*group_bucket)[gi] : bucket;
                 out->items.push_back(it);
             }
+            d += n;
+        }
+        out->bytes_read += (uint64_t)g.n * g.leaves.size() * dtsize;
+        out->bytes_written += (uint64_t)g.n * g.outs.size() * dtsize;
+        out->max_leaves = std::max<uint64_t>(out->max_leaves, g.leaves.size());
+    }
+    out->launches.push_back({0, (uint32_t)out->items.size()});
+    out->runs.push_back(0);
+}
+
+namespace {
+
+// A group's tree cut into at most `most` subtrees: their leaf ranges in leaf order, and the additions that follow each
+// when the subtree sums are joined on a stack.
+struct Cut {
+    std::vector<uint32_t> count;
+    std::vector<uint8_t> pops;
+};
+
+struct TreeNode {
+    int32_t a, b;  // children, or -1
+    uint32_t leaves;
+};
+
+void emit_cut(const std::vector<TreeNode>& t, const std::vector<char>& open, int32_t node, Cut* c) {
+    if (!open[node]) {
+        c->count.push_back(t[node].leaves);
+        c->pops.push_back(0);
+        return;
+    }
+    emit_cut(t, open, t[node].a, c);
+    emit_cut(t, open, t[node].b, c);
+    ++c->pops.back();
+}
+
+// additions after leaf k of a balanced tree
+uint8_t balanced_pops(size_t k) { return (uint8_t)__builtin_ctzll(k + 1); }
+
+// stack_need: raised to what the join of the parts needs
+Cut cut_tree(const Group& g, uint32_t most, int* stack_need) {
+    std::vector<TreeNode> t;
+    std::vector<int32_t> stack;
+    for (size_t k = 0; k < g.leaves.size(); ++k) {
+        t.push_back({-1, -1, 1});
+        stack.push_back((int32_t)t.size() - 1);
+        for (int p = g.pops.empty() ? balanced_pops(k) : g.pops[k]; p > 0; --p) {
+            const int32_t b = stack.back();
+            stack.pop_back();
+            t.push_back({stack.back(), b, t[stack.back()].leaves + t[b].leaves});
+            stack.back() = (int32_t)t.size() - 1;
+        }
+    }
+    std::vector<char> open(t.size(), 0);  // nodes joined from their children's sums
+    std::vector<int32_t> parts(1, stack[0]);
+    while (parts.size() < most) {  // open the subtree of most leaves
+        size_t w = 0;
+        for (size_t i = 1; i < parts.size(); ++i)
+            if (t[parts[i]].leaves > t[parts[w]].leaves) w = i;
+        if (t[parts[w]].leaves < 2) break;
+        open[parts[w]] = 1;
+        const int32_t a = t[parts[w]].a, b = t[parts[w]].b;
+        parts[w] = a;
+        parts.push_back(b);
+    }
+    Cut c;
+    emit_cut(t, open, stack[0], &c);
+    int depth = 0;
+    for (uint8_t p : c.pops) {
+        *stack_need = std::max(*stack_need, depth + 1);
+        depth += 1 - p;
+    }
+    return c;
+}
+
+}  // namespace
+
+void lower_trees(const std::vector<Group>& gs, int vec, uint32_t bucket, size_t dtsize, Lowered* out,
+                 const std::vector<uint32_t>* group_bucket) {
+    // Waves per workgroup: one for every 13 leaves, so that two groups of eight loads cover a wave's subtree; lists too
+    // small to fill the chip take one for every three leaves, up to four.  GPU time in microseconds with 1 / 2 / 4 / 8
+    // waves, fp32: 6 ranks of 32768 elements 4.4 / 3.7 / 3.8 / 4.4, of 2097152 19.0 / 20.6 / 28.4 / 50.2; 36 ranks of
+    // 131072 18.6 / 14.8 / 12.8 / 14.2; 100 ranks of 524288 116.8 / 112.7 / 101.3 / 96.3.
+    const int64_t tile = 64;  // units of a workgroup's tile, one per lane
+    size_t leaves = 1;
+    int64_t workgroups = 0;
+    for (const Group& g : gs) {
+        leaves = std::max(leaves, g.leaves.size());
+        workgroups += (narrow_units(g, vec) + tile - 1) / tile;
+    }
+    uint32_t waves = std::min(8u, pow2_at_least((leaves + 12) / 13));
+    if (workgroups < 1024) waves = std::max(waves, std::min(4u, pow2_at_least((leaves + 2) / 3)));
+    out->tree_waves = (int)waves;
+    for (size_t gi = 0; gi < gs.size(); ++gi) {
+        const Group& g = gs[gi];
+        if (g.n <= 0) continue;
+        const Cut c = cut_tree(g, waves, &out->tree_stack);
+        const uint32_t leaf_off = (uint32_t)out->pool.size();
+        for (size_t i = 0; i < c.count.size(); ++i) out->pool.push_back(PoolEntry{c.count[i], c.pops[i]});
+        size_t k = 0;
+        for (uint32_t n : c.count) {
+            uint32_t depth = 0;  // a subtree's last leaf is followed by its own additions only, not its parents'
+            for (uint32_t j = 0; j < n; ++j, ++k) {
+                const uint32_t pops = std::min<uint32_t>(g.pops.empty() ? balanced_pops(k) : g.pops[k], depth);
+                out->pool.push_back(PoolEntry{g.leaves[k].rb | (pops << 24), g.leaves[k].off});
+                out->tree_stack = std::max<int>(out->tree_stack, (int)depth + 1);
+                depth += 1 - pops;
+            }
+            for (uint32_t j = n; j % 8 != 0; ++j) out->pool.push_back(g.leaves[k - 1]);
+        }
+        const uint32_t out_off = (uint32_t)out->pool.size();
+        out->pool.insert(out->pool.end(), g.outs.begin(), g.outs.end());
+        const int64_t u = narrow_units(g, vec), tiles = (u + tile - 1) / tile;
+        const int64_t w = (u + tiles - 1) / tiles, elems = g.n >= vec ? w * vec : w;
+        for (int64_t d = 0; d < g.n;) {
+            int64_t n = std::min(elems, g.n - d);
+            const int64_t rest = g.n - d - n;
+            if (g.n >= vec && rest > 0 && rest < vec) n -= vec;  // the last tile holds a whole vector
+            GredItem it{};
+            it.leaf_off = leaf_off;
+            it.out_off = out_off;
+            it.lg = (uint16_t)c.count.size();
+            it.flags = ITEM_TREE;
+            it.nouts = (uint32_t)g.outs.size();
+            it.delta = (uint32_t)d;
+            it.n = (uint32_t)n;
+            it.bucket = group_bucket ? (*group_bucket)[gi] : bucket;
+            out->items.push_back(it);
             d += n;
         }
         out->bytes_read += (uint64_t)g.n * g.leaves.size() * dtsize;

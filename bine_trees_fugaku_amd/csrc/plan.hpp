@@ -75,7 +75,11 @@ struct Group {
     std::vector<PoolEntry> outs;
     int64_t n = 0;
     uint16_t lg = 0;
+    // not empty: a general tree, evaluated on a stack; pops[k] additions follow leaf k (lg: the rounded-up log2)
+    std::vector<uint8_t> pops;
 };
+
+constexpr int kMaxTreeStack = 12;  // values that the tree kernel's stack holds
 
 struct CompiledPlan {
     uint32_t P = 0;
@@ -85,6 +89,7 @@ struct CompiledPlan {
     std::vector<Group> fused;                     // the fused list (empty when not realisable)
     bool fused_ok = false;                        // exec = FUSED may run it
     bool auto_fused = false;                      // exec = AUTO runs it
+    bool trees = false;                           // its lists are for the tree kernel (lower_trees)
     bool aliased = false;                         // its outputs are its own leaves' memory (an in-place allreduce)
     std::string fused_why;                        // why fused_ok is false
 };
@@ -114,6 +119,8 @@ struct Lowered {
     std::vector<uint32_t> runs;  // per launch: how many of its items are ITEM_RUN items (they come last)
     uint64_t bytes_read = 0, bytes_written = 0, max_leaves = 0;
     int narrow_threads = 0;  // > 0: every item is ITEM_NARROW, run by the narrow kernel with workgroups of that many lanes
+    // tree_waves > 0: every item is ITEM_TREE, run by the tree kernel with that many waves and a stack that deep
+    int tree_waves = 0, tree_stack = 0;
     bool unaligned_outs = false;  // some vector item writes an output whose offset is not a whole number of vectors
 };
 // tile_elems: elements per work item; vec_elems: elements per 16-byte vector.
@@ -141,6 +148,9 @@ bool narrow_pays(const std::vector<std::vector<Group>>& launches, int vec_elems)
 // The list as ITEM_NARROW items; same groups, same results.  Arguments as for lower_groups.
 void lower_narrow(const std::vector<std::vector<Group>>& launches, int vec_elems, uint32_t bucket, size_t dtsize,
                   Lowered* out, const std::vector<uint32_t>* group_bucket = nullptr);
+// A list of general trees (and copies) as ITEM_TREE items.
+void lower_trees(const std::vector<Group>& groups, int vec_elems, uint32_t bucket, size_t dtsize, Lowered* out,
+                 const std::vector<uint32_t>* group_bucket = nullptr);
 // Whether some launch holds a reduction with several outputs (the lists a two-phase lowering changes).
 bool has_multi_output_reduction(const std::vector<std::vector<Group>>& launches);
 

@@ -244,7 +244,9 @@ int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* sendbuf, voi
  * info->n_launches pairs (first item, item count).  tile_elems: elements per
  * tile, 0 for the general launch shape's; -1: the fused list as a small call
  * uploads it, for the narrow kernel; -t (t > 1): the fused list in tiles of up to
- * t elements whose first and last vectors overlap their neighbours.  in_place: the allreduce
+ * t elements whose first and last vectors overlap their neighbours.  exec: as configured,
+ * or 3 for the list of general trees that AUTO runs where a schedule's trees are
+ * not perfect (AUTO itself dumps the steps there).  in_place: the allreduce
  * schedule for sendbuf == recvbuf (SEND has no extent).  two_phase: 0, or the
  * two-phase mode 1 or 2 of bine_batch_set_tuning, plus 4 for reduction items of
  * two tiles (the flags word shifted right by one).  No HIP call is made. */
