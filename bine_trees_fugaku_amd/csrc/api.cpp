@@ -31,6 +31,8 @@ hipError_t launch_gnarrow(int dtype, const GredItem* items, uint32_t n, const Po
                           const BufTable* tabs, bool batch, int threads, hipStream_t st);
 hipError_t launch_gtree(int dtype, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
                         const BufTable* tabs, bool batch, int waves, int stack, hipStream_t st);
+hipError_t launch_gpack(uint32_t esize, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
+                        const BufTable* tabs, bool batch, hipStream_t st);
 hipError_t launch_reduce_local(int dtype, const void* a, const void* b, void* out, uint64_t n, hipStream_t st);
 size_t scratch_bytes();
 hipError_t scratch_init(int device);
@@ -173,7 +175,7 @@ int upload(const std::vector<std::vector<Group>>& gs, size_t ds, const LaunchSha
         lower_narrow(gs, (int)(16 / ds), 0, ds, &low);
     else
         lower_groups(gs, shallow_tile_elems(sh, ds), (int)(16 / ds), 0, ds, &low, deep_tile_elems(sh, ds),
-                     split_lg(sh), nullptr, sh.two_phase, sh.double_tiles ? 2 : 1, write_heavy(gs) ? Ends::EXACT : ends);
+                     split_lg(sh), nullptr, sh.two_phase, sh.double_tiles ? 2 : 1, write_heavy(gs) ? Ends::EXACT : ends, true);
     return install(std::move(low), max_lg_of(gs), shallow_tile_elems(sh, ds), sh, d, retire);
 }
 
@@ -345,7 +347,7 @@ int get_plan(bine_vcomm_t comm, const CollRequest& req, int dtype, std::shared_p
 uint64_t kernel_launches(const Lowered& low) {
     uint64_t n = 0;
     for (size_t i = 0; i < low.launches.size(); ++i)
-        n += (low.launches[i].second > low.runs[i] ? 1 : 0) + (low.runs[i] ? 1 : 0);
+        n += (low.launches[i].second > low.runs[i] + low.packs[i] ? 1 : 0) + (low.runs[i] ? 1 : 0) + (low.packs[i] ? 1 : 0);
     return n;
 }
 
@@ -473,7 +475,7 @@ int launch_arrays(const DevArrays& d, int dtype, const BufTable& tab, hipStream_
             if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("narrow launch: ") + hipGetErrorString(e));
             continue;
         }
-        const uint32_t nrun = d.low.runs[li], nred = l.second - nrun;
+        const uint32_t nrun = d.low.runs[li], npack = d.low.packs[li], nred = l.second - nrun - npack;
         if (nred) {
             hipError_t e = launch_gred(dtype, d.max_lg, d.items + l.first, nred, d.pool, tab, nullptr, false,
                                        realign, d.shape, st);
@@ -483,6 +485,11 @@ int launch_arrays(const DevArrays& d, int dtype, const BufTable& tab, hipStream_
             hipError_t e = launch_grun((uint32_t)dtsize(dtype), d.items + l.first + nred, nrun, d.pool, tab, nullptr,
                                        false, d.shape, st);
             if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("copy-run launch: ") + hipGetErrorString(e));
+        }
+        if (npack) {
+            hipError_t e = launch_gpack((uint32_t)dtsize(dtype), d.items + l.first + nred + nrun, npack, d.pool, tab,
+                                        nullptr, false, st);
+            if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("copy-grid launch: ") + hipGetErrorString(e));
         }
     }
     return BINE_OK;
@@ -1002,10 +1009,10 @@ extern "C" int bine_plan_dump(const bine_vcomm_config_t* cfg, int32_t coll, int 
     else if (exec == BINE_EXEC_FUSED)
         lower_groups(std::vector<std::vector<Group>>(1, cp.fused), tile_elems, (int)(16 / ds), 0, ds, &low, deep, split_lg(sh),
                      nullptr, two_phase & 3, (two_phase & 4) ? 2 : 1,
-                     !shared_ends ? Ends::EXACT : cp.aliased ? Ends::IN_PLACE : Ends::SHARED);
+                     !shared_ends ? Ends::EXACT : cp.aliased ? Ends::IN_PLACE : Ends::SHARED, shared_ends);
     else
         lower_groups(cp.step_groups, tile_elems, (int)(16 / ds), 0, ds, &low, deep, split_lg(sh), nullptr,
-                     two_phase & 3, (two_phase & 4) ? 2 : 1);
+                     two_phase & 3, (two_phase & 4) ? 2 : 1, Ends::EXACT, shared_ends);
     info->n_items = low.items.size();
     info->n_pool = low.pool.size();
     info->n_launches = low.launches.size();
@@ -1190,7 +1197,7 @@ int lower_list(bine_batch_t b, bine_batch_s::TypeList& l) {
         else
             lower_groups(l.groups, shallow_tile_elems(l.shape, ds), (int)(16 / ds), 0, ds, &all,
                          deep_tile_elems(l.shape, ds), split_lg(l.shape), &l.group_bucket, l.shape.two_phase,
-                         l.shape.double_tiles ? 2 : 1, write_heavy(l.groups) ? Ends::EXACT : l.ends);
+                         l.shape.double_tiles ? 2 : 1, write_heavy(l.groups) ? Ends::EXACT : l.ends, true);
         int max_lg = max_lg_of(l.groups);
         bool tables_off16 = false;
         for (uint32_t gb : l.group_bucket) tables_off16 = tables_off16 || off16(b->tabs[gb]);
@@ -1227,7 +1234,8 @@ int run_list(bine_batch_t b, const bine_batch_s::TypeList& l, hipStream_t st) {
             if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("batch narrow launch: ") + hipGetErrorString(e));
             continue;
         }
-        const uint32_t first = low.launches[li].first, nrun = low.runs[li], nred = low.launches[li].second - nrun;
+        const uint32_t first = low.launches[li].first, nrun = low.runs[li], npack = low.packs[li];
+        const uint32_t nred = low.launches[li].second - nrun - npack;
         if (nred) {
             hipError_t e = launch_gred(l.dtype, l.arr.max_lg, l.arr.items + first, nred, l.arr.pool, BufTable{},
                                        b->d_tabs, true, l.realign, l.shape, st);
@@ -1237,6 +1245,11 @@ int run_list(bine_batch_t b, const bine_batch_s::TypeList& l, hipStream_t st) {
             hipError_t e = launch_grun((uint32_t)dtsize(l.dtype), l.arr.items + first + nred, nrun, l.arr.pool,
                                        BufTable{}, b->d_tabs, true, l.shape, st);
             if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("batch copy-run launch: ") + hipGetErrorString(e));
+        }
+        if (npack) {
+            hipError_t e = launch_gpack((uint32_t)dtsize(l.dtype), l.arr.items + first + nred + nrun, npack, l.arr.pool,
+                                        BufTable{}, b->d_tabs, true, st);
+            if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("batch copy-grid launch: ") + hipGetErrorString(e));
         }
     }
     return BINE_OK;

@@ -18,6 +18,7 @@ enum : uint16_t {
     ITEM_VEC = 1,  // the tile moves as 16-byte vectors, every leaf and output offset dword-aligned
     ITEM_RUN = 2,  // a run of `pad` one-leaf, one-output copies (see GredItem)
     ITEM_TREE = 16,  // a tile of the tree kernel
+    ITEM_PACK = 32,  // a grid of short copies (gpack.hip)
     ITEM_ANY = 8,  // the tile moves as 16-byte vectors, offsets at any byte
     ITEM_NARROW = 4,  // a tile of the narrow kernel (gnarrow.hip): any alignment, any length up to its workgroup's units
 };
@@ -27,6 +28,10 @@ enum : uint16_t {
 // (int64, 4 KiB per rank pair) runs of 2 moved 6.2 TB/s, of 4 5.9, of 8 5.9, of 16 5.6 and of 32 5.3 TB/s:
 // longer runs serialise passes inside one workgroup and leave fewer, longer items; unmerged copies ran 5.75.
 constexpr uint32_t kMaxRun = 2;
+
+// Items of the pack kernel (gpack.hip): a grid of pad % 2^16 by pad / 2^16 copies of n elements.  The pool holds six
+// entries at leaf_off: the first copy's source and destination, then their steps along the first axis, then along the
+// second (ranks and offsets add up, modulo 2^32).
 
 // Items of the tree kernel (gtree.hip): lg is the number of subtrees, at most one per wave.  The pool holds one entry
 // per subtree at leaf_off (rb: its number of leaves; off: the additions that follow when the subtree sums are joined on

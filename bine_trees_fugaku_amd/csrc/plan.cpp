@@ -1755,9 +1755,120 @@ bool compile_program(const Program& prog, bool want_fused, CompiledPlan* out, st
 // Lowering
 // ===========================================================================
 
+namespace {
+
+bool is_copy(const Group& g) { return g.lg == 0 && g.leaves.size() == 1 && g.outs.size() == 1 && g.n > 0; }
+
+// entries as points of (rank and buffer, offset), modulo 2^32
+PoolEntry minus(const PoolEntry& a, const PoolEntry& b) { return PoolEntry{a.rb - b.rb, a.off - b.off}; }
+PoolEntry plus(const PoolEntry& a, const PoolEntry& b, uint32_t k = 1) { return PoolEntry{a.rb + b.rb * k, a.off + b.off * k}; }
+bool same(const PoolEntry& a, const PoolEntry& b) { return a.rb == b.rb && a.off == b.off; }
+
+// A grid of k1 x k2 copies of one length.
+struct CopyGrid {
+    PoolEntry l0, o0, l1{}, o1{}, l2{}, o2{};
+    uint32_t n, bucket, k1 = 1, k2 = 1;
+};
+
+// Runs of copies whose source and destination advance by one step, then equal runs that advance by one step.
+void find_grids(const std::vector<Group>& gs, const std::vector<size_t>& which, const std::vector<uint32_t>* gbk,
+                uint32_t bucket, std::vector<CopyGrid>* out) {
+    std::vector<CopyGrid> rows;
+    for (size_t gi : which) {
+        const Group& g = gs[gi];
+        const uint32_t b = gbk ? (*gbk)[gi] : bucket;
+        const PoolEntry l = g.leaves[0], o = g.outs[0];
+        if (!rows.empty()) {
+            CopyGrid& r = rows.back();
+            if (r.n == (uint32_t)g.n && r.bucket == b && r.k1 < 0xFFFFu) {
+                if (r.k1 == 1) {
+                    r.l1 = minus(l, r.l0);
+                    r.o1 = minus(o, r.o0);
+                    r.k1 = 2;
+                    continue;
+                }
+                if (same(plus(r.l0, r.l1, r.k1), l) && same(plus(r.o0, r.o1, r.k1), o)) {
+                    ++r.k1;
+                    continue;
+                }
+            }
+        }
+        CopyGrid r;
+        r.l0 = l;
+        r.o0 = o;
+        r.n = (uint32_t)g.n;
+        r.bucket = b;
+        rows.push_back(r);
+    }
+    for (const CopyGrid& r : rows) {
+        if (!out->empty()) {
+            CopyGrid& p = out->back();
+            if (p.n == r.n && p.bucket == r.bucket && p.k1 == r.k1 && same(p.l1, r.l1) && same(p.o1, r.o1) && p.k2 < 0xFFFFu) {
+                if (p.k2 == 1) {
+                    p.l2 = minus(r.l0, p.l0);
+                    p.o2 = minus(r.o0, p.o0);
+                    p.k2 = 2;
+                    continue;
+                }
+                if (same(plus(p.l0, p.l2, p.k2), r.l0) && same(plus(p.o0, p.o2, p.k2), r.o0)) {
+                    ++p.k2;
+                    continue;
+                }
+            }
+        }
+        out->push_back(r);
+    }
+}
+
+uint32_t pow2_at_least(uint64_t x) {
+    uint32_t p = 1;
+    while (p < x) p <<= 1;
+    return p;
+}
+
+// Copies that go to the pack kernel: short ones, where the run kernel gives each pair of copies a workgroup, and longer
+// ones that are no whole number of vectors, which leave items of single elements.  GPU time in microseconds, runs /
+// packs, fp32: alltoall on 512 ranks of 16 elements a pair 241 / 7.8, of 25 566 / 11.3, of 256 267 / 108, of 512 302 /
+// 194, of 1024 397 / 389; on 64 ranks of 512 6.6 / 5.1, of 1024 7.4 / 7.7; scatter to 512 ranks of 1000 3.0 / 2.7, of
+// 4099 7.5 / 5.7, but of 16384 13.1 / 15.2 and to 8 ranks of 65537 5.4 / 28: a copy stays within one workgroup.
+bool packs(const Group& g, int vec, size_t dtsize) {
+    const uint64_t bytes = (uint64_t)g.n * dtsize;
+    return is_copy(g) && bytes <= (g.n % vec == 0 ? 2048u : 20480u);
+}
+
+// Cut a grid into items of about `tile` bytes, about as long along either axis where it has two.
+void emit_packs(const CopyGrid& g, size_t dtsize, uint64_t tile, Lowered* out) {
+    const uint64_t bytes = (uint64_t)g.n * dtsize;
+    const uint64_t copies = std::max<uint64_t>(1, tile / bytes);
+    uint32_t t1 = 1, t2 = 1;
+    while ((uint64_t)t1 * t2 * 2 <= copies && (t1 < g.k1 || t2 < g.k2)) {
+        if ((t1 <= t2 || t2 >= g.k2) && t1 < g.k1) t1 *= 2;
+        else t2 *= 2;
+    }
+    for (uint32_t j2 = 0; j2 < g.k2; j2 += t2)
+        for (uint32_t j1 = 0; j1 < g.k1; j1 += t1) {
+            GredItem it{};
+            it.leaf_off = it.out_off = (uint32_t)out->pool.size();
+            out->pool.push_back(plus(plus(g.l0, g.l1, j1), g.l2, j2));
+            out->pool.push_back(plus(plus(g.o0, g.o1, j1), g.o2, j2));
+            for (const PoolEntry& e : {g.l1, g.o1, g.l2, g.o2}) out->pool.push_back(e);
+            it.flags = ITEM_PACK;
+            it.nouts = 1;
+            it.n = g.n;
+            it.bucket = g.bucket;
+            it.pad = std::min(t1, g.k1 - j1) | (std::min(t2, g.k2 - j2) << 16);
+            out->items.push_back(it);
+        }
+    out->bytes_read += bytes * g.k1 * g.k2;
+    out->bytes_written += bytes * g.k1 * g.k2;
+    out->max_leaves = std::max<uint64_t>(out->max_leaves, 1);
+}
+
+}  // namespace
+
 void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shallow_tile, int vec, uint32_t bucket,
                   size_t dtsize, Lowered* out, int64_t deep_tile_elems, int deep_lg,
-                  const std::vector<uint32_t>* group_bucket, int two_phase, int reduction_tiles, Ends ends) {
+                  const std::vector<uint32_t>* group_bucket, int two_phase, int reduction_tiles, Ends ends, bool pack) {
     int widest_lg = 0;
     for (const auto& gs : launches)
         for (const Group& g : gs) widest_lg = std::max<int>(widest_lg, g.lg);
@@ -1786,10 +1897,15 @@ void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shall
         auto advance = [](const PoolEntry& a, const PoolEntry& st, uint32_t k) {
             return PoolEntry{a.rb + st.rb * k, a.off + st.off * k};
         };
+        std::vector<size_t> packed;
         for (size_t gi = 0; gi < gs.size(); ++gi) {
             const Group& g = gs[gi];
             const uint32_t gb = gbk ? (*gbk)[gi] : bucket;
             if (g.n <= 0) continue;
+            if (pack && packs(g, vec, dtsize)) {
+                packed.push_back(gi);
+                continue;
+            }
             if (single_copy(g) && run_item >= 0 && run_len < kMaxRun && out->items[run_item].n == (uint32_t)g.n &&
                 out->items[run_item].bucket == gb) {
                 bool ok;
@@ -1960,8 +2076,18 @@ void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shall
                     out->unaligned_outs |= ((int64_t)out->pool[it.out_off + o].off + it.delta) % vec != 0;
             }
         }
-        out->launches.push_back({first, (uint32_t)cnt});
+        if (!packed.empty()) {
+            std::vector<CopyGrid> grids;
+            find_grids(gs, packed, gbk, bucket, &grids);
+            uint64_t moved = 0;
+            for (const CopyGrid& g : grids) moved += (uint64_t)g.n * dtsize * g.k1 * g.k2;
+            // 16 KiB a workgroup (four 16-byte units per lane), less where that would give fewer than 2048 of them
+            const uint64_t tile = std::min<uint64_t>(16384, std::max<uint64_t>(1024, moved / 2048));
+            for (const CopyGrid& g : grids) emit_packs(g, dtsize, tile, out);
+        }
+        out->launches.push_back({first, (uint32_t)(out->items.size() - first)});
         out->runs.push_back(nrun);
+        out->packs.push_back((uint32_t)(out->items.size() - first - cnt));
     };
     for (size_t li = 0; li < launches.size(); ++li) {
         const std::vector<Group>& gs = launches[li];
@@ -2004,12 +2130,6 @@ namespace {
 
 // 16-byte units of a group's block: whole vectors plus one that ends at the block's end, or single elements.
 int64_t narrow_units(const Group& g, int vec) { return g.n >= vec ? (g.n + vec - 1) / vec : g.n; }
-
-uint32_t pow2_at_least(uint64_t x) {
-    uint32_t p = 1;
-    while (p < x) p <<= 1;
-    return p;
-}
 
 // Lanes that leave each one about eight leaves to load and eight outputs to store.
 uint64_t narrow_segments(const Group& g) {
@@ -2105,6 +2225,7 @@ void lower_narrow(const std::vector<std::vector<Group>>& launches, int vec, uint
     }
     out->launches.push_back({0, (uint32_t)out->items.size()});
     out->runs.push_back(0);
+    out->packs.push_back(0);
 }
 
 namespace {
@@ -2232,6 +2353,7 @@ void lower_trees(const std::vector<Group>& gs, int vec, uint32_t bucket, size_t 
     }
     out->launches.push_back({0, (uint32_t)out->items.size()});
     out->runs.push_back(0);
+    out->packs.push_back(0);
 }
 
 bool has_multi_output_reduction(const std::vector<std::vector<Group>>& launches) {

@@ -116,7 +116,8 @@ struct Lowered {
     std::vector<GredItem> items;
     std::vector<PoolEntry> pool;
     std::vector<std::pair<uint32_t, uint32_t>> launches;  // (first item, item count)
-    std::vector<uint32_t> runs;  // per launch: how many of its items are ITEM_RUN items (they come last)
+    std::vector<uint32_t> runs;   // per launch: how many of its items are ITEM_RUN items (after the others)
+    std::vector<uint32_t> packs;  // per launch: how many of its items are ITEM_PACK items (after the runs)
     uint64_t bytes_read = 0, bytes_written = 0, max_leaves = 0;
     int narrow_threads = 0;  // > 0: every item is ITEM_NARROW, run by the narrow kernel with workgroups of that many lanes
     // tree_waves > 0: every item is ITEM_TREE, run by the tree kernel with that many waves and a stack that deep
@@ -139,10 +140,11 @@ enum class Ends {
                // in them are computed and stored twice.  Only for lists whose outputs share no memory with their leaves.
     IN_PLACE,  // SHARED where the outputs are the item's own leaves and the tile allows it, else EXACT
 };
+// pack: short single copies become ITEM_PACK items.
 void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t tile_elems, int vec_elems,
                   uint32_t bucket, size_t dtsize, Lowered* out, int64_t deep_tile_elems = 0, int deep_lg = 99,
                   const std::vector<uint32_t>* group_bucket = nullptr, int two_phase = 0, int reduction_tiles = 1,
-                  Ends ends = Ends::EXACT);
+                  Ends ends = Ends::EXACT, bool pack = false);
 // Whether a list (one launch, at the general launch shape) is better run by the narrow kernel (gnarrow.hip).
 bool narrow_pays(const std::vector<std::vector<Group>>& launches, int vec_elems);
 // The list as ITEM_NARROW items; same groups, same results.  Arguments as for lower_groups.
