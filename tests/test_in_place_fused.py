@@ -11,6 +11,7 @@ from bine_trees_fugaku_amd.collectives import plan_dump
 from oracle import oracle as O
 from tests import emulator as E
 from tests.test_narrow import NP, data
+from tests.test_packs import expand
 
 VECTOR = 1 | 8
 
@@ -29,7 +30,9 @@ def test_in_place_lists(dims, algo, tile, two_phase):
             assert len(launches) == (1 if two_phase == 0 or tile == -1 else 2)
         for reverse in (False, True):
             bufs = E.alloc_buffers(meta, np.float32, recv=x)
-            E.run(meta, items, pool, launches, bufs, reverse=reverse)
+            for first, n in launches:  # per-step lists (algorithm L) may hold grids of copies
+                its, pl = expand(items[first:first + n], pool)
+                E.run(meta, its, pl, [(0, len(its))], bufs, reverse=reverse)
             want = O.allreduce(x, dims, algo=algo)
             assert bufs[E.BUF_RECV].tobytes() == want.tobytes(), (count, reverse)
 
