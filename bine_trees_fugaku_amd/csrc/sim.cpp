@@ -11,12 +11,9 @@
 
 #include "bine_hip.h"
 #include "sim_dest.hpp"
+#include "sim_launch.hpp"
 
 namespace bine {
-
-hipError_t launch_sim(const void* cases, const void* classes, uint32_t ncls, const void* count_blocks,
-                      uint32_t n_count_blocks, const void* scan_blocks, uint32_t n_scan_blocks, uint32_t* mult,
-                      uint64_t mult_len, uint32_t* max_hops, uint32_t* max_mult, uint64_t* sum_mult, hipStream_t st);
 
 static simd::TorusD dev_torus(const Torus& t) {
     simd::TorusD d;
@@ -127,7 +124,8 @@ struct bine_sim_s {
     uint32_t* d_mult = nullptr;
     uint32_t* d_count_blocks = nullptr;  // per workgroup of the count kernel: (class, first rank)
     uint32_t* d_scan_blocks = nullptr;   // per workgroup of the ring scan: (class, first ring-direction)
-    uint32_t n_count_blocks = 0, n_scan_blocks = 0;
+    uint32_t* d_slices = nullptr;        // per workgroup of the LDS kernel: (class, dimensions)
+    SimLaunch launch{};
     uint32_t* d_hops = nullptr;
     uint32_t* d_max = nullptr;
     uint64_t* d_sum = nullptr;
@@ -136,7 +134,7 @@ struct bine_sim_s {
     hipStream_t last = nullptr;  // stream of the last run; queries wait for it
     ~bine_sim_s() {
         for (void* p : {(void*)d_cases, (void*)d_classes, (void*)d_mult, (void*)d_hops, (void*)d_max, (void*)d_sum,
-                        (void*)d_count_blocks, (void*)d_scan_blocks})
+                        (void*)d_count_blocks, (void*)d_scan_blocks, (void*)d_slices})
             if (p) (void)hipFree(p);
     }
 };
@@ -185,6 +183,20 @@ extern "C" int bine_sim_create(const bine_sim_case_t* cases, int n, int device, 
     std::vector<SimCaseRec> crec;
     std::vector<SimClassRec> krec;
     std::vector<uint32_t> cblk, sblk;  // (class, first index) pairs
+    // (class, dimensions) pairs by LDS need: small tori run many workgroups per compute unit, the largest one
+    static const uint32_t kBinLds[3] = {16384, 65536, 0xFFFFFFFFu}, kBinThreads[3] = {256, 1024, 1024};
+    std::vector<uint32_t> slices[3];
+    uint32_t lds_limit = 0, bin_lds[3] = {0, 0, 0};
+    bool sliced = false;
+    SHIP(hipSetDevice(device));
+    SHIP(sim_lds_limit(device, &lds_limit));
+    auto slice = [&](uint32_t cls, uint32_t d0, uint32_t d1, uint32_t bytes) {
+        int b = 0;
+        while (bytes > kBinLds[b]) ++b;
+        slices[b].push_back(cls);
+        slices[b].push_back(d0 | (d1 << 8));
+        bin_lds[b] = std::max(bin_lds[b], bytes);
+    };
     uint64_t off = 0;
     for (int i = 0; i < n; ++i) {
         Torus t;
@@ -203,6 +215,15 @@ extern "C" int bine_sim_create(const bine_sim_case_t* cases, int n, int device, 
             krec.push_back(SimClassRec{c.kind, c.d, c.k, (uint32_t)i, off});
             s->mult_off.push_back(off);
             off += nl;
+            if ((uint64_t)nl * 4 <= lds_limit) {
+                slice(cls, 0, t.nd, nl * 4);
+                continue;
+            }
+            sliced = true;
+            if ((uint64_t)t.size * 8 <= lds_limit) {
+                for (uint32_t d = 0; d < t.nd; ++d) slice(cls, d, d + 1, t.size * 8);
+                continue;
+            }
             for (uint32_t r = 0; r < t.size; r += 256) {
                 cblk.push_back(cls);
                 cblk.push_back(r);
@@ -216,21 +237,43 @@ extern "C" int bine_sim_create(const bine_sim_case_t* cases, int n, int device, 
     }
     s->ncls = (uint32_t)krec.size();
     s->mult_len = off;
-    SHIP(hipSetDevice(device));
     SHIP(hipMalloc(&s->d_cases, sizeof(SimCaseRec) * crec.size()));
     SHIP(hipMemcpy(s->d_cases, crec.data(), sizeof(SimCaseRec) * crec.size(), hipMemcpyHostToDevice));
     SHIP(hipMalloc(&s->d_classes, sizeof(SimClassRec) * krec.size()));
     SHIP(hipMemcpy(s->d_classes, krec.data(), sizeof(SimClassRec) * krec.size(), hipMemcpyHostToDevice));
     SHIP(hipMalloc(&s->d_mult, sizeof(uint32_t) * off));
-    s->n_count_blocks = (uint32_t)(cblk.size() / 2);
-    s->n_scan_blocks = (uint32_t)(sblk.size() / 2);
-    SHIP(hipMalloc(&s->d_count_blocks, sizeof(uint32_t) * cblk.size()));
-    SHIP(hipMemcpy(s->d_count_blocks, cblk.data(), sizeof(uint32_t) * cblk.size(), hipMemcpyHostToDevice));
-    SHIP(hipMalloc(&s->d_scan_blocks, sizeof(uint32_t) * sblk.size()));
-    SHIP(hipMemcpy(s->d_scan_blocks, sblk.data(), sizeof(uint32_t) * sblk.size(), hipMemcpyHostToDevice));
+    auto put = [&](const std::vector<uint32_t>& v, uint32_t** p) {
+        if (v.empty()) return hipSuccess;
+        const hipError_t e = hipMalloc(p, sizeof(uint32_t) * v.size());
+        return e != hipSuccess ? e : hipMemcpy(*p, v.data(), sizeof(uint32_t) * v.size(), hipMemcpyHostToDevice);
+    };
+    SHIP(put(cblk, &s->d_count_blocks));
+    SHIP(put(sblk, &s->d_scan_blocks));
+    std::vector<uint32_t> all;
+    SimLaunch& L = s->launch;
+    for (int b = 2; b >= 0; --b) {  // the longest workgroups first
+        if (slices[b].empty()) continue;
+        L.bins[L.n_bins++] = SimBin{(uint32_t)(all.size() / 2), (uint32_t)(slices[b].size() / 2), kBinThreads[b], bin_lds[b]};
+        all.insert(all.end(), slices[b].begin(), slices[b].end());
+    }
+    SHIP(put(all, &s->d_slices));
     SHIP(hipMalloc(&s->d_hops, sizeof(uint32_t) * s->ncls));
     SHIP(hipMalloc(&s->d_max, sizeof(uint32_t) * s->ncls));
     SHIP(hipMalloc(&s->d_sum, sizeof(uint64_t) * s->ncls));
+    L.cases = s->d_cases;
+    L.classes = s->d_classes;
+    L.slices = s->d_slices;
+    L.count_blocks = s->d_count_blocks;
+    L.scan_blocks = s->d_scan_blocks;
+    L.n_count_blocks = (uint32_t)(cblk.size() / 2);
+    L.n_scan_blocks = (uint32_t)(sblk.size() / 2);
+    L.zero = sliced;
+    L.mult = s->d_mult;
+    L.mult_len = off;
+    L.ncls = s->ncls;
+    L.max_hops = s->d_hops;
+    L.max_mult = s->d_max;
+    L.sum_mult = s->d_sum;
     *out = s.release();
     return BINE_OK;
 }
@@ -238,8 +281,7 @@ extern "C" int bine_sim_create(const bine_sim_case_t* cases, int n, int device, 
 extern "C" int bine_sim_run(bine_sim_t s, void* stream) {
     if (!s) return sfail(BINE_ERR_ARG, "NULL simulation");
     SHIP(hipSetDevice(s->device));
-    SHIP(launch_sim(s->d_cases, s->d_classes, s->ncls, s->d_count_blocks, s->n_count_blocks, s->d_scan_blocks,
-                    s->n_scan_blocks, s->d_mult, s->mult_len, s->d_hops, s->d_max, s->d_sum, (hipStream_t)stream));
+    SHIP(launch_sim(s->launch, (hipStream_t)stream));
     s->last = (hipStream_t)stream;
     return BINE_OK;
 }
