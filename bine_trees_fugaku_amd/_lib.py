@@ -129,7 +129,7 @@ def _sig(L):
     L.bine_sim_create.argtypes = [psc, i32, i32, ctypes.POINTER(vp)]
     L.bine_sim_run.argtypes = [vp, vp]
     L.bine_sim_case_info.argtypes = [vp, i32, pu32, pu32]
-    L.bine_sim_class_stats.argtypes = [vp, i32, pu32, pu32, pu32, pu32, pu64, pu32]
+    L.bine_sim_class_stats.argtypes = [vp, i32, vp, vp, vp, vp, vp, vp]  # arrays by address
     L.bine_sim_link_counts.argtypes = [vp, i32, u32, pu32]
     L.bine_sim_destroy.argtypes = [vp]
     pf = ctypes.POINTER(ctypes.c_float)

@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -126,14 +127,20 @@ struct bine_sim_s {
     uint32_t* d_scan_blocks = nullptr;   // per workgroup of the ring scan: (class, first ring-direction)
     uint32_t* d_slices = nullptr;        // per workgroup of the LDS kernel: (class, dimensions)
     SimLaunch launch{};
-    uint32_t* d_hops = nullptr;
-    uint32_t* d_max = nullptr;
-    uint64_t* d_sum = nullptr;
+    // every class's statistics, one array: sums of link crossings (64 bits), then most loaded links, then longest routes
+    uint64_t* d_stats = nullptr;
+    std::vector<uint64_t> h_stats;
+    std::mutex mu;          // of h_stats
+    bool fetched = false;   // h_stats holds the last run's
+    bool captured = false;  // the last run was recorded into a graph: its results may change with every replay
+    uint32_t* d_max() const { return reinterpret_cast<uint32_t*>(d_stats + ncls); }
+    uint32_t* d_hops() const { return d_max() + ncls; }
+    size_t stats_words() const { return (size_t)ncls * 2; }
     uint64_t mult_len = 0;
     uint32_t ncls = 0;
     hipStream_t last = nullptr;  // stream of the last run; queries wait for it
     ~bine_sim_s() {
-        for (void* p : {(void*)d_cases, (void*)d_classes, (void*)d_mult, (void*)d_hops, (void*)d_max, (void*)d_sum,
+        for (void* p : {(void*)d_cases, (void*)d_classes, (void*)d_mult, (void*)d_stats,
                         (void*)d_count_blocks, (void*)d_scan_blocks, (void*)d_slices})
             if (p) (void)hipFree(p);
     }
@@ -257,9 +264,8 @@ extern "C" int bine_sim_create(const bine_sim_case_t* cases, int n, int device, 
         all.insert(all.end(), slices[b].begin(), slices[b].end());
     }
     SHIP(put(all, &s->d_slices));
-    SHIP(hipMalloc(&s->d_hops, sizeof(uint32_t) * s->ncls));
-    SHIP(hipMalloc(&s->d_max, sizeof(uint32_t) * s->ncls));
-    SHIP(hipMalloc(&s->d_sum, sizeof(uint64_t) * s->ncls));
+    s->h_stats.resize(s->stats_words());
+    SHIP(hipMalloc(&s->d_stats, sizeof(uint64_t) * s->stats_words()));
     L.cases = s->d_cases;
     L.classes = s->d_classes;
     L.slices = s->d_slices;
@@ -271,9 +277,9 @@ extern "C" int bine_sim_create(const bine_sim_case_t* cases, int n, int device, 
     L.mult = s->d_mult;
     L.mult_len = off;
     L.ncls = s->ncls;
-    L.max_hops = s->d_hops;
-    L.max_mult = s->d_max;
-    L.sum_mult = s->d_sum;
+    L.max_hops = s->d_hops();
+    L.max_mult = s->d_max();
+    L.sum_mult = s->d_stats;
     *out = s.release();
     return BINE_OK;
 }
@@ -281,8 +287,13 @@ extern "C" int bine_sim_create(const bine_sim_case_t* cases, int n, int device, 
 extern "C" int bine_sim_run(bine_sim_t s, void* stream) {
     if (!s) return sfail(BINE_ERR_ARG, "NULL simulation");
     SHIP(hipSetDevice(s->device));
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)stream, &cs) != hipSuccess) (void)hipGetLastError();
+    std::lock_guard<std::mutex> lock(s->mu);
     SHIP(launch_sim(s->launch, (hipStream_t)stream));
     s->last = (hipStream_t)stream;
+    s->fetched = false;
+    s->captured = cs != hipStreamCaptureStatusNone;
     return BINE_OK;
 }
 
@@ -296,8 +307,6 @@ extern "C" int bine_sim_case_info(bine_sim_t s, int i, uint32_t* nclasses, uint3
 extern "C" int bine_sim_class_stats(bine_sim_t s, int i, uint32_t* num, uint32_t* den, uint32_t* rep,
                                     uint32_t* max_mult, uint64_t* sum_mult, uint32_t* max_hops) {
     if (!s || i < 0 || i >= (int)s->cases.size()) return sfail(BINE_ERR_ARG, "bad case index");
-    SHIP(hipSetDevice(s->device));
-    SHIP(hipStreamSynchronize(s->last));
     const uint32_t first = s->class_first[i];
     const size_t nc = s->cases[i].classes.size();
     for (size_t c = 0; c < nc; ++c) {
@@ -306,9 +315,19 @@ extern "C" int bine_sim_class_stats(bine_sim_t s, int i, uint32_t* num, uint32_t
         if (den) den[c] = k.den;
         if (rep) rep[c] = k.rep;
     }
-    if (max_mult) SHIP(hipMemcpy(max_mult, s->d_max + first, nc * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    if (sum_mult) SHIP(hipMemcpy(sum_mult, s->d_sum + first, nc * sizeof(uint64_t), hipMemcpyDeviceToHost));
-    if (max_hops) SHIP(hipMemcpy(max_hops, s->d_hops + first, nc * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    // one wait and one copy per run for all cases: three copies a case took 50 us each time
+    std::lock_guard<std::mutex> lock(s->mu);
+    if (!s->fetched) {
+        SHIP(hipSetDevice(s->device));
+        SHIP(hipStreamSynchronize(s->last));
+        SHIP(hipMemcpy(s->h_stats.data(), s->d_stats, sizeof(uint64_t) * s->stats_words(), hipMemcpyDeviceToHost));
+        s->fetched = !s->captured;
+    }
+    const uint64_t* sums = s->h_stats.data();
+    const uint32_t* most = reinterpret_cast<const uint32_t*>(sums + s->ncls);
+    if (max_mult) std::copy_n(most + first, nc, max_mult);
+    if (sum_mult) std::copy_n(sums + first, nc, sum_mult);
+    if (max_hops) std::copy_n(most + s->ncls + first, nc, max_hops);
     return BINE_OK;
 }
 

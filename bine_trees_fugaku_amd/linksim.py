@@ -103,6 +103,7 @@ class LinkSim:
         h = ctypes.c_void_p()
         _lib.check(L.bine_sim_create(arr, len(self.cases), int(device), ctypes.byref(h)), "bine_sim_create")
         self._h = h
+        self._sizes = {}  # classes per case, as asked for
 
     def run(self, stream=None) -> None:
         s = None if stream is None else ctypes.c_void_p(getattr(stream, "cuda_stream", stream))
@@ -114,13 +115,14 @@ class LinkSim:
         return nc.value, nl.value
 
     def stats(self, i: int) -> ClassStats:
-        nc, _ = self.info(i)
-        a = {k: np.zeros(nc, np.uint32) for k in ("num", "den", "rep", "max_mult", "max_hops")}
-        sm = np.zeros(nc, np.uint64)
-        _lib.check(_lib.load().bine_sim_class_stats(
-            self._h, i, _u32p(a["num"]), _u32p(a["den"]), _u32p(a["rep"]), _u32p(a["max_mult"]),
-            sm.ctypes.data_as(ctypes.POINTER(ctypes.c_uint64)), _u32p(a["max_hops"])), "bine_sim_class_stats")
-        return ClassStats(a["num"], a["den"], a["rep"], a["max_mult"], sm, a["max_hops"])
+        if i not in self._sizes:
+            self._sizes[i] = self.info(i)[0]
+        nc = self._sizes[i]
+        a, sm = np.empty((5, nc), np.uint32), np.empty(nc, np.uint64)
+        p = a.ctypes.data
+        _lib.check(_lib.load().bine_sim_class_stats(self._h, i, p, p + 4 * nc, p + 8 * nc, p + 12 * nc, sm.ctypes.data,
+                                                    p + 16 * nc), "bine_sim_class_stats")
+        return ClassStats(a[0], a[1], a[2], a[3], sm, a[4])
 
     def link_counts(self, i: int, cls: int) -> np.ndarray:
         _, nl = self.info(i)
