@@ -28,7 +28,7 @@ hipError_t launch_gred(int dtype, int max_lg, const GredItem* items, uint32_t n,
 hipError_t launch_grun(uint32_t esize, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
                        const BufTable* tabs, bool batch, const LaunchShape& sh, hipStream_t st);
 hipError_t launch_gnarrow(int dtype, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
-                          const BufTable* tabs, bool batch, int threads, hipStream_t st);
+                          const BufTable* tabs, bool batch, int threads, bool stream, hipStream_t st);
 hipError_t launch_gtree(int dtype, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
                         const BufTable* tabs, bool batch, int waves, int stack, hipStream_t st);
 hipError_t launch_gpack(uint32_t esize, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
@@ -226,29 +226,84 @@ struct PlanKeyHash {
 LaunchShape default_shape() { return LaunchShape{1, 256, 0, 0}; }
 int64_t default_tile_elems(size_t ds) { return shallow_tile_elems(default_shape(), ds); }
 
-// The shape a fused work list starts with before any tuning.  Four vectors per thread, one-wave workgroups and
-// streaming loads and stores (the one-launch shape the autotuner keeps on long blocks) when the reductions of 64
-// leaves or more hold at least 90 % of the list's bytes in blocks of two whole tiles or more at that shape, and
-// those blocks give at least 1024 tiles, so every CU gets several.  Untuned, that shape moved the 512-rank fp64
-// allreduce of 4 MiB per rank at 6.1 TB/s against 4.5 with the general shape; on shorter blocks or fewer tiles
-// (the same torus at 256 KiB per rank, or 64 ranks of 2 MiB) it ran 10-67 % slower than the general shape, which
-// every other list starts at.
-LaunchShape initial_shape(const std::vector<std::vector<Group>>& gs, size_t ds) {
-    const LaunchShape wide{4, 64, 0, 1};
-    const int64_t tile = deep_tile_elems(wide, ds);
-    uint64_t bytes = 0, long_bytes = 0, tiles = 0;
+// The shape a fused work list starts with before any tuning.
+//
+// Below 64 MB the general shape and its narrow kernel are the fastest.  From there on loads and stores stream, since a
+// caller's next buffers are rarely in the memory-side cache (256 MB): the figures below rotate over buffers of 1.2 GB in
+// all.  The rest follows the kind of list (by bytes), its fan (leaves or outputs of the widest group), the blocks'
+// length in 16-byte units, and how many tiles a shape would give.  GPU time in microseconds, fp32, general / chosen:
+//   reductions with several outputs, fan >= 64, by T, the tiles of four vectors per lane of one wave:
+//     T >= 1024 (512 beyond 300 MB): that shape, and for a single collective with aligned outputs two phases, in group
+//       order below 4096 tiles, tile by tile with two-tile reductions from there on: 512 ranks of 524288 (T = 512) 571 /
+//       395, of 1048576 967 / 678 (one phase 705); 64 ranks of 1048576 115 / 89 (94), of 4194304 (T = 4096) 433 / 364
+//       (386; group order 402);
+//     blocks below a tile beyond 300 MB: two waves of four vectors: 512 ranks of 262144 257 / 198, 256 of 262144 178 / 106;
+//     at least 512 tiles of two vectors and two waves: that: 64 ranks of 262144 27.2 / 24.5, of 524288 57.5 / 47.4;
+//     at least 512 tiles of the general shape: it, streaming: 64 ranks of 131072 20.3 / 13.7, 128 of 131072 41.9 / 30.1;
+//     fan >= 256, blocks of 48 to 119 units, from 190 MB on: the same: 512 ranks of 98304 107 / 87, of 131072 142 / 98;
+//   fan below 64: two vectors, two waves: 8 ranks of 1048576 19.7 / 13.6, 16 of 524288 16.4 / 12.7, 32 of 262144 15.3 /
+//     13.8; with fan 32 from 200 MB on four vectors, one wave: of 1048576 57 / 48;
+//   reductions with one output: T >= 1024 and fan >= 64 four vectors, one wave: reduce_scatter on 512 ranks of 2048 370 /
+//     311, on 128 of 8192 158 / 86; at least 512 tiles of two waves and four vectors (or two): 64 ranks of 8192 27.4 / 23.3,
+//     256 of 1024 72 / 57, 16 of 262144 54.4 / 46.9; else the general shape, streaming: 64 ranks of 4096 15.2 / 14.5;
+//   copies to many outputs, aligned, 512 tiles of at least 96 units, or 256 full ones from 400 MB on: four vectors, one
+//     wave: allgather on 512 ranks of 512 138 / 92, on 16 of 65536 16.2 / 13.1, bcast to 512 of 262144 119 / 102; but
+//     allgather on 256 of 1024 (269 MB) 50.1 / 53.6, bcast to 64 of 262144 (67 MB) 15.4 / 16.8, to 16 of 8388608 101 / 109;
+//   single copies: the general shape, streaming: alltoall on 64 ranks of 4096 a pair 28.7 / 24.7; beyond 300 MB two
+//     vectors, two waves: on 512 ranks of 1024 410 / 338 (352).
+// aligned: every output starts on a 16-byte boundary; single: the list is one collective call's own.
+LaunchShape initial_shape(const std::vector<std::vector<Group>>& gs, size_t ds, bool aligned, bool single) {
+    constexpr uint64_t MB = 1u << 20;
+    const LaunchShape wide{4, 64, 0, 1}, pair{2, 128, 0, 1}, quad{4, 128, 0, 1}, general{1, 256, 0, 1};
+    const int64_t vec = (int64_t)(16 / ds), tile = deep_tile_elems(wide, ds);
+    enum Kind { SPREAD, REDUCE, COPY_MANY, COPY, KINDS };
+    uint64_t bytes[KINDS] = {}, all = 0, tiles = 0, pieces = 0, units = 0, blocks = 0, long_bytes = 0;
+    int64_t longest = 0, shortest = INT64_MAX;
+    size_t fan = 0;
     for (const auto& v : gs)
         for (const Group& g : v) {
-            if (g.lg == 0) continue;
+            if (g.n <= 0) continue;
             const uint64_t b = (uint64_t)g.n * (g.leaves.size() + g.outs.size()) * ds;
-            bytes += b;
-            if (g.lg >= 6 && g.n >= 2 * tile) {
-                long_bytes += b;
-                tiles += (uint64_t)(g.n / tile);
-            }
+            all += b;
+            bytes[g.lg > 0 ? (g.outs.size() > 1 ? SPREAD : REDUCE) : (g.outs.size() > 1 ? COPY_MANY : COPY)] += b;
+            fan = std::max({fan, g.leaves.size(), g.outs.size()});
+            tiles += (uint64_t)((g.n + tile / 4) / tile);  // a tile three quarters full counts
+            pieces += (uint64_t)((g.n + tile - 1) / tile);
+            units += (uint64_t)((g.n + vec - 1) / vec);
+            ++blocks;
+            longest = std::max(longest, g.n);
+            shortest = std::min(shortest, g.n);
+            if (g.n >= 2 * tile) long_bytes += b;
+            for (const PoolEntry& o : g.outs) aligned = aligned && o.off % vec == 0;
         }
-    if (tiles >= 1024 && long_bytes * 10 >= bytes * 9) return wide;
-    return default_shape();
+    int kind = 0;
+    while (kind < KINDS && bytes[kind] * 10 < all * 9) ++kind;
+    // blocks of unlike lengths (a batch): the one-wave shape where the long ones hold nearly all of it
+    if (longest > shortest + 1 && kind <= REDUCE) return tiles >= 1024 && fan >= 64 && long_bytes * 10 >= all * 9 ? wide : default_shape();
+    if (all < 64 * MB || kind == KINDS || (kind != COPY && fan < 8)) return default_shape();
+    const uint64_t length = units / blocks;  // a block's units
+    const bool large = all > 300 * MB;
+    const LaunchShape rest = length >= 64 && units >= 512 * 64 && !narrow_pays(gs, (int)vec) ? general : default_shape();
+    switch (kind) {
+    case SPREAD:
+        if (fan < 64) return fan == 32 && all >= 200 * MB ? wide : pair;
+        if (fan >= 256 && all >= 190 * MB && length >= 48 && length < 120) return general;
+        if (tiles >= (large ? 512u : 1024u)) {
+            if (!aligned || !single) return wide;  // a batch keeps one launch per list until it is tuned
+            return tiles < 4096 ? LaunchShape{4, 64, 0, 1, 1, 0} : LaunchShape{4, 64, 0, 1, 2, 1};
+        }
+        if (large) return quad;
+        return length >= 128 && units >= 512 * 128 ? pair : rest;
+    case REDUCE:
+        if (fan >= 64 && tiles >= 1024) return wide;
+        if (length >= 128 && units >= 512 * 256) return quad;
+        return length >= 128 && units >= 512 * 128 ? pair : rest;
+    case COPY_MANY:
+        if (!aligned || (fan < 32 && all > 400 * MB)) return default_shape();
+        return (length >= 256 && pieces >= 256 && all >= 400 * MB) || (length >= 96 && pieces >= 512) ? wide
+                                                                                              : default_shape();
+    default: return large ? pair : general;
+    }
 }
 
 }  // namespace
@@ -323,7 +378,7 @@ int get_plan(bine_vcomm_t comm, const CollRequest& req, int dtype, std::shared_p
     }
     if (dp->cp.auto_fused) {
         std::vector<std::vector<Group>> one(1, dp->cp.fused);
-        rc = upload(one, ds, initial_shape(one, ds), dp->fused_ends(), dp->cp.trees, &dp->fused);
+        rc = upload(one, ds, initial_shape(one, ds, (uint64_t)prog.extent[BUF_RECV] * ds % 16 == 0, true), dp->fused_ends(), dp->cp.trees, &dp->fused);
         if (rc) return rc;
     }
     // temporaries are allocated only when some step touches them
@@ -471,7 +526,7 @@ int launch_arrays(const DevArrays& d, int dtype, const BufTable& tab, hipStream_
         }
         if (d.low.narrow_threads) {
             hipError_t e = launch_gnarrow(dtype, d.items + l.first, l.second, d.pool, tab, nullptr, false,
-                                          d.low.narrow_threads, st);
+                                          d.low.narrow_threads, d.low.narrow_stream, st);
             if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("narrow launch: ") + hipGetErrorString(e));
             continue;
         }
@@ -1230,7 +1285,8 @@ int run_list(bine_batch_t b, const bine_batch_s::TypeList& l, hipStream_t st) {
         }
         if (low.narrow_threads) {
             hipError_t e = launch_gnarrow(l.dtype, l.arr.items + low.launches[li].first, low.launches[li].second,
-                                          l.arr.pool, BufTable{}, b->d_tabs, true, low.narrow_threads, st);
+                                          l.arr.pool, BufTable{}, b->d_tabs, true, low.narrow_threads,
+                                          low.narrow_stream, st);
             if (e != hipSuccess) return fail(BINE_ERR_HIP, std::string("batch narrow launch: ") + hipGetErrorString(e));
             continue;
         }
@@ -1327,7 +1383,11 @@ extern "C" int bine_batch_create(bine_vcomm_t comm, const bine_batch_item_t* ite
     HIPCHK(hipSetDevice(comm->cfg.device));
     HIPCHK(hipMalloc(&b->d_tabs, sizeof(BufTable) * b->tabs.size()));
     HIPCHK(hipMemcpy(b->d_tabs, b->tabs.data(), sizeof(BufTable) * b->tabs.size(), hipMemcpyHostToDevice));
-    for (auto& l : b->lists) l.shape = initial_shape(l.groups, dtsize(l.dtype));
+    for (auto& l : b->lists) {
+        bool aligned = true;
+        for (uint32_t gb : l.group_bucket) aligned = aligned && !off16(b->tabs[gb]);
+        l.shape = initial_shape(l.groups, dtsize(l.dtype), aligned, false);
+    }
     if (!b->lists.empty()) b->shape = b->lists[0].shape;
     int rc = batch_lower(b.get());
     if (rc) return rc;

@@ -47,7 +47,7 @@ __device__ __forceinline__ T lane_xor(T v, int mask) {
 }
 
 // One item, U = Vec<T> or T; `units` <= blockDim.x, `step` elements per unit.
-template <typename T, typename U>
+template <typename T, typename U, bool NT>
 __device__ __forceinline__ void narrow_item(const GredItem& it, const Table& t, const PoolEntry* pool, uint32_t units,
                                             uint32_t step, U* lds) {
     const uint32_t lgT = 31u - (uint32_t)__builtin_clz(blockDim.x);
@@ -70,7 +70,7 @@ __device__ __forceinline__ void narrow_item(const GredItem& it, const Table& t, 
     }
     auto load = [&](uint32_t k) __attribute__((always_inline)) {
         const PoolEntry e = cload(leaves + k);
-        return load_unit(t.at(e.rb, (uint64_t)e.off + at, sizeof(T)), (U*)nullptr);
+        return load_unit<NT>(t.at(e.rb, (uint64_t)e.off + at, sizeof(T)), (U*)nullptr);
     };
     auto add = [](const U& a, const U& b) __attribute__((always_inline)) { return add_unit(a, b); };
     U v{};
@@ -90,7 +90,7 @@ __device__ __forceinline__ void narrow_item(const GredItem& it, const Table& t, 
     for (uint32_t o = seg; o < nouts;) {
 #pragma unroll
         for (int j = 0; j < K; ++j)
-            if (o + j * S < nouts) store_unit(t.at(oe[j].rb, (uint64_t)oe[j].off + at, sizeof(T)), v);
+            if (o + j * S < nouts) store_unit<NT>(t.at(oe[j].rb, (uint64_t)oe[j].off + at, sizeof(T)), v);
         o += K * S;
 #pragma unroll
         for (int j = 0; j < K; ++j)
@@ -98,7 +98,7 @@ __device__ __forceinline__ void narrow_item(const GredItem& it, const Table& t, 
     }
 }
 
-template <typename T, bool BATCH>
+template <typename T, bool BATCH, bool NT>
 __global__ void __launch_bounds__(1024) gnarrow_kernel(const GredItem* __restrict__ items,
                                                        const PoolEntry* __restrict__ pool, BufTable tab,
                                                        const BufTable* __restrict__ tabs) {
@@ -113,37 +113,41 @@ __global__ void __launch_bounds__(1024) gnarrow_kernel(const GredItem* __restric
     }
     constexpr uint32_t VE = Vec<T>::N;
     if (it.n >= VE)
-        narrow_item<T, Vec<T>>(it, t, pool, (it.n + VE - 1) / VE, VE, reinterpret_cast<Vec<T>*>(lds_raw));
+        narrow_item<T, Vec<T>, NT>(it, t, pool, (it.n + VE - 1) / VE, VE, reinterpret_cast<Vec<T>*>(lds_raw));
     else
-        narrow_item<T, T>(it, t, pool, it.n, 1, reinterpret_cast<T*>(lds_raw));
+        narrow_item<T, T, false>(it, t, pool, it.n, 1, reinterpret_cast<T*>(lds_raw));
 }
 
-template <typename T>
+template <typename T, bool NT>
 hipError_t launch_t(const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
                     const BufTable* tabs, bool batch, int threads, hipStream_t st) {
     const size_t lds = (size_t)threads * 16;
     if (batch)
-        hipLaunchKernelGGL((gnarrow_kernel<T, true>), dim3(n), dim3(threads), lds, st, items, pool, tab, tabs);
+        hipLaunchKernelGGL((gnarrow_kernel<T, true, NT>), dim3(n), dim3(threads), lds, st, items, pool, tab, tabs);
     else
-        hipLaunchKernelGGL((gnarrow_kernel<T, false>), dim3(n), dim3(threads), lds, st, items, pool, tab, tabs);
+        hipLaunchKernelGGL((gnarrow_kernel<T, false, NT>), dim3(n), dim3(threads), lds, st, items, pool, tab, tabs);
     return hipGetLastError();
 }
 
 }  // namespace
 
-// One workgroup of `threads` lanes per item; every item's units must fit the workgroup (lower_narrow).
+// stream: vectors are loaded and stored past the caches.  One workgroup of `threads` lanes per item; every item's units must fit the workgroup (lower_narrow).
 hipError_t launch_gnarrow(int dtype, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
-                          const BufTable* tabs, bool batch, int threads, hipStream_t st) {
+                          const BufTable* tabs, bool batch, int threads, bool stream, hipStream_t st) {
     if (n == 0) return hipSuccess;
     if (threads < 64 || threads > 1024 || (threads & (threads - 1))) return hipErrorInvalidValue;
+#define BINE_NARROW(T)                                                                \
+    return stream ? launch_t<T, true>(items, n, pool, tab, tabs, batch, threads, st)  \
+                  : launch_t<T, false>(items, n, pool, tab, tabs, batch, threads, st)
     switch (dtype) {
-    case 0: return launch_t<int32_t>(items, n, pool, tab, tabs, batch, threads, st);
-    case 1: return launch_t<int64_t>(items, n, pool, tab, tabs, batch, threads, st);
-    case 2: return launch_t<float>(items, n, pool, tab, tabs, batch, threads, st);
-    case 3: return launch_t<double>(items, n, pool, tab, tabs, batch, threads, st);
-    case 4: return launch_t<int8_t>(items, n, pool, tab, tabs, batch, threads, st);
+    case 0: BINE_NARROW(int32_t);
+    case 1: BINE_NARROW(int64_t);
+    case 2: BINE_NARROW(float);
+    case 3: BINE_NARROW(double);
+    case 4: BINE_NARROW(int8_t);
     default: return hipErrorInvalidValue;
     }
+#undef BINE_NARROW
 }
 
 }  // namespace bine

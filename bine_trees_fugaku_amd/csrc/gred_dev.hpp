@@ -112,21 +112,19 @@ __device__ __forceinline__ void vstore(char* p, const Vec<T>& v) {
 }
 
 // Units of the narrow and tree kernels: a 16-byte vector at any byte address, or one element.
-template <typename T>
+template <bool NT = false, typename T>
 __device__ __forceinline__ Vec<T> load_unit(const char* p, Vec<T>*) {
-    Vec<T> r;
-    r.raw = *gptr<const u4b>(p);
-    return r;
+    return vload<T, NT>(p);
 }
-template <typename T>
+template <bool NT = false, typename T>
 __device__ __forceinline__ T load_unit(const char* p, T*) {
     return *gptr<const T>(p);
 }
-template <typename T>
+template <bool NT = false, typename T>
 __device__ __forceinline__ void store_unit(char* p, const Vec<T>& v) {
-    *gptr<u4b>(p) = v.raw;
+    vstore<T, NT>(p, v);
 }
-template <typename T>
+template <bool NT = false, typename T>
 __device__ __forceinline__ void store_unit(char* p, T v) {
     *gptr<T>(p) = v;
 }

@@ -2145,10 +2145,9 @@ constexpr uint32_t kNarrowThreads = 1024;
 // The narrow kernel spreads leaves and outputs over the lanes, the general shape (256 lanes, one vector each) only
 // elements, so the line is where the general shape leaves the chip idle: too few workgroups for 256 compute units, or
 // blocks that fill a small part of a tile.  Microseconds per launch, general / narrow, fp32:
-//   few workgroups: 512 ranks, reduce of 32768 elements (128 workgroups) 27.2 / 16.2, of 98304 (384) 34.6 / 43.8 or
-//     36.7 by workgroup size, of 131072 (512) 43 / 58; 64 ranks, allreduce of 65536 (256) 9.7 / 8.4, of 131072 (512)
-//     14.0 / 14.8; bcast to 512 ranks of 131072 (128) 84 / 44, of 262144 (256) 119 / 107
-//     but of 262146 (257, realigned stores) 156 / 167;
+//   few workgroups: 512 ranks, reduce of 32768 elements (128 workgroups) 27.2 / 16.2, of 65536 (256) 33.8 / 35.2 with
+//     buffers rotating; 64 ranks, allreduce of 65536 (256) 9.7 / 8.4, of 131072 (512) 14.0 / 14.8; bcast to 512 ranks of
+//     131072 (128) 84 / 44, of 262146 (257, realigned stores) 156 / 167;
 //   eight leaves or outputs need no spreading: 8 ranks, allreduce of 65536 (64) 4.65 / 4.58, of 131072 (128) 4.9 / 5.1;
 //   short blocks on 512 ranks: allreduce of 65536 (32 vectors a block) 92 / 53, of 262144 (128) 288 / 259; allgather of
 //     256 (64) 101 / 59, of 512 (128) 141 / 140; reduce_scatter of 128 (32) 36.9 / 31.0, of 192 (48) 37.5 / 45.1.
@@ -2156,10 +2155,10 @@ bool narrow_pays(const std::vector<std::vector<Group>>& launches, int vec) {
     if (launches.size() != 1) return false;
     size_t fan = 0;
     uint64_t workgroups = 0, units = 0, short_units = 0;
-    bool reduces = false;
+    bool spreads = false;  // reductions with several outputs
     for (const Group& g : launches[0]) {
         fan = std::max({fan, g.leaves.size(), g.outs.size()});
-        reduces = reduces || g.lg > 0;
+        spreads = spreads || (g.lg > 0 && g.outs.size() > 1);
         const uint64_t u = (uint64_t)narrow_units(g, vec), ends = g.leaves.size() + g.outs.size();
         const uint64_t tile = g.lg >= 5 ? 64 : 256;
         workgroups += (u + tile - 1) / tile;
@@ -2167,7 +2166,7 @@ bool narrow_pays(const std::vector<std::vector<Group>>& launches, int vec) {
         if (u <= (g.lg > 0 && g.outs.size() == 1 ? 32u : 128u)) short_units += u * ends;
     }
     if (fan < 16) return fan >= 4 && workgroups < 128;
-    return workgroups < (reduces ? 512u : 256u) || 2 * short_units >= units;
+    return workgroups < (spreads ? 512u : 256u) || 2 * short_units >= units;
 }
 
 void lower_narrow(const std::vector<std::vector<Group>>& launches, int vec, uint32_t bucket, size_t dtsize,
@@ -2185,6 +2184,18 @@ void lower_narrow(const std::vector<std::vector<Group>>& launches, int vec, uint
     const uint32_t threads =
         (uint32_t)std::min<uint64_t>(kNarrowThreads, std::max<uint64_t>({64, need, pow2_at_least(lanes / 256)}));
     out->narrow_threads = (int)threads;
+    // Reductions with several outputs stream from 16 MB on where their blocks hold whole lines (buffers rotating, GPU
+    // microseconds, plain / streaming): 512 ranks' allreduce of 16384 fp32 elements 22.6 / 16.9, of 65536 73.9 / 60.5, 64
+    // ranks' of 65536 11.8 / 9.2; with the buffers in cache 17.7 / 14.8, 53.9 / 58.3, 8.5 / 7.1.  Shorter or unaligned
+    // blocks do not (512 ranks of 5003 16.1 / 19.0), nor copies and single outputs (bcast to 512 ranks of 65536 34 / 40).
+    uint64_t moved = 0;
+    bool spread = true, lines = true;
+    for (const Group& g : gs) {
+        moved += (uint64_t)g.n * (g.leaves.size() + g.outs.size()) * dtsize;
+        spread = spread && g.lg > 0 && g.outs.size() > 1;
+        lines = lines && g.n % (8 * vec) == 0;
+    }
+    out->narrow_stream = spread && lines && moved >= (16u << 20);
     for (size_t gi = 0; gi < gs.size(); ++gi) {
         const Group& g = gs[gi];
         if (g.n <= 0) continue;

@@ -120,6 +120,7 @@ struct Lowered {
     std::vector<uint32_t> packs;  // per launch: how many of its items are ITEM_PACK items (after the runs)
     uint64_t bytes_read = 0, bytes_written = 0, max_leaves = 0;
     int narrow_threads = 0;  // > 0: every item is ITEM_NARROW, run by the narrow kernel with workgroups of that many lanes
+    bool narrow_stream = false;  // with streaming loads and stores
     // tree_waves > 0: every item is ITEM_TREE, run by the tree kernel with that many waves and a stack that deep
     int tree_waves = 0, tree_stack = 0;
     bool unaligned_outs = false;  // some vector item writes an output whose offset is not a whole number of vectors

@@ -87,7 +87,8 @@ typedef enum { BINE_REDUCE_BINOMIAL_TREE = 0, BINE_REDUCE_REDUCE_SCATTER_GATHER 
 
 /* How a collective executes on the GPU.  Both produce bit-identical results:
  * STEP launches one gather-reduce kernel per schedule step (the reference's
- * message structure); FUSED compiles the whole schedule into one launch that
+ * message structure); FUSED compiles the whole schedule into one launch (or two,
+ * where reductions write many outputs: first the sums, then their copies) that
  * reads every input once and writes every output once, replaying each output
  * element's reduction tree in the reference's association order. */
 typedef enum { BINE_EXEC_AUTO = 0, BINE_EXEC_STEP = 1, BINE_EXEC_FUSED = 2 } bine_exec_t;
