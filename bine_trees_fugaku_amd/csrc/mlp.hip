@@ -5,7 +5,8 @@
 // hidden layers apply ReLU, the last layer is linear.  Parameters live in one
 // flat fp32 buffer, layer by layer: W_l (out_l x in_l, row-major), then b_l.
 //
-// Every product is one tiled GEMM on the matrix cores: a 64x64 output tile
+// Networks no wider than 256 run whole rows through all layers per workgroup (mlp_rows).  In wider ones every
+// product is one tiled GEMM on the matrix cores: a 64x64 output tile
 // per 256-thread workgroup, each wave owning a 32x32 quarter built from 2x2
 // v_mfma_f32_16x16x4f32 blocks, operands staged through LDS in K chunks of 64
 // (16-byte loads and LDS stores), the next chunk loaded into registers while
@@ -111,27 +112,21 @@ struct Panel {
     }
 };
 
-// C[M x N] = op(A)[M x K] * op(B)[K x N] with the epilogue above.
+// One 64 x 64 tile (at row m0, column n0) of C[M x N] = op(A)[M x K] * op(B)[K x N] over k in [kbeg, kend), with the
+// epilogue above, by a workgroup of 256 lanes.
 // op(A)[m][k] = TA ? A[k * lda + m] : A[m * lda + k]
 // op(B)[k][n] = TB ? B[n * ldb + k] : B[k * ldb + n]
-// Split K: workgroup z covers k in [z * kc, min(K, (z + 1) * kc)) and, when
-// gridDim.z > 1, writes its partial product to C + z * M * ldc (EPI_PLAIN only;
-// sum_partials adds the slices in order).
 //
 // The K loop is software-pipelined: the next chunk's operands are loaded into
 // registers while the matrix cores work on the current chunk from LDS.
 template <bool TA, bool TB>
-__global__ __launch_bounds__(256) void gemm_f32(int M, int N, int K, int kc, const float* __restrict__ A, int lda,
-                                                const float* __restrict__ B, int ldb, float* __restrict__ C, int ldc,
-                                                const float* __restrict__ bias, const float* __restrict__ mask, int epi) {
+__device__ __forceinline__ void gemm_tile(int M, int N, int m0, int n0, int kbeg, int kend, const float* __restrict__ A,
+                                          int lda, const float* __restrict__ B, int ldb, float* __restrict__ C, int ldc,
+                                          const float* __restrict__ bias, const float* __restrict__ mask, int epi) {
     __shared__ __align__(16) float As[TK * SR];  // room for either orientation (SR >= SK)
     __shared__ __align__(16) float Bs[TK * SR];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    const int kbeg = blockIdx.z * kc;
-    const int kend = kbeg + kc < K ? kbeg + kc : K;
-    C += (size_t)blockIdx.z * M * ldc;
     const Panel<!TA> pa{A, lda, m0, M, (lda & 3) == 0 && ((uintptr_t)A & 15) == 0};
     const Panel<TB> pb{B, ldb, n0, N, (ldb & 3) == 0 && ((uintptr_t)B & 15) == 0};
     floatx4 acc[2][2];
@@ -248,6 +243,17 @@ __global__ __launch_bounds__(256) void gemm_f32(int M, int N, int K, int kc, con
     }
 }
 
+// The product's tiles over the grid.  Split K: workgroup z covers k in [z * kc, min(K, (z + 1) * kc)) and, when
+// gridDim.z > 1, writes its partial product to C + z * M * ldc (EPI_PLAIN only; sum_partials adds the slices in order).
+template <bool TA, bool TB>
+__global__ __launch_bounds__(256) void gemm_f32(int M, int N, int K, int kc, const float* __restrict__ A, int lda,
+                                                const float* __restrict__ B, int ldb, float* __restrict__ C, int ldc,
+                                                const float* __restrict__ bias, const float* __restrict__ mask, int epi) {
+    const int kbeg = blockIdx.z * kc;
+    gemm_tile<TA, TB>(M, N, blockIdx.y * TM, blockIdx.x * TN, kbeg, kbeg + kc < K ? kbeg + kc : K, A, lda, B, ldb,
+                      C + (size_t)blockIdx.z * M * ldc, ldc, bias, mask, epi);
+}
+
 // dY = 2 * mask * (Y - T) / max(count, 1); per-block partial sums of the loss
 // terms mask * (Y - T)^2 and of the mask, reduced in a fixed order.
 __global__ __launch_bounds__(256) void mse_grad(int n_elems, const float* __restrict__ Y, const float* __restrict__ T,
@@ -361,6 +367,337 @@ __global__ void adam_update(uint64_t n, float* __restrict__ p, const float* __re
     }
 }
 
+// ---- networks whose rows fit a workgroup --------------------------------------------------------------------------
+//
+// Widths up to 256: a workgroup takes 16 rows through every layer, forward and back, with their activations in LDS, so
+// a pass is one launch instead of one or two per layer, and the weight gradients of all layers are one more.  The limit
+// is what eight waves hold as 32 columns each; wider networks run layer by layer, as all did before.
+//
+// 18-256-256-256-28, microseconds of a forward pass and of loss and gradients (training step alike), layer by layer
+// (30 launches for the gradients) and here (3):
+//   rows       1           64          1007        4096        8192
+//   forward    42 -> 24    37 -> 25    49 -> 25    44 -> 26    55 -> 42
+//   gradients  113 -> 51   104 -> 53   172 -> 65   168 -> 82   222 -> 135
+// Of the 82 about 50 are mlp_rows, 29 mlp_weight_grads (1.2 GFLOP: 8 us of matrix instructions) and 5 mlp_finish.  A row
+// workgroup is bound by latency: its 256 x 256 layer is 3.4 us of matrix instructions and takes about 7, waiting for
+// weights out of L2.  Four waves of 64 columns took 10 (4096 rows: 29 and 90), three chunks of weights in flight going
+// back instead of two lost the second workgroup of a CU (8192 rows: 150 against 135), and more slices of the weight
+// gradients' rows changed nothing.
+
+constexpr int kRows = 16;    // rows per workgroup: one matrix-instruction tile
+constexpr int kWidth = 256;  // 32 columns for each of the eight waves
+constexpr int kWaves = 8;    // two on each SIMD: one multiplies while the other waits for its weights
+constexpr int kMaxLayers = 15;
+
+struct Net {
+    int layers;
+    int dims[kMaxLayers + 1];
+    const float* params;
+    uint32_t w_off[kMaxLayers], b_off[kMaxLayers];
+    float* act[kMaxLayers];  // outputs of each layer
+    float* dz[kMaxLayers];   // loss gradients of each layer's sums, before the factor 2 / count
+};
+
+__host__ __device__ inline int row_stride(int width) { return (width + 31) / 32 * 32 + 4; }  // floats of an LDS row
+
+typedef float f4w __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f2w __attribute__((ext_vector_type(2), aligned(4)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+
+// Four floats at p[0 .. 3], zero from `left` on.
+__device__ __forceinline__ floatx4 load4(const float* p, int left) {
+    if (left >= 4) return *reinterpret_cast<const f4w*>(p);
+    floatx4 v = {0.f, 0.f, 0.f, 0.f};
+    if (left > 0) v[0] = p[0];
+    if (left > 1) v[1] = p[1];
+    if (left > 2) v[2] = p[2];
+    return v;
+}
+
+// A wave's M column tiles (wave, wave + 8) of 16 rows times W^T: chunks of 32 k, so that a line of weights is used
+// whole when it is fetched (every workgroup reads them all from L2), the next chunk's loads in flight.  Whole chunks are
+// loaded without a test of the lane's own k, which would wait for each load, and M is a constant, so a chunk's products
+// are straight code.
+template <int M>
+__device__ __forceinline__ void forward_tiles(floatx4 (&acc)[2], const float* __restrict__ W, const float* src, int K,
+                                              int N, int S, int wave, int lr, int lk) {
+    const int chunks = (K + 31) / 32;
+    const float* wp[M];
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+        const int col = (wave + kWaves * i) * 16 + lr;
+        wp[i] = W + (size_t)(col < N ? col : N - 1) * K + 8 * lk;
+    }
+    auto fetch = [&](floatx4 (&w)[M][2], int c) __attribute__((always_inline)) {
+        if (32 * c + 32 <= K) {
+#pragma unroll
+            for (int i = 0; i < M; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) w[i][h] = *reinterpret_cast<const f4w*>(wp[i] + 32 * c + 4 * h);
+        } else if (c < chunks) {
+#pragma unroll
+            for (int i = 0; i < M; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) w[i][h] = load4(wp[i] + 32 * c + 4 * h, K - 32 * c - 8 * lk - 4 * h);
+        }
+    };
+    auto multiply = [&](const floatx4 (&w)[M][2], int c) __attribute__((always_inline)) {
+        floatx4 a[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) a[h] = *reinterpret_cast<const floatx4*>(src + lr * S + 32 * c + 8 * lk + 4 * h);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < M; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h][j], w[i][h][j], acc[i], 0, 0, 0);
+    };
+    floatx4 w0[M][2] = {}, w1[M][2] = {};
+    fetch(w0, 0);
+    for (int c = 0; c < chunks; c += 2) {
+        fetch(w1, c + 1);
+        multiply(w0, c);
+        if (c + 1 >= chunks) break;
+        fetch(w0, c + 2);
+        multiply(w1, c + 1);
+    }
+}
+
+// Forward pass of 16 rows; BACK: also the loss terms and the gradients dz down to the first layer.  Lane l of a wave
+// supplies row l % 16 and eight consecutive k of a chunk of 32, one per matrix instruction, so fragments are read 16
+// bytes at a time.  Forward, a wave owns the column tiles wave and wave + 8; backward, 32 consecutive
+// columns, tile j holding the columns 2 i + j, so that a row of weights is read and a row of results written 8 bytes a
+// lane.  Registers are held to 128, for two workgroups on a CU.
+template <bool BACK>
+__global__ __launch_bounds__(64 * kWaves, 4) void mlp_rows(Net net, const float* __restrict__ x, int n, float* __restrict__ y,
+                                                const float* __restrict__ t, const float* __restrict__ mask,
+                                                float* __restrict__ partial) {
+    extern __shared__ __align__(16) float slots[];  // the rows' inputs, then every layer's outputs
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row0 = blockIdx.x * kRows, rows = n - row0 < kRows ? n - row0 : kRows;
+    const int L = net.layers;
+    float* src = slots;
+    {
+        const int K = net.dims[0], S = row_stride(K);
+        for (int i = tid; i < kRows * S; i += 64 * kWaves) {
+            const int r = i / S, c = i - r * S;
+            src[i] = r < rows && c < K ? x[(size_t)(row0 + r) * K + c] : 0.f;
+        }
+    }
+    __syncthreads();
+    for (int l = 0; l < L; ++l) {
+        const int K = net.dims[l], N = net.dims[l + 1], S = row_stride(K), T = row_stride(N);
+        float* dst = src + kRows * S;
+        const float* W = net.params + net.w_off[l];
+        const int tiles = (N + 15) / 16, mine = (tiles - wave + kWaves - 1) / kWaves;
+        floatx4 acc[2] = {};
+        switch (mine) {
+        case 2: forward_tiles<2>(acc, W, src, K, N, S, wave, lr, lk); break;
+        case 1: forward_tiles<1>(acc, W, src, K, N, S, wave, lr, lk); break;
+        default: break;
+        }
+        const bool last = l == L - 1;
+        float* out = last && !BACK ? y : net.act[l];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if (i >= mine) continue;
+            const int col = (wave + kWaves * i) * 16 + lr;
+            const float b = col < N ? net.params[net.b_off[l] + col] : 0.f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 4 * lk + r;
+                float v = acc[i][r] + b;
+                if (!last) v = v > 0.f ? v : 0.f;
+                dst[row * T + col] = col < N ? v : 0.f;  // the columns up to a whole chunk are the next layer's zeros
+                if ((BACK || last) && row < rows && col < N) out[(size_t)(row0 + row) * N + col] = v;
+            }
+        }
+        if ((tiles & 1) && tid < 256) dst[(tid >> 4) * T + 16 * tiles + (tid & 15)] = 0.f;
+        __syncthreads();
+        src = dst;
+    }
+    if (!BACK) return;
+    float loss = 0.f, count = 0.f;
+    {
+        const int N = net.dims[L], S = row_stride(N);
+        for (int i = tid; i < rows * N; i += 64 * kWaves) {
+            const int r = i / N, c = i - r * N;
+            const size_t g = (size_t)row0 * N + i;
+            const float m = mask[g], d = m > 0.f ? src[r * S + c] - t[g] : 0.f;
+            src[r * S + c] = d;
+            net.dz[L - 1][g] = d;
+            loss += d * d;
+            count += m > 0.f ? 1.f : 0.f;
+        }
+        for (int i = tid; i < (kRows - rows) * N; i += 64 * kWaves) src[(rows + i / N) * S + i % N] = 0.f;  // rows past the batch
+    }
+    __syncthreads();
+    for (int l = L - 1; l > 0; --l) {
+        const int K = net.dims[l + 1], N = net.dims[l], S = row_stride(K), T = row_stride(N);
+        float* dst = src - kRows * T;  // the activations below: read as the ReLU's mask, replaced by their gradient
+        const int col = wave * 32 + 2 * lr;
+        if (wave * 32 < N) {
+            const float* wp = net.params + net.w_off[l] + (uint32_t)(8 * lk * N + col);
+            const int chunks = (K + 31) / 32;
+            floatx4 acc[2] = {};
+            const bool wide = wave * 32 + 32 <= N;
+            auto fetch = [&](floatx2 (&w)[8], int c) __attribute__((always_inline)) {
+                if (wide && 32 * c + 32 <= K) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) w[j] = *reinterpret_cast<const f2w*>(wp + (uint32_t)((32 * c + j) * N));
+                } else if (c < chunks) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const int k = 32 * c + 8 * lk + j;
+                        w[j][0] = k < K && col < N ? wp[(uint32_t)((32 * c + j) * N)] : 0.f;
+                        w[j][1] = k < K && col + 1 < N ? wp[(uint32_t)((32 * c + j) * N) + 1] : 0.f;
+                    }
+                }
+            };
+            auto multiply = [&](const floatx2 (&w)[8], int c) __attribute__((always_inline)) {
+                floatx4 a[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) a[h] = *reinterpret_cast<const floatx4*>(src + lr * S + 32 * c + 8 * lk + 4 * h);
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j >> 2][j & 3], w[j][i], acc[i], 0, 0, 0);
+            };
+            floatx2 w0[8], w1[8] = {};
+            fetch(w0, 0);
+            for (int c = 0; c < chunks; c += 2) {
+                fetch(w1, c + 1);
+                multiply(w0, c);
+                if (c + 1 >= chunks) break;
+                fetch(w0, c + 2);
+                multiply(w1, c + 1);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 4 * lk + r;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    if (col + i >= N) continue;
+                    float* p = dst + row * T + col + i;
+                    const float v = *p > 0.f ? acc[i][r] : 0.f;
+                    *p = v;
+                    if (row < rows) net.dz[l - 1][(size_t)(row0 + row) * N + col + i] = v;
+                }
+            }
+        }
+        __syncthreads();
+        src = dst;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        loss += __shfl_xor(loss, o, 64);
+        count += __shfl_xor(count, o, 64);
+    }
+    __syncthreads();
+    if (lane == 0) {
+        slots[2 * wave] = loss;
+        slots[2 * wave + 1] = count;
+    }
+    __syncthreads();
+    if (tid < 2) {
+        float v = 0.f;
+        for (int w = 0; w < kWaves; ++w) v += slots[2 * w + tid];
+        partial[2 * blockIdx.x + tid] = v;
+    }
+}
+
+// Rows [z * kc, (z + 1) * kc) of every layer's weight and bias gradients, into work + z * stride at the parameters' own
+// offsets.  A workgroup takes a 64 x 64 tile of one layer's weights, or 64 of its biases, or (the last one) the totals
+// of the loss terms; first[l] is layer l's first weight tile, first_bias[l] its first group of biases.
+struct GradTiles {
+    int first[kMaxLayers + 1], first_bias[kMaxLayers + 1];
+};
+
+__global__ __launch_bounds__(256) void mlp_weight_grads(Net net, GradTiles g, const float* __restrict__ x, int n, int kc,
+                                                        float* __restrict__ work, uint64_t stride, int nb,
+                                                        const float* __restrict__ partial, float* __restrict__ totals) {
+    __shared__ float s[4][64];
+    const int L = net.layers, b = blockIdx.x, z = blockIdx.y;
+    const int k0 = z * kc, k1 = k0 + kc < n ? k0 + kc : n;
+    float* out = work + (uint64_t)z * stride;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (b < g.first[L]) {
+        int l = 0;
+        while (b >= g.first[l + 1]) ++l;
+        const int M = net.dims[l + 1], N = net.dims[l], across = (N + TN - 1) / TN, tile = b - g.first[l];
+        gemm_tile<true, false>(M, N, tile / across * TM, tile % across * TN, k0, k1, net.dz[l], M, l ? net.act[l - 1] : x, N,
+                               out + net.w_off[l], N, nullptr, nullptr, EPI_PLAIN);
+    } else if (b < g.first_bias[L]) {
+        int l = 0;
+        while (b >= g.first_bias[l + 1]) ++l;
+        const int cols = net.dims[l + 1], col = (b - g.first_bias[l]) * 64 + lane;
+        const float* dz = net.dz[l];
+        float acc = 0.f;
+        if (col < cols) {
+            int i = k0 + wave;
+            for (; i + 28 < k1; i += 32) {  // eight rows loaded, then added in order
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = dz[(size_t)(i + 4 * u) * cols + col];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) acc += v[u];
+            }
+            for (; i < k1; i += 4) acc += dz[(size_t)i * cols + col];
+        }
+        s[wave][lane] = acc;
+        __syncthreads();
+        if (wave == 0 && col < cols) out[net.b_off[l] + col] = (s[0][lane] + s[1][lane]) + (s[2][lane] + s[3][lane]);
+    } else if (z == 0) {
+        float v[2] = {0.f, 0.f};
+        for (int i = tid; i < nb; i += 256) {
+            v[0] += partial[2 * i];
+            v[1] += partial[2 * i + 1];
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            v[0] += __shfl_xor(v[0], o, 64);
+            v[1] += __shfl_xor(v[1], o, 64);
+        }
+        if (lane == 0) {
+            s[wave][0] = v[0];
+            s[wave][1] = v[1];
+        }
+        __syncthreads();
+        if (tid < 2) totals[tid] = (s[0][tid] + s[1][tid]) + (s[2][tid] + s[3][tid]);
+    }
+}
+
+// The slices' sum in order, times 2 / count: into grads, or (p not NULL) as the gradient of one Adam step.
+__global__ void mlp_finish(uint64_t n, int nz, const float* __restrict__ work, const float* __restrict__ totals,
+                           float* __restrict__ grads, float* __restrict__ loss_out, float* __restrict__ p,
+                           float* __restrict__ m, float* __restrict__ v, float lr, float b1, float b2, float eps, float c1,
+                           float c2) {
+    const float cnt = fmaxf(totals[1], 1.f), inv = 2.f / cnt;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+        float acc = work[i];
+        int z = 1;
+        for (; z + 8 <= nz; z += 8) {  // eight slices loaded, then added in order
+            float a[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) a[u] = work[(uint64_t)(z + u) * n + i];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) acc += a[u];
+        }
+        for (; z < nz; ++z) acc += work[(uint64_t)z * n + i];
+        const float gi = inv * acc;
+        if (p) {
+            const float mi = b1 * m[i] + (1.f - b1) * gi;
+            const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
+            m[i] = mi;
+            v[i] = vi;
+            p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+        } else {
+            grads[i] = gi;
+        }
+    }
+    if (loss_out && blockIdx.x == 0 && threadIdx.x == 0) loss_out[0] = totals[0] / cnt;
+}
+
 template <bool TA, bool TB>
 void gemm(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C, int ldc, const float* bias,
           const float* mask, int epi, hipStream_t st) {
@@ -425,12 +762,17 @@ struct bine_mlp_s {
     float *dz0 = nullptr, *dz1 = nullptr;  // ping-pong n x max width
     float *partial = nullptr, *totals = nullptr;
     float* work = nullptr;  // split-K partial products
+    bool rows = false;         // mlp_rows and its companions run this network
+    std::vector<float*> dz;    // per layer, for them
+    size_t rows_lds = 0;
     uint64_t step = 0;
     hipStream_t last = nullptr;  // stream of the last launch; host copies wait for it
     ~bine_mlp_s() {
         for (float* p : {params, grads, adam_m, adam_v, dz0, dz1, partial, totals, work})
             if (p) (void)hipFree(p);
         for (float* p : act)
+            if (p) (void)hipFree(p);
+        for (float* p : dz)
             if (p) (void)hipFree(p);
     }
     int layers() const { return (int)dims.size() - 1; }
@@ -451,6 +793,46 @@ uint64_t splitmix64(uint64_t& s) {
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
     return z ^ (z >> 31);
+}
+
+Net net_of(bine_mlp_t m) {
+    Net net{};
+    net.layers = m->layers();
+    for (int l = 0; l <= net.layers; ++l) net.dims[l] = m->dims[l];
+    net.params = m->params;
+    for (int l = 0; l < net.layers; ++l) {
+        net.w_off[l] = (uint32_t)m->w_off[l];
+        net.b_off[l] = (uint32_t)m->b_off[l];
+        net.act[l] = m->act[l];
+        net.dz[l] = m->dz[l];
+    }
+    return net;
+}
+
+// Forward pass over n rows of x into y.
+void rows_forward(bine_mlp_t m, const float* x, int n, float* y, hipStream_t st) {
+    hipLaunchKernelGGL((mlp_rows<false>), dim3((n + kRows - 1) / kRows), dim3(64 * kWaves), m->rows_lds, st, net_of(m), x, n, y,
+                       nullptr, nullptr, nullptr);
+}
+
+// Loss and gradients of the masked MSE into grads, or (lr > 0) one Adam step.
+void rows_gradients(bine_mlp_t m, const float* x, const float* t, const float* mask, int n, float* grads, float* loss,
+                    float lr, float b1, float b2, float c1, float c2, hipStream_t st) {
+    const Net net = net_of(m);
+    const int nb = (n + kRows - 1) / kRows;
+    hipLaunchKernelGGL((mlp_rows<true>), dim3(nb), dim3(64 * kWaves), m->rows_lds, st, net, x, n, nullptr, t, mask, m->partial);
+    GradTiles g{};
+    for (int l = 0; l < net.layers; ++l)
+        g.first[l + 1] = g.first[l] + ((net.dims[l + 1] + TM - 1) / TM) * ((net.dims[l] + TN - 1) / TN);
+    g.first_bias[0] = g.first[net.layers];
+    for (int l = 0; l < net.layers; ++l) g.first_bias[l + 1] = g.first_bias[l] + (net.dims[l + 1] + 63) / 64;
+    const int tiles = g.first[net.layers], nz = k_slices(n, tiles);
+    const int kc = ((n + nz - 1) / nz + TK - 1) / TK * TK, nzr = (n + kc - 1) / kc;
+    hipLaunchKernelGGL(mlp_weight_grads, dim3(g.first_bias[net.layers] + 1, nzr), dim3(256), 0, st, net, g, x, n, kc,
+                       m->work, m->nparams, nb, m->partial, m->totals);
+    hipLaunchKernelGGL(mlp_finish, dim3((int)std::min<uint64_t>(1024, (m->nparams + 255) / 256)), dim3(256), 0, st,
+                       m->nparams, nzr, m->work, m->totals, grads, loss, lr > 0.f ? m->params : nullptr, m->adam_m,
+                       m->adam_v, lr, b1, b2, 1e-8f, c1, c2);
 }
 
 // Forward pass over n rows of x; leaves every layer's output in m->act.
@@ -543,6 +925,36 @@ extern "C" int bine_mlp_create(const int32_t* dims, int32_t ndims, int32_t max_b
         MHIP(hipMalloc(&a, sizeof(float) * (size_t)max_batch * dims[l + 1]));
         m->act.push_back(a);
     }
+    // widths a workgroup of eight waves covers and activations that LDS holds: the whole network per 16 rows
+    for (int i = 0; i < ndims; ++i) m->rows_lds += sizeof(float) * kRows * row_stride(dims[i]);
+    int lds = 0;
+    MHIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
+    m->rows = widest <= kWidth && ndims - 1 <= kMaxLayers && m->rows_lds <= (size_t)lds;
+    if (m->rows && m->rows_lds > 65536) {
+        if (hipFuncSetAttribute((const void*)mlp_rows<false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess ||
+            hipFuncSetAttribute((const void*)mlp_rows<true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) {
+            (void)hipGetLastError();
+            m->rows = false;
+        }
+    }
+    for (int l = 0; m->rows && l + 1 < ndims; ++l) {  // without room for every layer's gradients: layer by layer
+        float* a = nullptr;
+        if (hipMalloc(&a, sizeof(float) * (size_t)max_batch * dims[l + 1]) == hipSuccess) {
+            m->dz.push_back(a);
+            continue;
+        }
+        (void)hipGetLastError();
+        for (float* d : m->dz) (void)hipFree(d);
+        m->dz.clear();
+        m->rows = false;
+    }
+    if (m->rows) {
+        MHIP(hipMalloc(&m->work, sizeof(float) * kMaxSplit * off));
+        MHIP(hipMalloc(&m->partial, sizeof(float) * 2 * (((size_t)max_batch + kRows - 1) / kRows)));
+        MHIP(hipMalloc(&m->totals, sizeof(float) * 2));
+        *out = m.release();
+        return BINE_OK;
+    }
     MHIP(hipMalloc(&m->dz0, sizeof(float) * (size_t)max_batch * widest));
     MHIP(hipMalloc(&m->dz1, sizeof(float) * (size_t)max_batch * widest));
     size_t widest_w = 0;
@@ -587,6 +999,16 @@ extern "C" int bine_mlp_forward(bine_mlp_t m, const float* x, int32_t n, float* 
     MHIP(hipSetDevice(m->device));
     hipStream_t st = (hipStream_t)stream;
     m->last = st;
+    if (m->rows) {
+        // workgroups read and write rows at different times: an output over the input is written elsewhere first
+        const float *x_end = x + (size_t)n * m->dims.front(), *y_end = y + (size_t)n * m->dims.back();
+        const bool over = y < x_end && x < y_end;
+        rows_forward(m, x, n, over ? m->act.back() : y, st);
+        if (over)
+            MHIP(hipMemcpyAsync(y, m->act.back(), sizeof(float) * (size_t)n * m->dims.back(), hipMemcpyDeviceToDevice, st));
+        MHIP(hipGetLastError());
+        return BINE_OK;
+    }
     forward(m, x, n, st);
     MHIP(hipMemcpyAsync(y, m->act.back(), sizeof(float) * (size_t)n * m->dims.back(), hipMemcpyDeviceToDevice, st));
     MHIP(hipGetLastError());
@@ -601,6 +1023,11 @@ extern "C" int bine_mlp_gradients(bine_mlp_t m, const float* x, const float* t, 
     MHIP(hipSetDevice(m->device));
     hipStream_t st = (hipStream_t)stream;
     m->last = st;
+    if (m->rows) {
+        rows_gradients(m, x, t, mask, n, grads, loss, 0.f, 0.f, 0.f, 1.f, 1.f, st);
+        MHIP(hipGetLastError());
+        return BINE_OK;
+    }
     forward(m, x, n, st);
     backward(m, x, t, mask, n, loss, st);
     MHIP(hipMemcpyAsync(grads, m->grads, sizeof(float) * m->nparams, hipMemcpyDeviceToDevice, st));
@@ -617,11 +1044,17 @@ extern "C" int bine_mlp_train_step(bine_mlp_t m, const float* x, const float* t,
     MHIP(hipSetDevice(m->device));
     hipStream_t st = (hipStream_t)stream;
     m->last = st;
+    const float b1 = 0.9f, b2 = 0.999f;
+    const float s1 = (float)(m->step + 1), c1 = 1.f - std::pow(b1, s1), c2 = 1.f - std::pow(b2, s1);
+    if (m->rows) {
+        rows_gradients(m, x, t, mask, n, nullptr, loss, lr, b1, b2, c1, c2, st);
+        MHIP(hipGetLastError());
+        m->step += 1;
+        return BINE_OK;
+    }
     forward(m, x, n, st);
     backward(m, x, t, mask, n, loss, st);
     m->step += 1;
-    const float b1 = 0.9f, b2 = 0.999f;
-    const float c1 = 1.f - std::pow(b1, (float)m->step), c2 = 1.f - std::pow(b2, (float)m->step);
     const uint64_t np = m->nparams;
     const int blocks = (int)std::min<uint64_t>(1024, (np + 255) / 256);
     hipLaunchKernelGGL(adam_update, dim3(blocks), dim3(256), 0, st, np, m->params, m->grads, m->adam_m, m->adam_v, lr,
