@@ -329,6 +329,7 @@ struct bine_vcomm_s {
     uint32_t max_plans = kDefaultMaxPlans;
     uint64_t clock = 0;
     hipError_t scratch_err = hipSuccess;  // resolving the allocation-free entry point's workspace at creation
+    bool trees = false;  // compile lists of general trees: some call may run as AUTO
 };
 
 namespace {
@@ -365,7 +366,7 @@ int get_plan(bine_vcomm_t comm, const CollRequest& req, int dtype, std::shared_p
     for (int b = 0; b < kNumBufs; ++b)
         if ((uint64_t)prog.extent[b] >= (1ull << 32)) return fail(BINE_ERR_UNSUPPORTED, "per-rank buffer exceeds 2^32 elements");
     auto dp = std::make_shared<DevPlan>();
-    if (!compile_program(prog, true, &dp->cp, &err)) {
+    if (!compile_program(prog, true, comm->trees, &dp->cp, &err)) {
         if (req.in_place) err = "schedule cannot run in place (sendbuf == recvbuf): " + err;
         return fail(BINE_ERR_UNSUPPORTED, err);
     }
@@ -739,6 +740,7 @@ extern "C" int bine_vcomm_create(const bine_vcomm_config_t* cfg, bine_vcomm_t* o
     auto* c = new bine_vcomm_s();
     c->cfg = *cfg;
     c->t = t;
+    c->trees = cfg->exec == BINE_EXEC_AUTO;
     // set-up of bine_allreduce_noalloc: the device address of its workspace, once per device
     c->scratch_err = scratch_init(cfg->device);
     *out = c;
@@ -760,6 +762,8 @@ extern "C" int bine_vcomm_size(bine_vcomm_t comm, uint32_t* size) {
 
 extern "C" int bine_vcomm_set_exec(bine_vcomm_t comm, int32_t exec) {
     if (!comm || exec < 0 || exec > 2) return fail(BINE_ERR_ARG, "bad exec");
+    std::lock_guard<std::mutex> lock(comm->mu);
+    comm->trees = comm->trees || exec == BINE_EXEC_AUTO;
     comm->cfg.exec = exec;
     return BINE_OK;
 }
@@ -1047,7 +1051,7 @@ extern "C" int bine_plan_dump(const bine_vcomm_config_t* cfg, int32_t coll, int 
     CompiledPlan cp;
     std::string err;
     if (!build_program(t, *cfg, r, &prog, &err)) return fail(BINE_ERR_UNSUPPORTED, err);
-    if (!compile_program(prog, true, &cp, &err)) return fail(BINE_ERR_UNSUPPORTED, err);
+    if (!compile_program(prog, true, exec == kDumpTrees, &cp, &err)) return fail(BINE_ERR_UNSUPPORTED, err);
     if (exec == BINE_EXEC_FUSED && !cp.fused_ok) return fail(BINE_ERR_UNSUPPORTED, "schedule cannot be fused: " + cp.fused_why);
     const bool trees = exec == kDumpTrees;
     if (trees && !cp.trees) return fail(BINE_ERR_UNSUPPORTED, "no list of general trees: AUTO runs the steps");

@@ -1498,27 +1498,42 @@ struct PairHash {
     size_t operator()(const std::pair<int32_t, int64_t>& p) const { return mix64((uint64_t)p.first * 1000003ull ^ (uint64_t)p.second); }
 };
 
+// memo: values of (node, position) hashed before, or NULL
 uint64_t canon_hash(const Sym& s, int32_t node, int64_t pos, std::unordered_map<std::pair<int32_t, int64_t>, uint64_t, PairHash>* memo) {
-    auto k = std::make_pair(node, pos);
-    auto it = memo->find(k);
-    if (it != memo->end()) return it->second;
     const Node& n = s.nodes[node];
-    uint64_t h;
-    if (n.kind == 0) {
-        h = mix64(((uint64_t)n.buf << 56) ^ ((uint64_t)n.rank << 36) ^ (uint64_t)pos);
-    } else {
-        uint64_t ha = canon_hash(s, n.a.node, pos + n.a.delta, memo);
-        uint64_t hb = canon_hash(s, n.b.node, pos + n.b.delta, memo);
-        if (ha > hb) std::swap(ha, hb);
-        h = mix64(ha * 31 + mix64(hb ^ 0x5bd1e995ull));
+    if (n.kind == 0) return mix64(((uint64_t)n.buf << 56) ^ ((uint64_t)n.rank << 36) ^ (uint64_t)pos);
+    const auto k = std::make_pair(node, pos);
+    if (memo) {
+        auto it = memo->find(k);
+        if (it != memo->end()) return it->second;
     }
-    (*memo)[k] = h;
+    uint64_t ha = canon_hash(s, n.a.node, pos + n.a.delta, memo);
+    uint64_t hb = canon_hash(s, n.b.node, pos + n.b.delta, memo);
+    if (ha > hb) std::swap(ha, hb);
+    const uint64_t h = mix64(ha * 31 + mix64(hb ^ 0x5bd1e995ull));
+    if (memo) (*memo)[k] = h;
     return h;
 }
 
+// A distinct value of the outputs: node over `n` positions from pos.
+struct ValueKey {
+    int32_t node;
+    int64_t pos, n;
+    bool operator==(const ValueKey& o) const { return node == o.node && pos == o.pos && n == o.n; }
+};
+struct ValueHash {
+    size_t operator()(const ValueKey& k) const { return mix64(mix64((uint64_t)k.pos ^ ((uint64_t)k.node << 36)) ^ (uint64_t)k.n); }
+};
+struct Value {
+    int32_t node;
+    int64_t pos, n;
+    uint64_t outs;
+    uint32_t group;
+};
+
 }  // namespace
 
-bool compile_program(const Program& prog, bool want_fused, CompiledPlan* out, std::string* err) {
+bool compile_program(const Program& prog, bool want_fused, bool want_trees, CompiledPlan* out, std::string* err) {
     *out = CompiledPlan();
     out->P = prog.P;
     for (int b = 0; b < kNumBufs; ++b) {
@@ -1601,22 +1616,27 @@ bool compile_program(const Program& prog, bool want_fused, CompiledPlan* out, st
         out->step_groups.push_back(std::move(gs));
     }
 
-    // Final state: verify MPI semantics and group for the fused execution.
-    std::unordered_map<std::pair<int32_t, int64_t>, uint64_t, PairHash> memo;
-    std::unordered_map<uint64_t, size_t> group_of;  // (hash, len) -> group index
+    // Final state: verify MPI semantics and find the distinct values of the outputs for the fused execution.
     std::unordered_map<uint64_t, char> verified;  // (node, pos, expected source) already checked
-    bool fused_ok = want_fused;
+    const bool fuse = want_fused && !prog.outputs.empty();
     bool perfect = true;  // every tree is
-    bool trees_fit = prog.P < (1u << 24);  // the tree kernel's entries hold 24 bits of rank
+    bool trees_fit = want_trees && prog.P < (1u << 24);  // the tree kernel's entries hold 24 bits of rank
+    std::vector<Value> values;                                       // in order of appearance
+    std::unordered_map<ValueKey, uint32_t, ValueHash> value_of;
     std::string why;
     std::vector<Flat> fl;
+    std::vector<uint8_t> pops;
     std::vector<char> seen(prog.P);
+    // an input left in place: nothing to write
+    auto identity = [&](const Program::Output& o, const SymVal& v) {
+        const Node& nd = sym.nodes[v.node];
+        return nd.kind == 0 && nd.buf == o.buf && nd.rank == o.rank && v.delta == 0;
+    };
     for (const auto& o : prog.outputs) {
         const auto& m = sym.maps[(size_t)o.buf * prog.P + o.rank];
         for (auto it = m.begin(); it != m.end() && it->first < o.n; ++it) {
             const int64_t lo = it->first, hi = std::min(it->second.end, o.n);
             const SymVal v = it->second.v;
-            const Node& nd = sym.nodes[v.node];
             const int64_t pos = lo + v.delta;
             uint64_t vkey = 0;
             if (prog.expect.kind != Expect::NONE) {
@@ -1657,65 +1677,113 @@ bool compile_program(const Program& prog, bool want_fused, CompiledPlan* out, st
                     }
                 }
             }
-            if (!fused_ok) continue;
-            // identity output (an input left in place): nothing to write
-            if (nd.kind == 0 && nd.buf == o.buf && nd.rank == o.rank && pos == lo) continue;
-            if (!nd.perfect) {
-                perfect = false;
-                why = "a reduction tree is not perfect (non power-of-two schedule)";
+            if (!fuse || (!perfect && !trees_fit) || identity(o, v)) continue;
+            const auto at = value_of.try_emplace(ValueKey{v.node, pos, hi - lo}, (uint32_t)values.size());
+            if (at.second) {
+                const Node& nd = sym.nodes[v.node];
+                perfect = perfect && nd.perfect;
+                trees_fit = trees_fit && (nd.perfect ? nd.height < kMaxTreeStack : nd.need <= kMaxTreeStack);
+                values.push_back(Value{v.node, pos, hi - lo, 0, 0});
             }
-            uint64_t h = canon_hash(sym, v.node, pos, &memo);
-            uint64_t gk = mix64(h ^ mix64((uint64_t)(hi - lo)));
-            auto git = group_of.find(gk);
-            if (git == group_of.end()) {
-                Group g;
-                g.n = hi - lo;
-                fl.clear();
-                if (nd.perfect) {
-                    flatten(sym, v.node, pos, &fl);
-                    g.lg = (uint16_t)nd.height;
-                    trees_fit = trees_fit && nd.height < kMaxTreeStack;
-                } else {
-                    flatten_postfix(sym, v.node, pos, &fl, &g.pops);
-                    g.lg = (uint16_t)ceil_log2((uint32_t)fl.size());
-                    trees_fit = trees_fit && nd.need <= kMaxTreeStack;
-                }
-                for (const Flat& f : fl) g.leaves.push_back(make_entry(f.buf, f.rank, (uint32_t)f.pos));
-                g.outs.push_back(make_entry(o.buf, o.rank, (uint32_t)lo));
-                group_of[gk] = out->fused.size();
-                out->fused.push_back(std::move(g));
-            } else {
-                out->fused[git->second].outs.push_back(make_entry(o.buf, o.rank, (uint32_t)lo));
-            }
+            ++values[at.first->second].outs;
         }
     }
+    if (!perfect) why = "a reduction tree is not perfect (non power-of-two schedule)";
+    // Equal values (sums of the same tree, whichever way its children are named) form one group.  Whether a list of
+    // general trees fits and pays is told from the values alone, before any list is made: on a torus of 18x18x18 it
+    // does not, and making its 34 million leaves and outputs took 336 s and 17.9 GB where the steps alone take 104 s and 12.3.
+    bool listed = fuse && (perfect || trees_fit);
+    if (listed) {
+        std::unordered_map<std::pair<int32_t, int64_t>, uint64_t, PairHash> memo;
+        std::unordered_map<uint64_t, uint32_t> group_of;  // (hash, length) -> group
+        std::vector<uint32_t> first;                      // per group, its first value
+        std::vector<uint64_t> outs;                       // and number of outputs
+        for (size_t i = 0; i < values.size(); ++i) {
+            Value& x = values[i];
+            // the nodes of general trees are hashed anew for each value: remembering them all takes longer
+            const uint64_t h = canon_hash(sym, x.node, x.pos, sym.nodes[x.node].perfect ? &memo : nullptr);
+            const auto at = group_of.try_emplace(mix64(h ^ mix64((uint64_t)x.n)), (uint32_t)first.size());
+            if (at.second) {
+                first.push_back((uint32_t)i);
+                outs.push_back(0);
+            }
+            x.group = at.first->second;
+            outs[x.group] += x.outs;
+        }
+        if (!perfect) {
+            // general trees pay where they move no more than the schedule's steps do: an allreduce whose ranks each
+            // build a tree of their own would read every input once per rank
+            uint64_t moved = 0, stepped = 0;
+            for (size_t g = 0; g < first.size(); ++g)
+                moved += (uint64_t)values[first[g]].n * (sym.nodes[values[first[g]].node].nleaves + outs[g]);
+            for (const auto& gs : out->step_groups)
+                for (const Group& g : gs) stepped += (uint64_t)g.n * (g.leaves.size() + g.outs.size());
+            listed = moved <= stepped;
+        }
+        for (size_t i = 0; listed && i < first.size(); ++i) {
+            const Value& x = values[first[i]];
+            const Node& nd = sym.nodes[x.node];
+            Group g;
+            g.n = x.n;
+            fl.clear();
+            pops.clear();
+            if (nd.perfect) {
+                flatten(sym, x.node, x.pos, &fl);
+                g.lg = nd.height;
+                for (size_t k = 0; !perfect && k < fl.size(); ++k) pops.push_back((uint8_t)__builtin_ctzll(k + 1));
+            } else {
+                flatten_postfix(sym, x.node, x.pos, &fl, &pops);
+                g.lg = (uint16_t)ceil_log2((uint32_t)fl.size());
+            }
+            g.leaves.reserve(fl.size());
+            for (const Flat& f : fl) g.leaves.push_back(make_entry(f.buf, f.rank, (uint32_t)f.pos));
+            for (size_t k = 0; k < pops.size(); ++k) g.leaves[k].rb |= (uint32_t)pops[k] << kPopsShift;
+            g.outs.reserve(outs[i]);
+            out->fused.push_back(std::move(g));
+        }
+    }
+    if (listed)
+        for (const auto& o : prog.outputs) {
+            const auto& m = sym.maps[(size_t)o.buf * prog.P + o.rank];
+            for (auto it = m.begin(); it != m.end() && it->first < o.n; ++it) {
+                const int64_t lo = it->first, hi = std::min(it->second.end, o.n);
+                const SymVal v = it->second.v;
+                if (identity(o, v)) continue;
+                const Value& x = values[value_of.find(ValueKey{v.node, lo + v.delta, hi - lo})->second];
+                out->fused[x.group].outs.push_back(make_entry(o.buf, o.rank, (uint32_t)lo));
+            }
+        }
     // The fused launch reads the initial inputs while it writes the outputs: no output may overlap a leaf's input
     // range, except that of its own group at the same place (an in-place allreduce).  There a work item reads its
     // elements of every leaf before it writes any of them, and no other item touches them: 64 ranks, 1 MiB each, in
     // place 87.7 us in 12 launches, 21.0 in one.
     bool aliased = false;
-    if (fused_ok) {
+    if (listed) {
         struct Span {
             int64_t lo, hi;
             size_t group;
             int64_t reach;  // the furthest end of this span and those before it
         };
-        std::unordered_map<uint64_t, std::vector<Span>> in_ranges;
+        const uint32_t rank_bits = perfect ? 0x0FFFFFFFu : (1u << kPopsShift) - 1;
+        auto place = [&](const PoolEntry& e) { return (size_t)(e.rb >> 28) * prog.P + (e.rb & rank_bits); };
+        std::vector<char> written((size_t)kNumBufs * prog.P, 0);
+        for (const Group& g : out->fused)
+            for (const PoolEntry& o : g.outs) written[place(o)] = 1;
+        std::vector<std::vector<Span>> in_ranges(written.size());  // leaves in partitions that are written
         for (size_t gi = 0; gi < out->fused.size(); ++gi)
             for (const PoolEntry& l : out->fused[gi].leaves)
-                in_ranges[l.rb].push_back({l.off, l.off + out->fused[gi].n, gi, 0});
-        for (auto& kv : in_ranges) {
-            std::sort(kv.second.begin(), kv.second.end(), [](const Span& x, const Span& y) { return x.lo < y.lo; });
+                if (written[place(l)]) in_ranges[place(l)].push_back({l.off, l.off + out->fused[gi].n, gi, 0});
+        for (auto& v : in_ranges) {
+            auto by_start = [](const Span& x, const Span& y) { return x.lo < y.lo; };
+            if (!std::is_sorted(v.begin(), v.end(), by_start)) std::sort(v.begin(), v.end(), by_start);
             int64_t reach = 0;
-            for (Span& x : kv.second) x.reach = reach = std::max(reach, x.hi);
+            for (Span& x : v) x.reach = reach = std::max(reach, x.hi);
         }
         bool own = true;  // every overlap is an output's with its own group's leaf, and exact
         for (size_t gi = 0; gi < out->fused.size(); ++gi) {
             const Group& g = out->fused[gi];
             for (const PoolEntry& o : g.outs) {
-                auto it = in_ranges.find(o.rb);
-                if (it == in_ranges.end()) continue;
-                const std::vector<Span>& v = it->second;
+                const std::vector<Span>& v = in_ranges[place(o)];
                 const int64_t lo = o.off, hi = lo + g.n;
                 auto q = std::lower_bound(v.begin(), v.end(), hi, [](const Span& x, int64_t e) { return x.lo < e; });
                 while (q != v.begin() && std::prev(q)->reach > lo) {
@@ -1729,22 +1797,8 @@ bool compile_program(const Program& prog, bool want_fused, CompiledPlan* out, st
         if (aliased && perfect) why = "an output overlaps an input of the fused launch";
         out->auto_fused = !aliased || own;
     }
-    if (want_fused && prog.outputs.empty()) fused_ok = out->auto_fused = false;
-    if (!perfect) {
-        // general trees pay where they move no more than the schedule's steps do: allreduce L, whose ranks each build a
-        // tree of their own, would read every input once per rank
-        auto moved = [](const std::vector<Group>& gs) {
-            uint64_t n = 0;
-            for (const Group& g : gs) n += (uint64_t)g.n * (g.leaves.size() + g.outs.size());
-            return n;
-        };
-        uint64_t stepped = 0;
-        for (const auto& gs : out->step_groups) stepped += moved(gs);
-        out->auto_fused = out->auto_fused && trees_fit && moved(out->fused) <= stepped;
-        out->trees = out->auto_fused;
-    }
-    fused_ok = fused_ok && perfect && !aliased;
-    out->fused_ok = fused_ok;
+    out->trees = out->auto_fused && !perfect;
+    out->fused_ok = listed && perfect && !aliased;
     out->aliased = aliased && out->auto_fused;
     out->fused_why = why;
     if (!out->auto_fused) out->fused.clear();
@@ -2264,8 +2318,7 @@ void emit_cut(const std::vector<TreeNode>& t, const std::vector<char>& open, int
     ++c->pops.back();
 }
 
-// additions after leaf k of a balanced tree
-uint8_t balanced_pops(size_t k) { return (uint8_t)__builtin_ctzll(k + 1); }
+uint32_t pops_after(const PoolEntry& leaf) { return (leaf.rb >> kPopsShift) & 15u; }
 
 // stack_need: raised to what the join of the parts needs
 Cut cut_tree(const Group& g, uint32_t most, int* stack_need) {
@@ -2274,7 +2327,7 @@ Cut cut_tree(const Group& g, uint32_t most, int* stack_need) {
     for (size_t k = 0; k < g.leaves.size(); ++k) {
         t.push_back({-1, -1, 1});
         stack.push_back((int32_t)t.size() - 1);
-        for (int p = g.pops.empty() ? balanced_pops(k) : g.pops[k]; p > 0; --p) {
+        for (uint32_t p = pops_after(g.leaves[k]); p > 0; --p) {
             const int32_t b = stack.back();
             stack.pop_back();
             t.push_back({stack.back(), b, t[stack.back()].leaves + t[b].leaves});
@@ -2329,14 +2382,16 @@ void lower_trees(const std::vector<Group>& gs, int vec, uint32_t bucket, size_t 
         for (size_t i = 0; i < c.count.size(); ++i) out->pool.push_back(PoolEntry{c.count[i], c.pops[i]});
         size_t k = 0;
         for (uint32_t n : c.count) {
+            PoolEntry leaf{};
             uint32_t depth = 0;  // a subtree's last leaf is followed by its own additions only, not its parents'
             for (uint32_t j = 0; j < n; ++j, ++k) {
-                const uint32_t pops = std::min<uint32_t>(g.pops.empty() ? balanced_pops(k) : g.pops[k], depth);
-                out->pool.push_back(PoolEntry{g.leaves[k].rb | (pops << 24), g.leaves[k].off});
+                const uint32_t pops = std::min(pops_after(g.leaves[k]), depth);
+                leaf = PoolEntry{g.leaves[k].rb & ~(15u << kPopsShift), g.leaves[k].off};
+                out->pool.push_back(PoolEntry{leaf.rb | (pops << kPopsShift), leaf.off});
                 out->tree_stack = std::max<int>(out->tree_stack, (int)depth + 1);
                 depth += 1 - pops;
             }
-            for (uint32_t j = n; j % 8 != 0; ++j) out->pool.push_back(g.leaves[k - 1]);
+            for (uint32_t j = n; j % 8 != 0; ++j) out->pool.push_back(leaf);
         }
         const uint32_t out_off = (uint32_t)out->pool.size();
         out->pool.insert(out->pool.end(), g.outs.begin(), g.outs.end());

@@ -75,11 +75,13 @@ struct Group {
     std::vector<PoolEntry> outs;
     int64_t n = 0;
     uint16_t lg = 0;
-    // not empty: a general tree, evaluated on a stack; pops[k] additions follow leaf k (lg: the rounded-up log2)
-    std::vector<uint8_t> pops;
 };
 
-constexpr int kMaxTreeStack = 12;  // values that the tree kernel's stack holds
+// Lists of general trees (CompiledPlan::trees): trees are evaluated on a stack, and a leaf's rb holds the rank below
+// bit kPopsShift and in the four bits from there on the number of additions that follow the leaf; lg is the rounded-up
+// log2 of the leaves.
+constexpr int kPopsShift = 24;
+constexpr int kMaxTreeStack = 12;  // values that the tree kernel's stack holds, so at most 11 additions follow a leaf
 
 struct CompiledPlan {
     uint32_t P = 0;
@@ -108,8 +110,8 @@ struct CollRequest {
 bool build_program(const Torus& t, const bine_vcomm_config_t& cfg, const CollRequest& req, Program* out,
                    std::string* err);
 
-// Run the program symbolically: race check, semantic check, fused grouping.
-bool compile_program(const Program& prog, bool want_fused, CompiledPlan* out, std::string* err);
+// Run the program symbolically: race check, semantic check, fused grouping (want_trees: also where its trees are general).
+bool compile_program(const Program& prog, bool want_fused, bool want_trees, CompiledPlan* out, std::string* err);
 
 // Work items for the kernel.
 struct Lowered {

@@ -126,7 +126,9 @@ int bine_vcomm_create(const bine_vcomm_config_t* cfg, bine_vcomm_t* out);
 int bine_vcomm_destroy(bine_vcomm_t comm);
 /* MPI_Comm_size on the virtual communicator. */
 int bine_vcomm_size(bine_vcomm_t comm, uint32_t* size);
-/* Replace the execution mode of an existing vcomm (cached schedules are kept). */
+/* Replace the execution mode of an existing vcomm (cached schedules are kept: on
+ * a torus that is no power of two, those compiled before the vcomm was ever AUTO
+ * run per step under AUTO as well). */
 int bine_vcomm_set_exec(bine_vcomm_t comm, int32_t exec);
 /* Plan cache (no counterpart in the reference, whose bitmap and tree caches are never evicted,
  * lib/libbine_common.cc:1671-1675, lib/libbine_coll.cc:334-389).  At most max_plans schedules stay
