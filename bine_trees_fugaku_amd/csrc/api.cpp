@@ -69,14 +69,13 @@ size_t dtsize(int dt) {
 
 struct DevArrays {
     Lowered low;
-    GredItem* items = nullptr;
+    GredItem* items = nullptr;  // the allocation that holds the pool as well
     PoolEntry* pool = nullptr;
     int max_lg = 0;
     int64_t tile_elems = 0;
     LaunchShape shape;
     void release() {
         if (items) (void)hipFree(items);
-        if (pool) (void)hipFree(pool);
         items = nullptr;
         pool = nullptr;
         low = Lowered();
@@ -88,7 +87,6 @@ struct Retired {
     std::vector<void*> ptrs;
     void keep(DevArrays* d) {
         if (d->items) ptrs.push_back(d->items);
-        if (d->pool) ptrs.push_back(d->pool);
         d->items = nullptr;
         d->pool = nullptr;
     }
@@ -97,7 +95,8 @@ struct Retired {
     }
 };
 
-// Copy a lowered work list to the device.  The new arrays replace d's only once every allocation and copy
+// Copy a lowered work list to the device, items and pool in one allocation and, where small, one copy: a schedule has
+// up to two lists, and each call of the runtime costs a first call of a new size 30 us or so.  The new arrays replace d's only once every allocation and copy
 // has succeeded; on failure d is left as it was.  The old arrays are freed, or kept in `retire` when a
 // captured graph may name them.
 int install(Lowered&& low, int max_lg, int64_t tile_elems, const LaunchShape& sh, DevArrays* d, Retired* retire) {
@@ -107,15 +106,19 @@ int install(Lowered&& low, int max_lg, int64_t tile_elems, const LaunchShape& sh
     n.tile_elems = tile_elems;
     n.shape = sh;
     hipError_t e = hipSuccess;
-    if (!n.low.items.empty()) {
-        e = hipMalloc(&n.items, n.low.items.size() * sizeof(GredItem));
-        if (e == hipSuccess)
-            e = hipMemcpy(n.items, n.low.items.data(), n.low.items.size() * sizeof(GredItem), hipMemcpyHostToDevice);
-    }
-    if (e == hipSuccess && !n.low.pool.empty()) {
-        e = hipMalloc(&n.pool, n.low.pool.size() * sizeof(PoolEntry));
-        if (e == hipSuccess)
-            e = hipMemcpy(n.pool, n.low.pool.data(), n.low.pool.size() * sizeof(PoolEntry), hipMemcpyHostToDevice);
+    const size_t ib = n.low.items.size() * sizeof(GredItem), pb = n.low.pool.size() * sizeof(PoolEntry);
+    if (ib) {
+        e = hipMalloc(&n.items, ib + pb);
+        if (e == hipSuccess) n.pool = reinterpret_cast<PoolEntry*>(n.items + n.low.items.size());
+        if (e == hipSuccess && ib + pb <= (1u << 20)) {
+            std::vector<char> both(ib + pb);
+            std::memcpy(both.data(), n.low.items.data(), ib);
+            if (pb) std::memcpy(both.data() + ib, n.low.pool.data(), pb);
+            e = hipMemcpy(n.items, both.data(), ib + pb, hipMemcpyHostToDevice);
+        } else if (e == hipSuccess) {
+            e = hipMemcpy(n.items, n.low.items.data(), ib, hipMemcpyHostToDevice);
+            if (e == hipSuccess && pb) e = hipMemcpy(n.pool, n.low.pool.data(), pb, hipMemcpyHostToDevice);
+        }
     }
     if (e != hipSuccess) {
         (void)hipGetLastError();
@@ -374,16 +377,18 @@ int get_plan(bine_vcomm_t comm, const CollRequest& req, int dtype, std::shared_p
     dp->ds = ds;
     int rc = upload(dp->cp.step_groups, ds, default_shape(), Ends::EXACT, false, &dp->step);
     if (rc) return rc;
-    if (dp->cp.auto_fused && max_lg_of(std::vector<std::vector<Group>>(1, dp->cp.fused)) > 14) {
+    std::vector<std::vector<Group>> one(1);  // as one launch
+    one[0].swap(dp->cp.fused);
+    if (dp->cp.auto_fused && max_lg_of(one) > 14) {
         dp->cp.fused_ok = dp->cp.auto_fused = false;  // the kernel's register stack holds trees of up to 2^14 leaves
-        dp->cp.fused.clear();
+        one[0].clear();
         dp->cp.fused_why = "reduction tree wider than 2^14 leaves";
     }
     if (dp->cp.auto_fused) {
-        std::vector<std::vector<Group>> one(1, dp->cp.fused);
         rc = upload(one, ds, initial_shape(one, ds, (uint64_t)prog.extent[BUF_RECV] * ds % 16 == 0, true), dp->fused_ends(), dp->cp.trees, &dp->fused);
         if (rc) return rc;
     }
+    one[0].swap(dp->cp.fused);
     // temporaries are allocated only when some step touches them
     bool used[kNumBufs] = {false, false, false, false};
     for (const auto& launch : dp->cp.step_groups)

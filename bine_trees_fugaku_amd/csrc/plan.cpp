@@ -2323,6 +2323,7 @@ uint32_t pops_after(const PoolEntry& leaf) { return (leaf.rb >> kPopsShift) & 15
 // stack_need: raised to what the join of the parts needs
 Cut cut_tree(const Group& g, uint32_t most, int* stack_need) {
     std::vector<TreeNode> t;
+    t.reserve(2 * g.leaves.size());
     std::vector<int32_t> stack;
     for (size_t k = 0; k < g.leaves.size(); ++k) {
         t.push_back({-1, -1, 1});
@@ -2374,6 +2375,9 @@ void lower_trees(const std::vector<Group>& gs, int vec, uint32_t bucket, size_t 
     uint32_t waves = std::min(8u, pow2_at_least((leaves + 12) / 13));
     if (workgroups < 1024) waves = std::max(waves, std::min(4u, pow2_at_least((leaves + 2) / 3)));
     out->tree_waves = (int)waves;
+    size_t entries = 0;
+    for (const Group& g : gs) entries += 2 * waves + g.leaves.size() + 7 * waves + g.outs.size();
+    out->pool.reserve(entries);
     for (size_t gi = 0; gi < gs.size(); ++gi) {
         const Group& g = gs[gi];
         if (g.n <= 0) continue;
