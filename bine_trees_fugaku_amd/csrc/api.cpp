@@ -981,6 +981,7 @@ extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* s
     const Ends ends = exec == BINE_EXEC_FUSED ? dp->fused_ends() : Ends::EXACT;
     const bool trees = exec == BINE_EXEC_FUSED && dp->cp.trees;
     if (coll == BINE_COLL_BCAST) sendbuf = nullptr;  // as in bine_bcast
+    if (trees) return run_coll(comm, r, datatype, sendbuf, recvbuf, stream, exec);  // no launch shape changes such a list
     DevArrays& d = exec == BINE_EXEC_FUSED ? dp->fused : dp->step;
     const std::vector<std::vector<Group>> one(1, dp->cp.fused);
     const std::vector<std::vector<Group>>& groups = exec == BINE_EXEC_FUSED ? one : dp->cp.step_groups;
@@ -1001,7 +1002,7 @@ extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* s
     auto trial = [&](const LaunchShape& c) {
         // the arrays in place before the call may be named by captured graphs: they are kept, not freed;
         // the candidates' own arrays never leave this loop
-        if ((rc = upload(groups, dp->ds, c, ends, trees, &d, first ? &dp->retired : nullptr))) return;
+        if ((rc = upload(groups, dp->ds, c, ends, false, &d, first ? &dp->retired : nullptr))) return;
         first = false;
         if ((rc = run_coll(comm, r, datatype, sendbuf, recvbuf, stream, exec))) return;
         if (hipEventRecord(e0, st) != hipSuccess) {
@@ -1024,7 +1025,7 @@ extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* s
         trial(c);
         if (rc) break;
     }
-    if (!rc && !trees && has_multi_output_reduction(groups))
+    if (!rc && has_multi_output_reduction(groups))
         for (const LaunchShape& c : two_phase_trials(timed)) {
             trial(c);
             if (rc) break;
@@ -1032,7 +1033,7 @@ extern "C" int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* s
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc;
-    return upload(groups, dp->ds, bestc, ends, trees, &d);
+    return upload(groups, dp->ds, bestc, ends, false, &d);
 }
 
 // bine_plan_dump: the list of general trees that AUTO runs where FUSED is refused
@@ -1562,7 +1563,11 @@ extern "C" int bine_batch_autotune(bine_batch_t b, void* stream, int iters) {
     HIPCHK(hipSetDevice(b->comm->cfg.device));
     hipStream_t st = (hipStream_t)stream;
     const std::vector<LaunchShape> cands = tuning_candidates(device_cus(b->comm->cfg.device));
-    // every element type's list is timed alone at every candidate and keeps its fastest shape
+    // every element type's list is timed alone at every candidate and keeps its fastest shape; no shape changes a list
+    // of general trees, which keeps its own
+    std::vector<size_t> tuned;
+    for (size_t i = 0; i < b->lists.size(); ++i)
+        if (!b->lists[i].trees) tuned.push_back(i);
     const size_t nl = b->lists.size();
     std::vector<float> best(nl, 1e30f);
     std::vector<LaunchShape> pick(nl, default_shape());
@@ -1593,14 +1598,14 @@ extern "C" int bine_batch_autotune(bine_batch_t b, void* stream, int iters) {
         return BINE_OK;
     };
     for (const LaunchShape& c : cands)
-        for (size_t i = 0; i < nl; ++i)
+        for (size_t i : tuned)
             if (int rc = trial(i, c)) return rc;
-    for (size_t i = 0; i < nl; ++i)
-        if (!b->lists[i].trees && has_multi_output_reduction(b->lists[i].groups))
+    for (size_t i : tuned)
+        if (has_multi_output_reduction(b->lists[i].groups))
             for (const LaunchShape& c : two_phase_trials(timed[i]))
                 if (int rc = trial(i, c)) return rc;
-    size_t dominant = 0;
-    for (size_t i = 0; i < nl; ++i) {
+    size_t dominant = tuned.empty() ? 0 : tuned[0];
+    for (size_t i : tuned) {
         auto& l = b->lists[i];
         const bool relower = !same_lowering(pick[i], l.shape);
         l.shape = pick[i];
@@ -1610,7 +1615,7 @@ extern "C" int bine_batch_autotune(bine_batch_t b, void* stream, int iters) {
         }
         if (best[i] > best[dominant]) dominant = i;
     }
-    if (nl) b->shape = pick[dominant];
+    if (!tuned.empty()) b->shape = pick[dominant];
     return BINE_OK;
 }
 
