@@ -369,7 +369,7 @@ int get_plan(bine_vcomm_t comm, const CollRequest& req, int dtype, std::shared_p
     for (int b = 0; b < kNumBufs; ++b)
         if ((uint64_t)prog.extent[b] >= (1ull << 32)) return fail(BINE_ERR_UNSUPPORTED, "per-rank buffer exceeds 2^32 elements");
     auto dp = std::make_shared<DevPlan>();
-    if (!compile_program(prog, true, comm->trees, &dp->cp, &err)) {
+    if (!compile_program(prog, true, comm->trees ? ds : 0, &dp->cp, &err)) {
         if (req.in_place) err = "schedule cannot run in place (sendbuf == recvbuf): " + err;
         return fail(BINE_ERR_UNSUPPORTED, err);
     }
@@ -1057,7 +1057,7 @@ extern "C" int bine_plan_dump(const bine_vcomm_config_t* cfg, int32_t coll, int 
     CompiledPlan cp;
     std::string err;
     if (!build_program(t, *cfg, r, &prog, &err)) return fail(BINE_ERR_UNSUPPORTED, err);
-    if (!compile_program(prog, true, exec == kDumpTrees, &cp, &err)) return fail(BINE_ERR_UNSUPPORTED, err);
+    if (!compile_program(prog, true, exec == kDumpTrees ? ds : 0, &cp, &err)) return fail(BINE_ERR_UNSUPPORTED, err);
     if (exec == BINE_EXEC_FUSED && !cp.fused_ok) return fail(BINE_ERR_UNSUPPORTED, "schedule cannot be fused: " + cp.fused_why);
     const bool trees = exec == kDumpTrees;
     if (trees && !cp.trees) return fail(BINE_ERR_UNSUPPORTED, "no list of general trees: AUTO runs the steps");

@@ -33,6 +33,13 @@ constexpr uint32_t kMaxRun = 2;
 // entries at leaf_off: the first copy's source and destination, then their steps along the first axis, then along the
 // second (ranks and offsets add up, modulo 2^32).
 
+// Lists of general trees (CompiledPlan::trees): trees are evaluated on a stack, and a leaf's rb holds the rank below
+// bit kPopsShift and in the four bits from there on the number of additions that follow the leaf; a group's lg is the
+// rounded-up log2 of its leaves.
+constexpr int kPopsShift = 24;
+constexpr int kMaxTreeStack = 12;  // values that the tree kernel's stack holds, so at most 11 additions follow a leaf
+constexpr int kShallowStack = 6;   // and those that its smaller instantiation's holds
+
 // Items of the tree kernel (gtree.hip): lg is the number of subtrees, at most one per wave.  The pool holds one entry
 // per subtree at leaf_off (rb: its number of leaves; off: the additions that follow when the subtree sums are joined on
 // a stack), then the subtrees' leaves, each padded to whole groups of eight; a leaf's rb holds the rank in bits 0..23

@@ -181,8 +181,8 @@ hipError_t launch_d(const GredItem* items, uint32_t n, const PoolEntry* pool, co
 template <typename T>
 hipError_t launch_t(const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab, const BufTable* tabs,
                     bool batch, int waves, int stack, hipStream_t st) {
-    return stack <= 6 ? launch_d<T, 5>(items, n, pool, tab, tabs, batch, waves, st)
-                      : launch_d<T, 11>(items, n, pool, tab, tabs, batch, waves, st);
+    return stack <= kShallowStack ? launch_d<T, kShallowStack - 1>(items, n, pool, tab, tabs, batch, waves, st)
+                                  : launch_d<T, kMaxTreeStack - 1>(items, n, pool, tab, tabs, batch, waves, st);
 }
 
 }  // namespace
@@ -191,7 +191,7 @@ hipError_t launch_t(const GredItem* items, uint32_t n, const PoolEntry* pool, co
 hipError_t launch_gtree(int dtype, const GredItem* items, uint32_t n, const PoolEntry* pool, const BufTable& tab,
                         const BufTable* tabs, bool batch, int waves, int stack, hipStream_t st) {
     if (n == 0) return hipSuccess;
-    if (waves < 1 || waves > 8 || stack > 12) return hipErrorInvalidValue;
+    if (waves < 1 || waves > 8 || stack > kMaxTreeStack) return hipErrorInvalidValue;
     switch (dtype) {
     case 0: return launch_t<int32_t>(items, n, pool, tab, tabs, batch, waves, stack, st);
     case 1: return launch_t<int64_t>(items, n, pool, tab, tabs, batch, waves, stack, st);

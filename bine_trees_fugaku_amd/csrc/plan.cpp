@@ -1531,9 +1531,30 @@ struct Value {
     uint32_t group;
 };
 
+// The most that a wave of the tree kernel takes of a list whose trees are cut for eight waves (as cut_tree does).
+struct WavePart {
+    uint32_t leaves = 0;
+    int need = 0;
+};
+void widest_part(const Sym& s, int32_t root, WavePart* w) {
+    auto leaves = [&](int32_t n) { return s.nodes[n].nleaves; };
+    std::vector<int32_t> parts(1, root);
+    while (parts.size() < 8) {
+        auto most = std::max_element(parts.begin(), parts.end(), [&](int32_t a, int32_t b) { return leaves(a) < leaves(b); });
+        if (leaves(*most) < 2) break;
+        const Node& n = s.nodes[*most];
+        *most = n.a.node;
+        parts.push_back(n.b.node);
+    }
+    for (int32_t n : parts) {
+        w->leaves = std::max(w->leaves, leaves(n));
+        w->need = std::max<int>(w->need, s.nodes[n].need);
+    }
+}
+
 }  // namespace
 
-bool compile_program(const Program& prog, bool want_fused, bool want_trees, CompiledPlan* out, std::string* err) {
+bool compile_program(const Program& prog, bool want_fused, size_t tree_bytes, CompiledPlan* out, std::string* err) {
     *out = CompiledPlan();
     out->P = prog.P;
     for (int b = 0; b < kNumBufs; ++b) {
@@ -1620,7 +1641,7 @@ bool compile_program(const Program& prog, bool want_fused, bool want_trees, Comp
     std::unordered_map<uint64_t, char> verified;  // (node, pos, expected source) already checked
     const bool fuse = want_fused && !prog.outputs.empty();
     bool perfect = true;  // every tree is
-    bool trees_fit = want_trees && prog.P < (1u << 24);  // the tree kernel's entries hold 24 bits of rank
+    bool trees_fit = tree_bytes > 0 && prog.P < (1u << 24);  // the tree kernel's entries hold 24 bits of rank
     std::vector<Value> values;                                       // in order of appearance
     std::unordered_map<ValueKey, uint32_t, ValueHash> value_of;
     std::string why;
@@ -1719,6 +1740,23 @@ bool compile_program(const Program& prog, bool want_fused, bool want_trees, Comp
             for (const auto& gs : out->step_groups)
                 for (const Group& g : gs) stepped += (uint64_t)g.n * (g.leaves.size() + g.outs.size());
             listed = moved <= stepped;
+            WavePart part;
+            for (size_t g = 0; listed && g < first.size(); ++g) widest_part(sym, values[first[g]].node, &part);
+            if (listed && part.need > kShallowStack) {
+                // Beyond that depth the kernel takes 0.66 us for each leaf of a wave, its code no longer fitting the
+                // instruction cache, or what 4.5 TB/s move; steps take 3.2 us a launch, 6 TB/s and 1.1 ns an operation.
+                // A fifth to spare: without it 4x10x10 of 1000 ran 41 / 43 and 20x18 of 20000 fp64 204 / 221.
+                // Allreduce L, fp32, steps / one launch, microseconds: 20x20 of 1000 elements 41 / 51, of 8192 81 / 63,
+                // of 65536 322 / 393; 12x12x6 of 1000 48 / 95, of 8192 106 / 102, of 65536 469 / 257; 10x10x10 of 1000
+                // 57 / 100, of 8192 142 / 105, of 65536 852 / 497; B on a ring of 400 of 403 262 / 83, of 262144
+                // 996 / 260, on 10x10x10 of 1003 921 / 358.  Shallower lists gained at every size measured (1.5 times
+                // and more: L on 18x18 of 1000 41 / 21, of 65536 286 / 177).
+                double operations = 0;
+                for (const auto& gs : out->step_groups) operations += (double)gs.size();
+                const double steps_us = 3.2 * (double)out->step_groups.size() + (double)(stepped * tree_bytes) / 6e6 +
+                                        1.1e-3 * operations;
+                listed = 1.2 * std::max(0.66 * part.leaves, (double)(moved * tree_bytes) / 4.5e6) <= steps_us;
+            }
         }
         for (size_t i = 0; listed && i < first.size(); ++i) {
             const Value& x = values[first[i]];

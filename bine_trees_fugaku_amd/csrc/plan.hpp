@@ -77,12 +77,6 @@ struct Group {
     uint16_t lg = 0;
 };
 
-// Lists of general trees (CompiledPlan::trees): trees are evaluated on a stack, and a leaf's rb holds the rank below
-// bit kPopsShift and in the four bits from there on the number of additions that follow the leaf; lg is the rounded-up
-// log2 of the leaves.
-constexpr int kPopsShift = 24;
-constexpr int kMaxTreeStack = 12;  // values that the tree kernel's stack holds, so at most 11 additions follow a leaf
-
 struct CompiledPlan {
     uint32_t P = 0;
     int64_t extent[kNumBufs] = {0, 0, 0, 0};
@@ -110,8 +104,9 @@ struct CollRequest {
 bool build_program(const Torus& t, const bine_vcomm_config_t& cfg, const CollRequest& req, Program* out,
                    std::string* err);
 
-// Run the program symbolically: race check, semantic check, fused grouping (want_trees: also where its trees are general).
-bool compile_program(const Program& prog, bool want_fused, bool want_trees, CompiledPlan* out, std::string* err);
+// Run the program symbolically: race check, semantic check, fused grouping (tree_bytes, the size of an element, or 0: also
+// where its trees are general).
+bool compile_program(const Program& prog, bool want_fused, size_t tree_bytes, CompiledPlan* out, std::string* err);
 
 // Work items for the kernel.
 struct Lowered {
