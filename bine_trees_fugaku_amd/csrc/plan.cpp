@@ -1922,10 +1922,26 @@ uint32_t pow2_at_least(uint64_t x) {
 // ones that are no whole number of vectors, which leave items of single elements.  GPU time in microseconds, runs /
 // packs, fp32: alltoall on 512 ranks of 16 elements a pair 241 / 7.8, of 25 566 / 11.3, of 256 267 / 108, of 512 302 /
 // 194, of 1024 397 / 389; on 64 ranks of 512 6.6 / 5.1, of 1024 7.4 / 7.7; scatter to 512 ranks of 1000 3.0 / 2.7, of
-// 4099 7.5 / 5.7, but of 16384 13.1 / 15.2 and to 8 ranks of 65537 5.4 / 28: a copy stays within one workgroup.
+// 4099 8.3 / 6.3, of 5119 9.4 / 6.8, to 8 ranks of 5119 5.6 / 4.1, but to 512 of 16384 13.1 / 15.2 and to 8 of 65537 5.4 /
+// 28: a copy stays within one workgroup.
+constexpr uint64_t kShortCopy = 2048;  // bytes
 bool packs(const Group& g, int vec, size_t dtsize) {
     const uint64_t bytes = (uint64_t)g.n * dtsize;
-    return is_copy(g) && bytes <= (g.n % vec == 0 ? 2048u : 20480u);
+    return is_copy(g) && bytes <= (g.n % vec == 0 ? kShortCopy : 20480u);
+}
+
+// The longest copies of a launch, in bytes, that go there.  Beside other items the pack kernel is a launch more, about
+// 3 us, which only some thousands of short copies are worth (a workgroup of the run kernel holds two of them and takes
+// 1.8 ns of the chip): per-step allreduces, all packable copies / this, microseconds: 6x6 of 131072 fp32 109 / 88, 4x4x4
+// of 272203 158 / 147.
+uint64_t packed_bytes(const std::vector<Group>& gs, int vec, size_t dtsize) {
+    size_t others = 0, shorts = 0;
+    for (const Group& g : gs) {
+        if (g.n <= 0) continue;
+        others += !packs(g, vec, dtsize);
+        shorts += packs(g, vec, dtsize) && (uint64_t)g.n * dtsize <= kShortCopy;
+    }
+    return others == 0 ? UINT64_MAX : shorts >= 4096 ? kShortCopy : 0;
 }
 
 // Cut a grid into items of about `tile` bytes, about as long along either axis where it has two.
@@ -1989,13 +2005,14 @@ void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shall
         auto advance = [](const PoolEntry& a, const PoolEntry& st, uint32_t k) {
             return PoolEntry{a.rb + st.rb * k, a.off + st.off * k};
         };
-        std::vector<size_t> packed;
+        const uint64_t packed = pack ? packed_bytes(gs, vec, dtsize) : 0;
+        std::vector<size_t> to_pack;
         for (size_t gi = 0; gi < gs.size(); ++gi) {
             const Group& g = gs[gi];
             const uint32_t gb = gbk ? (*gbk)[gi] : bucket;
             if (g.n <= 0) continue;
-            if (pack && packs(g, vec, dtsize)) {
-                packed.push_back(gi);
+            if ((uint64_t)g.n * dtsize <= packed && packs(g, vec, dtsize)) {
+                to_pack.push_back(gi);
                 continue;
             }
             if (single_copy(g) && run_item >= 0 && run_len < kMaxRun && out->items[run_item].n == (uint32_t)g.n &&
@@ -2168,9 +2185,9 @@ void lower_groups(const std::vector<std::vector<Group>>& launches, int64_t shall
                     out->unaligned_outs |= ((int64_t)out->pool[it.out_off + o].off + it.delta) % vec != 0;
             }
         }
-        if (!packed.empty()) {
+        if (!to_pack.empty()) {
             std::vector<CopyGrid> grids;
-            find_grids(gs, packed, gbk, bucket, &grids);
+            find_grids(gs, to_pack, gbk, bucket, &grids);
             uint64_t moved = 0;
             for (const CopyGrid& g : grids) moved += (uint64_t)g.n * dtsize * g.k1 * g.k2;
             // 16 KiB a workgroup (four 16-byte units per lane), less where that would give fewer than 2048 of them
