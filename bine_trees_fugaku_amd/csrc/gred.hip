@@ -238,11 +238,11 @@ __global__ void __launch_bounds__(512) gred_kernel(const GredItem* __restrict__ 
         const BINE_CONST PoolEntry* outs = cptr(pool + it.out_off);
         const uint32_t lg = it.lg;
         // byte offset of vector v inside the tile (see GredItem::pad)
-        int32_t pad = (int32_t)it.pad, last = (int32_t)it.n - VE;
+        int32_t pad = (int32_t)(it.pad * sizeof(T)), last = (int32_t)((it.n - VE) * sizeof(T));
         asm("" : "+v"(pad), "+v"(last));
         auto at = [&](uint32_t v) __attribute__((always_inline)) {
-            const int32_t e = (int32_t)(v * VE) - pad;
-            return (uint32_t)((e < 0 ? 0 : e > last ? last : e) * (int32_t)sizeof(T));
+            const int32_t b = (int32_t)(v * 16) - pad;
+            return (uint32_t)min(max(b, 0), last);
         };
         auto addp = [](const Pack<T, VPT>& a, const Pack<T, VPT>& b) __attribute__((always_inline)) {
             Pack<T, VPT> r;
