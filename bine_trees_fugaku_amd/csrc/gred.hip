@@ -241,6 +241,7 @@ __global__ void __launch_bounds__(512) gred_kernel(const GredItem* __restrict__ 
         int32_t pad = (int32_t)(it.pad * sizeof(T)), last = (int32_t)((it.n - VE) * sizeof(T));
         asm("" : "+v"(pad), "+v"(last));
         auto at = [&](uint32_t v) __attribute__((always_inline)) {
+            if (REALIGN) return v * 16u;  // its lists hold whole vectors
             const int32_t b = (int32_t)(v * 16) - pad;
             return (uint32_t)min(max(b, 0), last);
         };
