@@ -2258,13 +2258,21 @@ constexpr uint32_t kNarrowThreads = 1024;
 //     buffers rotating; 64 ranks, allreduce of 65536 (256) 9.7 / 8.4, of 131072 (512) 14.0 / 14.8; bcast to 512 ranks of
 //     131072 (128) 84 / 44, of 262146 (257, realigned stores) 156 / 167;
 //   eight leaves or outputs need no spreading: 8 ranks, allreduce of 65536 (64) 4.65 / 4.58, of 131072 (128) 4.9 / 5.1;
-//   short blocks on 512 ranks: allreduce of 65536 (32 vectors a block) 92 / 53, of 262144 (128) 288 / 259; allgather of
-//     256 (64) 101 / 59, of 512 (128) 141 / 140; reduce_scatter of 128 (32) 36.9 / 31.0, of 192 (48) 37.5 / 45.1.
+//   short blocks: allgather on 512 ranks of 256 (64) 101 / 59, of 512 (128) 141 / 140; reduce_scatter of 128 (32) 36.9 /
+//     31.0, of 192 (48) 37.5 / 45.1; allreduce where the units of a block times its leaves are few, since more leaves leave
+//     fewer lanes for units (buffers in cache, from memory): 128 ranks of 57440 (113 units) 21.0, 25.4 / 15.8, 19.9; 256 of
+//     41152 (41) 35.8, 47.4 / 26.7, 34.8, of 81920 (80) 37.5, 56.6 / 51.8, 50.3, of 98496 (97) 39.7, 63.8 / 52.7, 71.8; 512
+//     of 65536 (32) 98, 104 / 61, 61, of 98688 (49) 128, 128 / 147, 149; 1024 of 66304 (17) 294, 294 / 214, 215, of 99072
+//     (25) 318, 316 / 323, 325; and up to 128 units where blocks are whole lines and the list is beyond the cache: 512 of
+//     98304 (48) 127, 125 / 95, 94, of 262144 (128) 292, 283 / 224, 223, 1024 of 131072 (32) 344, 344 / 253, 255.
 bool narrow_pays(const std::vector<std::vector<Group>>& launches, int vec) {
     if (launches.size() != 1) return false;
     size_t fan = 0;
     uint64_t workgroups = 0, units = 0, short_units = 0;
     bool spreads = false;  // reductions with several outputs
+    uint64_t bytes = 0;
+    for (const Group& g : launches[0]) bytes += (uint64_t)g.n * (g.leaves.size() + g.outs.size()) * (uint64_t)(16 / vec);
+    const bool cached = bytes <= (300ull << 20);
     for (const Group& g : launches[0]) {
         fan = std::max({fan, g.leaves.size(), g.outs.size()});
         spreads = spreads || (g.lg > 0 && g.outs.size() > 1);
@@ -2272,7 +2280,10 @@ bool narrow_pays(const std::vector<std::vector<Group>>& launches, int vec) {
         const uint64_t tile = g.lg >= 5 ? 64 : 256;
         workgroups += (u + tile - 1) / tile;
         units += u * ends;
-        if (u <= (g.lg > 0 && g.outs.size() == 1 ? 32u : 128u)) short_units += u * ends;
+        uint64_t most = 128;
+        if (g.lg > 0 && g.outs.size() == 1) most = 32;
+        else if (g.lg > 0 && (cached || g.n % (8 * vec))) most = std::min<uint64_t>(most, 17408 / g.leaves.size());
+        if (u <= most) short_units += u * ends;
     }
     if (fan < 16) return fan >= 4 && workgroups < 128;
     return workgroups < (spreads ? 512u : 256u) || 2 * short_units >= units;
