@@ -231,33 +231,42 @@ int64_t default_tile_elems(size_t ds) { return shallow_tile_elems(default_shape(
 
 // The shape a fused work list starts with before any tuning.
 //
-// Below 64 MB the general shape and its narrow kernel are the fastest.  From there on loads and stores stream, since a
-// caller's next buffers are rarely in the memory-side cache (256 MB): the figures below rotate over buffers of 1.2 GB in
-// all.  The rest follows the kind of list (by bytes), its fan (leaves or outputs of the widest group), the blocks'
-// length in 16-byte units, and how many tiles a shape would give.  GPU time in microseconds, fp32, general / chosen:
-//   reductions with several outputs, fan >= 64, by T, the tiles of four vectors per lane of one wave:
-//     T >= 1024 (512 beyond 300 MB): that shape, and for a single collective with aligned outputs two phases, in group
-//       order below 4096 tiles, tile by tile with two-tile reductions from there on: 512 ranks of 524288 (T = 512) 571 /
-//       395, of 1048576 967 / 678 (one phase 705); 64 ranks of 1048576 115 / 89 (94), of 4194304 (T = 4096) 433 / 364
-//       (386; group order 402);
-//     blocks below a tile beyond 300 MB: two waves of four vectors: 512 ranks of 262144 257 / 198, 256 of 262144 178 / 106;
-//     at least 512 tiles of two vectors and two waves: that: 64 ranks of 262144 27.2 / 24.5, of 524288 57.5 / 47.4;
-//     at least 512 tiles of the general shape: it, streaming: 64 ranks of 131072 20.3 / 13.7, 128 of 131072 41.9 / 30.1;
-//     fan >= 256, blocks of 48 to 119 units, from 190 MB on: the same: 512 ranks of 98304 107 / 87, of 131072 142 / 98;
-//   fan below 64: two vectors, two waves: 8 ranks of 1048576 19.7 / 13.6, 16 of 524288 16.4 / 12.7, 32 of 262144 15.3 /
-//     13.8; with fan 32 from 200 MB on four vectors, one wave: of 1048576 57 / 48;
-//   reductions with one output: T >= 1024 and fan >= 64 four vectors, one wave: reduce_scatter on 512 ranks of 2048 370 /
-//     311, on 128 of 8192 158 / 86; at least 512 tiles of two waves and four vectors (or two): 64 ranks of 8192 27.4 / 23.3,
-//     256 of 1024 72 / 57, 16 of 262144 54.4 / 46.9; else the general shape, streaming: 64 ranks of 4096 15.2 / 14.5;
-//   copies to many outputs, aligned, 512 tiles of at least 96 units, or 256 full ones from 400 MB on: four vectors, one
-//     wave: allgather on 512 ranks of 512 138 / 92, on 16 of 65536 16.2 / 13.1, bcast to 512 of 262144 119 / 102; but
-//     allgather on 256 of 1024 (269 MB) 50.1 / 53.6, bcast to 64 of 262144 (67 MB) 15.4 / 16.8, to 16 of 8388608 101 / 109;
-//   single copies: the general shape, streaming: alltoall on 64 ranks of 4096 a pair 28.7 / 24.7; beyond 300 MB two
-//     vectors, two waves: on 512 ranks of 1024 410 / 338 (352).
-// In place a list touches half the bytes it moves, so a program that cycles through few buffers finds them in the cache:
-// 64 ranks of 262144 take 22.9 / 25.1 over 200 MB of buffers, but 34.6 / 25.1 over 1.2 GB; the rule stays the same there.
-// aligned: every output starts on a 16-byte boundary; single: the list is one collective call's own.
-LaunchShape initial_shape(const std::vector<std::vector<Group>>& gs, size_t ds, bool aligned, bool single) {
+// Lists that fit the memory-side cache (256 MB) find their buffers there when a program calls them again, and streaming
+// loads and stores pass it by; buffers that come from memory move faster with them.  A list starts with a streaming
+// shape only where that is no slower with the buffers in cache and faster with buffers rotating over 1.2 GB: from 64 to
+// 96 MB, where the cache holds several such lists, and beyond it, from 300 MB on.  Between, in cache / from memory, the
+// general shape against the best streaming one, GPU microseconds, fp32: allreduce on 8 ranks of 4194304 (268 MB) 42 / 53
+// against 48 / 49, on 64 ranks of 390400 (200 MB) 33 / 50 against 40 / 41, bcast to 64 of 1048576 39 / 50 against 48 / 47.
+// In place a list touches half the bytes it moves, each twice, and stays in cache up to 400 MB: 64 ranks of 781250 54 / 91
+// against 80 / 78.  Lists below 64 MB and those between start with the general shape and its narrow kernel, except long
+// reductions with one output (64 ranks' reduce_scatter of 16128, 268 MB, 43 / 53 against 43 / 45).
+// The rest follows the kind of list (by bytes), its fan (leaves or outputs of the widest group), the blocks' length in
+// 16-byte units, and how many tiles a shape would give.  In cache / from memory, general against chosen:
+//   reductions with several outputs
+//     fan below 64, blocks of at least a tile: one wave of four vectors for fan 8 and, from 300 MB on, for all: 8 ranks,
+//       85 MB, 16.2 / 21.6 against 15.7 / 17.0, 32 ranks, 340 MB, 73 / 76 against 67 / 68; to 96 MB two waves of four vectors
+//       for fan 16 (85 MB 16.7 / 23.5 against 15.9 / 17.0), of two for fan 32 (75 MB 15.1 / 20.4 against 14.7 / 15.6);
+//     fan 64 and more, from 300 MB on, by T, the tiles of four vectors per lane of one wave:
+//       T >= 512: that shape, and for a single collective with aligned outputs two phases, in group order below 4096
+//       tiles, tile by tile with two-tile reductions from there on: from memory 512 ranks of 524288 (T = 512) 571 / 395,
+//       of 1048576 967 / 678 (one phase 705); 64 ranks of 4194304 (T = 4096) 433 / 364 (386; group order 402);
+//       shorter blocks, 120 units or more: two waves of four vectors: 256 ranks of 169984 91 / 93 against 71 / 71, 512 of
+//       262144 from memory 257 against 198; more than 32: the general shape, streaming: 512 ranks of 83968 (41 units)
+//       110 / 119 against 96 / 93 (two waves of four vectors 157 / 155), of 169984 233 / 236 against 182 / 183;
+//       32 or less: the narrow kernel: 1024 ranks of 45056 (11 units) 165 / 166 (two waves of four vectors 279 / 277);
+//   reductions with one output: T >= 1024 and fan >= 64 four vectors, one wave: reduce_scatter on 512 ranks of 2048 from
+//     memory 370 / 311, on 64 of 20416 64 / 66 against 53 / 54; at least 512 tiles of two waves and four vectors, or 640 of two:
+//     16 ranks of 78080 15.9 / 18.9 against 14.1 / 16.1, 64 of 5056 16.1 / 18.4 against 14.6 / 16.0; else the
+//     general shape, streaming: 64 ranks of 4096 14.2 / 15.1 against 12.7 / 13.2;
+//   copies to 32 outputs or more, aligned, 512 tiles of at least 96 units, or 256 full ones: four vectors, one wave, to 96 MB
+//     and from 330 MB on, from 128 outputs on already from 300: allgather on 32 ranks of 17024 (71 MB) 16.8 / 16.6 against
+//     14.4 / 14.6, on 256 of 1280 77 / 81 against 57 / 56, bcast to 64 of 1367168 (350 MB) 74 / 71 against 66 / 66, but
+//     of 1250048 (320 MB) 58 / 63 against 64 / 62;
+//   single copies: the general shape, streaming: alltoall on 64 ranks of 2560 22.2 / 26.4 against 21.8 / 22.2; from 300 MB on
+//     two vectors, two waves: on 256 ranks of 640 84 / 86 against 58 / 58.
+// aligned: every output starts on a 16-byte boundary; single: the list is one collective call's own; aliased: it runs in
+// place.
+LaunchShape initial_shape(const std::vector<std::vector<Group>>& gs, size_t ds, bool aligned, bool single, bool aliased) {
     constexpr uint64_t MB = 1u << 20;
     const LaunchShape wide{4, 64, 0, 1}, pair{2, 128, 0, 1}, quad{4, 128, 0, 1}, general{1, 256, 0, 1};
     const int64_t vec = (int64_t)(16 / ds), tile = deep_tile_elems(wide, ds);
@@ -285,28 +294,27 @@ LaunchShape initial_shape(const std::vector<std::vector<Group>>& gs, size_t ds, 
     while (kind < KINDS && bytes[kind] * 10 < all * 9) ++kind;
     // blocks of unlike lengths (a batch): the one-wave shape where the long ones hold nearly all of it
     if (longest > shortest + 1 && kind <= REDUCE) return tiles >= 1024 && fan >= 64 && long_bytes * 10 >= all * 9 ? wide : default_shape();
+    const bool large = (aliased ? all / 2 : all) > (aliased ? 400 : 300) * MB;
     if (all < 64 * MB || kind == KINDS || (kind != COPY && fan < 8)) return default_shape();
+    if (all > 96 * MB && !large) return kind == REDUCE && fan >= 64 && tiles >= 1024 ? wide : default_shape();
     const uint64_t length = units / blocks;  // a block's units
-    const bool large = all > 300 * MB;
     const LaunchShape rest = length >= 64 && units >= 512 * 64 && !narrow_pays(gs, (int)vec) ? general : default_shape();
     switch (kind) {
     case SPREAD:
-        if (fan < 64) return fan == 32 && all >= 200 * MB ? wide : pair;
-        if (fan >= 256 && all >= 190 * MB && length >= 48 && length < 120) return general;
-        if (tiles >= (large ? 512u : 1024u)) {
+        if (fan < 64) return length < 256 ? default_shape() : large || fan < 16 ? wide : fan < 32 ? quad : pair;
+        if (!large) return default_shape();
+        if (tiles >= 512) {
             if (!aligned || !single) return wide;  // a batch keeps one launch per list until it is tuned
             return tiles < 4096 ? LaunchShape{4, 64, 0, 1, 1, 0} : LaunchShape{4, 64, 0, 1, 2, 1};
         }
-        if (large) return quad;
-        return length >= 128 && units >= 512 * 128 ? pair : rest;
+        return length >= 120 ? quad : length > 32 ? general : default_shape();
     case REDUCE:
         if (fan >= 64 && tiles >= 1024) return wide;
         if (length >= 128 && units >= 512 * 256) return quad;
-        return length >= 128 && units >= 512 * 128 ? pair : rest;
+        return length >= 128 && units >= 640 * 128 ? pair : rest;
     case COPY_MANY:
-        if (!aligned || (fan < 32 && all > 400 * MB)) return default_shape();
-        return (length >= 256 && pieces >= 256 && all >= 400 * MB) || (length >= 96 && pieces >= 512) ? wide
-                                                                                              : default_shape();
+        if (!aligned || fan < 32 || (large && fan < 128 && all < 330 * MB)) return default_shape();
+        return (length >= 96 && pieces >= 512) || (large && length >= 256 && pieces >= 256) ? wide : default_shape();
     default: return large ? pair : general;
     }
 }
@@ -385,7 +393,7 @@ int get_plan(bine_vcomm_t comm, const CollRequest& req, int dtype, std::shared_p
         dp->cp.fused_why = "reduction tree wider than 2^14 leaves";
     }
     if (dp->cp.auto_fused) {
-        rc = upload(one, ds, initial_shape(one, ds, (uint64_t)prog.extent[BUF_RECV] * ds % 16 == 0, true), dp->fused_ends(), dp->cp.trees, &dp->fused);
+        rc = upload(one, ds, initial_shape(one, ds, (uint64_t)prog.extent[BUF_RECV] * ds % 16 == 0, true, dp->cp.aliased), dp->fused_ends(), dp->cp.trees, &dp->fused);
         if (rc) return rc;
     }
     one[0].swap(dp->cp.fused);
@@ -1398,7 +1406,7 @@ extern "C" int bine_batch_create(bine_vcomm_t comm, const bine_batch_item_t* ite
     for (auto& l : b->lists) {
         bool aligned = true;
         for (uint32_t gb : l.group_bucket) aligned = aligned && !off16(b->tabs[gb]);
-        l.shape = initial_shape(l.groups, dtsize(l.dtype), aligned, false);
+        l.shape = initial_shape(l.groups, dtsize(l.dtype), aligned, false, l.ends == Ends::IN_PLACE);
     }
     if (!b->lists.empty()) b->shape = b->lists[0].shape;
     int rc = batch_lower(b.get());
