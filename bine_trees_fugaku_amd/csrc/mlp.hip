@@ -395,7 +395,9 @@ struct Net {
     const float* params;
     uint32_t w_off[kMaxLayers], b_off[kMaxLayers];
     float* act[kMaxLayers];  // outputs of each layer but the last
-    float* dz[kMaxLayers];   // loss gradients of each layer's sums, before the factor 2 / count
+    float* dz[kMaxLayers];   // loss gradients of each layer's sums: kept without the factor 2 / count, times `down`
+    float down;              // a power of two below 2 / (terms of the batch), which mlp_finish takes out again: the
+                             // sums over the rows stay in range wherever those of the whole gradients do
 };
 
 __host__ __device__ inline int row_stride(int width) { return (width + 31) / 32 * 32 + 4; }  // floats of an LDS row
@@ -525,8 +527,8 @@ __global__ __launch_bounds__(64 * kWaves, 4) void mlp_rows(Net net, const float*
             const int r = i / N, c = i - r * N;
             const size_t g = (size_t)row0 * N + i;
             const float m = mask[g], d = m > 0.f ? src[r * S + c] - t[g] : 0.f;
-            src[r * S + c] = d;
-            net.dz[L - 1][g] = d;
+            src[r * S + c] = net.down * d;
+            net.dz[L - 1][g] = net.down * d;
             loss += d * d;
             count += m > 0.f ? 1.f : 0.f;
         }
@@ -667,12 +669,13 @@ __global__ __launch_bounds__(256) void mlp_weight_grads(Net net, GradTiles g, co
     }
 }
 
-// The slices' sum in order, times 2 / count: into grads, or (p not NULL) as the gradient of one Adam step.
-__global__ void mlp_finish(uint64_t n, int nz, const float* __restrict__ work, const float* __restrict__ totals,
+// The slices' sum in order, times 2 / count and `up` (1 / down): into grads, or (p not NULL) as the gradient of one
+// Adam step.
+__global__ void mlp_finish(uint64_t n, int nz, const float* __restrict__ work, const float* __restrict__ totals, float up,
                            float* __restrict__ grads, float* __restrict__ loss_out, float* __restrict__ p,
                            float* __restrict__ m, float* __restrict__ v, float lr, float b1, float b2, float eps, float c1,
                            float c2) {
-    const float cnt = fmaxf(totals[1], 1.f), inv = 2.f / cnt;
+    const float cnt = fmaxf(totals[1], 1.f), inv = 2.f / cnt * up;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
         float acc = work[i];
         int z = 1;
@@ -854,7 +857,9 @@ void rows_forward(bine_mlp_t m, const float* x, int n, float* y, hipStream_t st)
 // Loss and gradients of the masked MSE into grads, or (lr > 0) one Adam step.
 void rows_gradients(bine_mlp_t m, const float* x, const float* t, const float* mask, int n, float* grads, float* loss,
                     float lr, float b1, float b2, float c1, float c2, hipStream_t st) {
-    const Net net = net_of(m);
+    Net net = net_of(m);
+    const int terms = std::ilogb((double)n * m->dims.back());
+    net.down = std::ldexp(1.f, -terms);
     const int nb = (n + kRows - 1) / kRows;
     hipLaunchKernelGGL((mlp_rows<true>), dim3(nb), dim3(64 * kWaves), m->rows_lds, st, net, x, n, nullptr, t, mask, m->partial);
     GradTiles g{};
@@ -866,7 +871,7 @@ void rows_gradients(bine_mlp_t m, const float* x, const float* t, const float* m
     hipLaunchKernelGGL(mlp_weight_grads, dim3(g.first_bias[net.layers] + 1, nzr), dim3(256), 0, st, net, g, x, n, kc,
                        m->work, m->nparams, nb, m->partial, m->totals);
     hipLaunchKernelGGL(mlp_finish, dim3((int)std::min<uint64_t>(1024, (m->nparams + 255) / 256)), dim3(256), 0, st,
-                       m->nparams, nzr, m->work, m->totals, grads, loss, lr > 0.f ? m->params : nullptr, m->adam_m,
+                       m->nparams, nzr, m->work, m->totals, std::ldexp(1.f, terms), grads, loss, lr > 0.f ? m->params : nullptr, m->adam_m,
                        m->adam_v, lr, b1, b2, 1e-8f, c1, c2);
 }
 
