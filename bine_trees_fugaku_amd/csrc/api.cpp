@@ -233,19 +233,26 @@ int64_t default_tile_elems(size_t ds) { return shallow_tile_elems(default_shape(
 //
 // Lists that fit the memory-side cache (256 MB) find their buffers there when a program calls them again, and streaming
 // loads and stores pass it by; buffers that come from memory move faster with them.  A list starts with a streaming
-// shape only where that is no slower with the buffers in cache and faster with buffers rotating over 1.2 GB: from 64 to
-// 96 MB, where the cache holds several such lists, and beyond it, from 300 MB on.  Between, in cache / from memory, the
-// general shape against the best streaming one, GPU microseconds, fp32: allreduce on 8 ranks of 4194304 (268 MB) 42 / 53
-// against 48 / 49, on 64 ranks of 390400 (200 MB) 33 / 50 against 40 / 41, bcast to 64 of 1048576 39 / 50 against 48 / 47.
-// In place a list touches half the bytes it moves, each twice, and stays in cache up to 400 MB: 64 ranks of 781250 54 / 91
-// against 80 / 78.  Lists below 64 MB and those between start with the general shape and its narrow kernel, except long
-// reductions with one output (64 ranks' reduce_scatter of 16128, 268 MB, 43 / 53 against 43 / 45).
+// shape only where buffers rotating over 1.2 GB gain more by it than buffers in cache lose, and these lose a tenth at
+// most (blocks at odd bytes apart, see below): from 64 MB on while the cache holds several such lists, to 128 MB for
+// reductions out of place and to 96 MB for others, and beyond the cache, from 300 MB on.  Between, in cache / from memory,
+// the general shape against the best streaming one, GPU microseconds, fp32: allreduce on 8 ranks of 4194304 (268 MB)
+// 42 / 53 against 48 / 49, on 64 ranks of 390400 (200 MB) 33 / 50 against 40 / 41, bcast to 64 of 1048576 39 / 50 against
+// 48 / 47.  In place a list touches half the bytes it moves, each twice, and stays in cache up to 400 MB: 64 ranks of
+// 781250 54 / 91 against 80 / 78.  Lists below 64 MB and those between start with the general shape and its narrow kernel,
+// except long reductions with one output (64 ranks' reduce_scatter of 16128, 268 MB, 43 / 53 against 43 / 45).
 // The rest follows the kind of list (by bytes), its fan (leaves or outputs of the widest group), the blocks' length in
 // 16-byte units, and how many tiles a shape would give.  In cache / from memory, general against chosen:
 //   reductions with several outputs
 //     fan below 64, blocks of at least a tile: one wave of four vectors for fan 8 and, from 300 MB on, for all: 8 ranks,
-//       85 MB, 16.2 / 21.6 against 15.7 / 17.0, 32 ranks, 340 MB, 73 / 76 against 67 / 68; to 96 MB two waves of four vectors
+//       85 MB, 16.2 / 21.6 against 15.7 / 17.0, 32 ranks, 340 MB, 73 / 76 against 67 / 68; to 128 MB two waves of four vectors
 //       for fan 16 (85 MB 16.7 / 23.5 against 15.9 / 17.0), of two for fan 32 (75 MB 15.1 / 20.4 against 14.7 / 15.6);
+//     fan 64 and more, to 128 MB: four waves of two vectors: 64 ranks of 214016 (110 MB) 20.3 / 31.9 against 17.8 / 20.1, of
+//       262144 (134 MB) 22.2 / 28.9 against 21.2 / 23.5, 128 ranks of 79872 (82 MB) 20.9 / 23.6 against 16.6 / 17.7; from
+//       96 MB on only for blocks of four of its tiles (128 ranks of 129024, 132 MB, 22.1 / 29.0 against 23.3 / 26.4).  Blocks at
+//       odd bytes, which this shape serves no better than the general one, start with two waves of two vectors or the
+//       general shape, streaming, for buffers from memory: 64 ranks of 764925 bytes (98 MB) 17.6 / 27.1 against 24.0 / 23.9, of
+//       1048573 27.2 / 34.0 against 31.8 / 32.3;
 //     fan 64 and more, from 300 MB on, by T, the tiles of four vectors per lane of one wave:
 //       T >= 512: that shape, and for a single collective with aligned outputs two phases, in group order below 4096
 //       tiles, tile by tile with two-tile reductions from there on: from memory 512 ranks of 524288 (T = 512) 571 / 395,
@@ -268,12 +275,13 @@ int64_t default_tile_elems(size_t ds) { return shallow_tile_elems(default_shape(
 // place.
 LaunchShape initial_shape(const std::vector<std::vector<Group>>& gs, size_t ds, bool aligned, bool single, bool aliased) {
     constexpr uint64_t MB = 1u << 20;
-    const LaunchShape wide{4, 64, 0, 1}, pair{2, 128, 0, 1}, quad{4, 128, 0, 1}, general{1, 256, 0, 1};
+    const LaunchShape wide{4, 64, 0, 1}, pair{2, 128, 0, 1}, quad{4, 128, 0, 1}, broad{2, 256, 0, 1}, general{1, 256, 0, 1};
     const int64_t vec = (int64_t)(16 / ds), tile = deep_tile_elems(wide, ds);
     enum Kind { SPREAD, REDUCE, COPY_MANY, COPY, KINDS };
     uint64_t bytes[KINDS] = {}, all = 0, tiles = 0, pieces = 0, units = 0, blocks = 0, long_bytes = 0;
     int64_t longest = 0, shortest = INT64_MAX;
     size_t fan = 0;
+    bool words = true;  // every output on a dword
     for (const auto& v : gs)
         for (const Group& g : v) {
             if (g.n <= 0) continue;
@@ -288,7 +296,10 @@ LaunchShape initial_shape(const std::vector<std::vector<Group>>& gs, size_t ds, 
             longest = std::max(longest, g.n);
             shortest = std::min(shortest, g.n);
             if (g.n >= 2 * tile) long_bytes += b;
-            for (const PoolEntry& o : g.outs) aligned = aligned && o.off % vec == 0;
+            for (const PoolEntry& o : g.outs) {
+                aligned = aligned && o.off % vec == 0;
+                words = words && o.off * ds % 4 == 0;
+            }
         }
     int kind = 0;
     while (kind < KINDS && bytes[kind] * 10 < all * 9) ++kind;
@@ -296,13 +307,17 @@ LaunchShape initial_shape(const std::vector<std::vector<Group>>& gs, size_t ds, 
     if (longest > shortest + 1 && kind <= REDUCE) return tiles >= 1024 && fan >= 64 && long_bytes * 10 >= all * 9 ? wide : default_shape();
     const bool large = (aliased ? all / 2 : all) > (aliased ? 400 : 300) * MB;
     if (all < 64 * MB || kind == KINDS || (kind != COPY && fan < 8)) return default_shape();
-    if (all > 96 * MB && !large) return kind == REDUCE && fan >= 64 && tiles >= 1024 ? wide : default_shape();
+    const uint64_t cached = (kind <= REDUCE && !aliased ? 128 : 96) * MB;
+    if (all > cached && !large) return kind == REDUCE && fan >= 64 && tiles >= 1024 ? wide : default_shape();
     const uint64_t length = units / blocks;  // a block's units
     const LaunchShape rest = length >= 64 && units >= 512 * 64 && !narrow_pays(gs, (int)vec) ? general : default_shape();
     switch (kind) {
     case SPREAD:
         if (fan < 64) return length < 256 ? default_shape() : large || fan < 16 ? wide : fan < 32 ? quad : pair;
-        if (!large) return default_shape();
+        if (!large) {
+            if (aliased || length <= 128 || (all > 96 * MB && length < 512)) return default_shape();
+            return words ? broad : units >= 512 * 128 ? pair : rest;
+        }
         if (tiles >= 512) {
             if (!aligned || !single) return wide;  // a batch keeps one launch per list until it is tuned
             return tiles < 4096 ? LaunchShape{4, 64, 0, 1, 1, 0} : LaunchShape{4, 64, 0, 1, 2, 1};

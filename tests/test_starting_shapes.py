@@ -3,7 +3,8 @@ import pytest
 
 from bine_trees_fugaku_amd import Batch, VComm
 
-GENERAL, GENERAL_STREAM, PAIR, QUAD, WIDE = (1, 256, 0), (1, 256, 1), (2, 128, 1), (4, 128, 1), (4, 64, 1)
+GENERAL, GENERAL_STREAM, PAIR, BROAD = (1, 256, 0), (1, 256, 1), (2, 128, 1), (2, 256, 1)
+QUAD, WIDE = (4, 128, 1), (4, 64, 1)
 
 ROWS = [
     # below 64 MB, and lists that stay in the memory-side cache
@@ -12,9 +13,13 @@ ROWS = [
     ("scatter", [2, 2, 2], "float32", 2097152, GENERAL), ("reduce_scatter", [2, 4], "float64", 262144, GENERAL),
     ("in place", [4, 4, 4], "int32", 262144, GENERAL), ("in place", [4, 4, 4], "float32", 1048576, GENERAL),
     ("reduce_scatter", [4, 4, 4], "float32", 16384, WIDE),
-    # 64 to 96 MB
+    # 64 to 96 MB, reductions out of place to 128 MB
     ("allreduce", [2, 4], "float32", 1310720, WIDE), ("allreduce", [16], "float32", 655360, QUAD),
-    ("allreduce", [4, 8], "float32", 294912, PAIR), ("allreduce", [4, 4, 4], "float32", 163840, GENERAL),
+    ("allreduce", [4, 8], "float32", 294912, PAIR), ("allreduce", [4, 4, 4], "float32", 163840, BROAD),
+    ("allreduce", [4, 4, 4], "float32", 262144, BROAD), ("allreduce", [4, 4, 4], "float32", 266240, GENERAL),
+    ("allreduce", [4, 4, 8], "float32", 79872, BROAD), ("allreduce", [4, 4, 8], "float32", 116736, GENERAL),
+    ("allreduce", [4, 4, 4], "int8", 764925, GENERAL_STREAM), ("allreduce", [4, 4, 4], "int8", 1048573, PAIR),
+    ("in place", [4, 4, 4], "int32", 163840, GENERAL),
     ("reduce_scatter", [16], "float32", 78080, QUAD), ("reduce_scatter", [4, 4, 4], "float32", 5120, PAIR),
     ("allgather", [4, 8], "float32", 17024, WIDE), ("alltoall", [4, 4, 4], "float32", 2560, GENERAL_STREAM),
     ("in place", [2, 4], "float32", 1310720, WIDE),
