@@ -235,7 +235,7 @@ int64_t default_tile_elems(size_t ds) { return shallow_tile_elems(default_shape(
 // loads and stores pass it by; buffers that come from memory move faster with them.  A list starts with a streaming
 // shape only where buffers rotating over 1.2 GB gain more by it than buffers in cache lose, and these lose a tenth at
 // most (blocks at odd bytes apart, see below): from 64 MB on while the cache holds several such lists, to 128 MB for
-// reductions out of place and to 96 MB for others, and beyond the cache, from 300 MB on.  Between, in cache / from memory,
+// reductions out of place and to 96 MB for others, and beyond the cache, from 250 or 300 MB on.  Between, in cache / from memory,
 // the general shape against the best streaming one, GPU microseconds, fp32: allreduce on 8 ranks of 4194304 (268 MB)
 // 42 / 53 against 48 / 49, on 64 ranks of 390400 (200 MB) 33 / 50 against 40 / 41, bcast to 64 of 1048576 39 / 50 against
 // 48 / 47.  In place a list touches half the bytes it moves, each twice, and stays in cache up to 400 MB: 64 ranks of
@@ -253,14 +253,22 @@ int64_t default_tile_elems(size_t ds) { return shallow_tile_elems(default_shape(
 //       odd bytes, which this shape serves no better than the general one, start with two waves of two vectors or the
 //       general shape, streaming, for buffers from memory: 64 ranks of 764925 bytes (98 MB) 17.6 / 27.1 against 24.0 / 23.9, of
 //       1048573 27.2 / 34.0 against 31.8 / 32.3;
-//     fan 64 and more, from 300 MB on, by T, the tiles of four vectors per lane of one wave:
-//       T >= 512: that shape, and for a single collective with aligned outputs two phases, in group order below 4096
-//       tiles, tile by tile with two-tile reductions from there on: from memory 512 ranks of 524288 (T = 512) 571 / 395,
-//       of 1048576 967 / 678 (one phase 705); 64 ranks of 4194304 (T = 4096) 433 / 364 (386; group order 402);
-//       shorter blocks, 120 units or more: two waves of four vectors: 256 ranks of 169984 91 / 93 against 71 / 71, 512 of
-//       262144 from memory 257 against 198; more than 32: the general shape, streaming: 512 ranks of 83968 (41 units)
-//       110 / 119 against 96 / 93 (two waves of four vectors 157 / 155), of 169984 233 / 236 against 182 / 183;
-//       32 or less: the narrow kernel: 1024 ranks of 45056 (11 units) 165 / 166 (two waves of four vectors 279 / 277);
+//     fan 64 and more, beyond the cache, already from 250 MB on (256 MB for 128 outputs and for bytes; blocks at odd bytes
+//       300): 64 ranks of 549888 (282 MB) 56 / 68 against 51 / 54, of 493568 (253 MB) 40 / 55 against 43 / 46; by T, the
+//       tiles of four vectors per lane of one wave:
+//       T >= 512, or 768 for fewer than 128 outputs and for bytes: that shape, and for a single collective with aligned
+//       outputs two phases, in group order below 4096 tiles, tile by tile with two-tile reductions from there on: from
+//       memory 512 ranks of 524288 (T = 512) 571 / 395, of 1048576 967 / 678 (one phase 705); 64 ranks of 4194304
+//       (T = 4096) 433 / 364 (386; group order 402), of 620544 (318 MB, T = 576) 57 with the next one against 61; 128 ranks
+//       of 2537472 bytes (T = 640) 136 against 155;
+//       else by all blocks' units, from memory, the general shape / two waves of four vectors / two waves of two / four
+//       waves of two: from 96 Ki on (64 Ki from 256 outputs on, 128 Ki for bytes) two of four: 64 ranks of 556032
+//       (139 Ki) 69 / 54 / 62 / 65, 128 of 419840 (102 Ki) 110 / 81 / 87 / 93, 512 of 385024 (94 Ki) 425 / 294 / - / 327;
+//       below, to 255 outputs or in blocks of 256 units, two of two: 128 ranks of 331776 (81 Ki) 81 / 66 / 61 / 64, of
+//       1327104 bytes 86 / 80 / 63 / 65, 256 of 1462272 bytes (89 Ki) 215 / 184 / 161 / 169; beyond 32 Ki four of two:
+//       256 ranks of 151552 (37 Ki) 81 / 69 / 73 / 59, of 618496 bytes 86 / 115 / 93 / 76, 512 of 139264 (34 Ki)
+//       167 / 165 / 142 / 114; blocks of more than 32 units the general shape, streaming: 512 ranks of 81920 (20 Ki) 114,
+//       streaming 69 (four of two 76); shorter ones the narrow kernel: 1024 ranks of 45056 (11 units) 165 / 166 (279 / 277);
 //   reductions with one output: T >= 1024 and fan >= 64 four vectors, one wave: reduce_scatter on 512 ranks of 2048 from
 //     memory 370 / 311, on 64 of 20416 64 / 66 against 53 / 54; at least 512 tiles of two waves and four vectors, or 640 of two:
 //     16 ranks of 78080 15.9 / 18.9 against 14.1 / 16.1, 64 of 5056 16.1 / 18.4 against 14.6 / 16.0; else the
@@ -305,7 +313,8 @@ LaunchShape initial_shape(const std::vector<std::vector<Group>>& gs, size_t ds, 
     while (kind < KINDS && bytes[kind] * 10 < all * 9) ++kind;
     // blocks of unlike lengths (a batch): the one-wave shape where the long ones hold nearly all of it
     if (longest > shortest + 1 && kind <= REDUCE) return tiles >= 1024 && fan >= 64 && long_bytes * 10 >= all * 9 ? wide : default_shape();
-    const bool large = (aliased ? all / 2 : all) > (aliased ? 400 : 300) * MB;
+    const uint64_t beyond = aliased ? 800 : kind != SPREAD || fan < 64 || !words ? 300 : ds == 1 || fan / 128 == 1 ? 256 : 250;
+    const bool large = all > beyond * MB;
     if (all < 64 * MB || kind == KINDS || (kind != COPY && fan < 8)) return default_shape();
     const uint64_t cached = (kind <= REDUCE && !aliased ? 128 : 96) * MB;
     if (all > cached && !large) return kind == REDUCE && fan >= 64 && tiles >= 1024 ? wide : default_shape();
@@ -318,11 +327,13 @@ LaunchShape initial_shape(const std::vector<std::vector<Group>>& gs, size_t ds, 
             if (aliased || length <= 128 || (all > 96 * MB && length < 512)) return default_shape();
             return words ? broad : units >= 512 * 128 ? pair : rest;
         }
-        if (tiles >= 512) {
+        if (tiles >= (fan < 128 || ds == 1 ? 768 : 512)) {
             if (!aligned || !single) return wide;  // a batch keeps one launch per list until it is tuned
             return tiles < 4096 ? LaunchShape{4, 64, 0, 1, 1, 0} : LaunchShape{4, 64, 0, 1, 2, 1};
         }
-        return length >= 120 ? quad : length > 32 ? general : default_shape();
+        if (units >= (ds == 1 ? 128u : fan < 256 ? 96u : 64u) * 1024) return quad;
+        if (fan < 256 || length >= 256) return pair;
+        return units > 512 * 64 ? broad : length > 32 ? general : default_shape();
     case REDUCE:
         if (fan >= 64 && tiles >= 1024) return wide;
         if (length >= 128 && units >= 512 * 256) return quad;

@@ -19,7 +19,7 @@ enum : uint16_t {
     ITEM_RUN = 2,  // a run of `pad` one-leaf, one-output copies (see GredItem)
     ITEM_TREE = 16,  // a tile of the tree kernel
     ITEM_PACK = 32,  // a grid of short copies (gpack.hip)
-    ITEM_ANY = 8,  // the tile moves as 16-byte vectors, offsets at any byte
+    ITEM_ANY = 8,  // the tile moves as 16-byte vectors, offsets at any byte (the kernels treat both alike)
     ITEM_NARROW = 4,  // a tile of the narrow kernel (gnarrow.hip): any alignment, any length up to its workgroup's units
 };
 

@@ -9,7 +9,7 @@ QUAD, WIDE = (4, 128, 1), (4, 64, 1)
 ROWS = [
     # below 64 MB, and lists that stay in the memory-side cache
     ("allreduce", [2, 2, 2], "int32", 262144, GENERAL), ("allreduce", [2, 4], "int32", 4194304, GENERAL),
-    ("allreduce", [4, 4, 4], "float32", 524288, GENERAL), ("bcast", [16], "float32", 4194304, GENERAL),
+    ("allreduce", [4, 4, 4], "float32", 507904, GENERAL), ("bcast", [16], "float32", 4194304, GENERAL),
     ("scatter", [2, 2, 2], "float32", 2097152, GENERAL), ("reduce_scatter", [2, 4], "float64", 262144, GENERAL),
     ("in place", [4, 4, 4], "int32", 262144, GENERAL), ("in place", [4, 4, 4], "float32", 1048576, GENERAL),
     ("reduce_scatter", [4, 4, 4], "float32", 16384, WIDE),
@@ -25,7 +25,14 @@ ROWS = [
     ("in place", [2, 4], "float32", 1310720, WIDE),
     # beyond the cache
     ("allreduce", [2, 4], "float32", 6291456, WIDE), ("allreduce", [4, 8], "int8", 6291456, WIDE),
-    ("allreduce", [16, 16], "float32", 172032, QUAD), ("allreduce", [8, 8, 8], "float32", 83968, GENERAL_STREAM),
+    ("allreduce", [16, 16], "float32", 172032, BROAD), ("allreduce", [8, 8, 8], "float32", 83968, GENERAL_STREAM),
+    ("allreduce", [4, 4, 4], "float32", 524288, QUAD), ("allreduce", [4, 4, 4], "int8", 2097152, GENERAL),
+    ("allreduce", [4, 4, 4], "float32", 552957, QUAD), ("allreduce", [4, 4, 4], "int8", 2211837, GENERAL),
+    ("allreduce", [4, 4, 4], "float32", 663552, QUAD), ("allreduce", [4, 4, 4], "float32", 819200, WIDE),
+    ("allreduce", [4, 4, 8], "float32", 262144, GENERAL), ("allreduce", [4, 4, 8], "float32", 331776, PAIR),
+    ("allreduce", [4, 4, 8], "float32", 655360, WIDE), ("allreduce", [4, 4, 8], "int8", 2621440, QUAD),
+    ("allreduce", [16, 16], "int8", 1462272, PAIR), ("allreduce", [8, 8, 8], "float32", 139264, BROAD),
+    ("allreduce", [8, 8, 8], "float32", 385024, QUAD),
     ("allreduce", [8, 8, 16], "float32", 45056, GENERAL), ("allreduce", [8, 8, 16], "float32", 65536, GENERAL),
     ("allreduce", [4, 4, 4], "float64", 1048576, WIDE), ("allgather", [16, 16], "float32", 1280, WIDE),
     ("bcast", [4, 4, 4], "float32", 1250048, GENERAL), ("bcast", [4, 4, 4], "float32", 1441792, WIDE),
