@@ -1,5 +1,5 @@
-// gpack.hip -- short copies, many to a workgroup: the alltoall of small messages, and scatters and gathers of short or
-// odd blocks.
+// gpack.hip -- short copies, many to a workgroup: the alltoall of small messages, and scatters and gathers of short
+// blocks, or of blocks up to 20 KiB that are no whole number of vectors.
 //
 // An item is a grid of t1 x t2 copies of one length whose source and destination both advance by a fixed (rank, offset)
 // step along either axis (GredItem), so no pool entry is read per copy: an alltoall is one such grid of P x P copies, a

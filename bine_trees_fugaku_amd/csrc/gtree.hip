@@ -11,7 +11,10 @@
 // registers picked by uniform branches; selects over all levels took twice the time (100 ranks of 1000 elements 23.0
 // against 13.0 us with four waves).  At large sizes memory: 100 ranks of 2097152 fp32 elements (1.7 GB) move at 4.5
 // TB/s.  Against the schedule's steps, GPU time per call, fp32: 36 ranks of 131072 84.8 -> 12.8 us, of 2097152
-// 423 -> 138; 100 ranks of 32768 109 -> 12.9; 12 ranks of 1000 25 -> 4.0.
+// 423 -> 138; 100 ranks of 32768 109 -> 12.9; 12 ranks of 1000 25 -> 4.0.  Stacks of more than six values run an
+// instantiation of their own, whose code no longer fits the instruction cache: 0.66 us for each leaf of a wave (a ring of
+// 400 ranks of 403 262 -> 83).  Evaluated with the levels by lane address it takes half of that at small sizes and 5 to
+// 20 % more from 100 ranks of 32768 on.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

@@ -233,8 +233,9 @@ int bine_plan_stats(bine_vcomm_t comm, int32_t coll, int count, bine_datatype_t 
  * per candidate (bine_tuning_candidates lists them; 28 on an MI355X), then,
  * where the schedule holds reductions with several outputs, at the three
  * fastest shapes in both two-phase modes, with reduction items of one and two
- * tiles (twelve more; see bine_batch_set_tuning).  The
- * work list in place before the call stays allocated until the vcomm is
+ * tiles (twelve more; see bine_batch_set_tuning).  A list of general trees (an
+ * AUTO allreduce on a torus that is no power of two) takes no shape: it runs
+ * once and stays as it is.  The work list in place before the call stays allocated until the vcomm is
  * destroyed, so graphs captured earlier keep running the old launch shape.
  * Must not run concurrently with other calls on the same vcomm. */
 int bine_plan_autotune(bine_vcomm_t comm, int32_t coll, const void* sendbuf, void* recvbuf, int count,
@@ -282,8 +283,9 @@ typedef struct bine_batch_s* bine_batch_t;
 /* Compile `n` collectives on one vcomm into one fused work list.  The buffers
  * are bound here and must stay allocated, and the vcomm alive, until
  * bine_batch_destroy.  An allreduce item with sendbuf == recvbuf runs in place:
- * with the fused lists where its schedule allows (powers of two, algorithms B and
- * B_CONT), else per step after them.  Retuning a batch (set_tuning, autotune)
+ * with the fused lists, those of general trees included, wherever every output
+ * that overlaps an input of its list lies exactly on a leaf of its own group,
+ * whatever the algorithm; else per step after them.  Retuning a batch (set_tuning, autotune)
  * replaces its work lists: graphs the caller captured from bine_batch_launch
  * before that must be captured again (bine_batch_launch_graph does so itself). */
 int bine_batch_create(bine_vcomm_t comm, const bine_batch_item_t* items, int n, bine_batch_t* out);
@@ -293,7 +295,8 @@ int bine_batch_launch(bine_batch_t batch, void* stream);
 int bine_batch_launch_graph(bine_batch_t batch, void* stream);
 /* Time candidate (vector width, workgroup, persistence, streaming) shapes and keep the fastest, chosen
  * separately for each element type's work list; a list holding reductions with several outputs is also
- * timed at its three fastest shapes in both two-phase modes, with reduction items of one and two tiles. */
+ * timed at its three fastest shapes in both two-phase modes, with reduction items of one and two tiles.
+ * Lists of general trees take no shape and are left alone. */
 int bine_batch_autotune(bine_batch_t batch, void* stream, int iters);
 int bine_batch_stats(bine_batch_t batch, bine_plan_stats_t* out);
 /* Launch shape: 16-byte vectors per thread (1, 2, 4), threads per workgroup (64..512, power of two),
@@ -305,9 +308,10 @@ int bine_batch_stats(bine_batch_t batch, bine_plan_stats_t* out);
  * copies issued tile by tile across the blocks instead of block by block; BINE_TUNE_DOUBLE_TILES (8), with a
  * two-phase mode, gives the reduction launch items of two tiles (half as many).  get returns the last shape
  * set, or after autotuning the shape of the list that takes longest, or before either the first list's
- * starting shape (4, 64, 0, streaming where reductions of 64 leaves or more over blocks of two whole
- * tiles or more hold 90 % of the list's bytes in at least 1024 tiles; 1, 256, 0, 0 otherwise); set
- * applies one shape to every list. */
+ * starting shape, which follows the kind of list, its bytes and its blocks (1, 256, 0, 0 for small or
+ * mixed lists; 4, 64, 0, streaming for large reductions, with uneven blocks only where reductions of 64
+ * leaves or more over blocks of two whole tiles or more hold 90 % of the bytes in at least 1024 tiles);
+ * set applies one shape to every list. */
 enum { BINE_TUNE_NONTEMPORAL = 1, BINE_TUNE_TWO_PHASE = 2, BINE_TUNE_TWO_PHASE_BY_TILE = 4, BINE_TUNE_DOUBLE_TILES = 8 };
 int bine_batch_get_tuning(bine_batch_t batch, int32_t* vpt, int32_t* threads, int32_t* persistent_wgs,
                           int32_t* flags);
