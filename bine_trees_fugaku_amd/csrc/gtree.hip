@@ -14,7 +14,7 @@
 // 423 -> 138; 100 ranks of 32768 109 -> 12.9; 12 ranks of 1000 25 -> 4.0.  Stacks of more than six values run an
 // instantiation of their own, whose code no longer fits the instruction cache: 0.66 us for each leaf of a wave (a ring of
 // 400 ranks of 403 262 -> 83).  Evaluated with the levels by lane address it takes half of that at small sizes and 5 to
-// 20 % more from 100 ranks of 32768 on.
+// 20 % more at middle and large ones.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
